@@ -15,6 +15,7 @@
 #include <array>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "comd_internal.h"
@@ -132,6 +133,7 @@ struct comd_ctx {
     // host memory and its device copy, stage_cap bytes each
     char *stage_h, *stage_d;
     size_t stage_cap;
+    hipStream_t xf_stream;  // the second copying thread's stream of state transfers
     std::vector<double> cheb_host;  // current value series phi, rho, F (3 x cn) of replica 0
     // force-kernel launch shape (comd_tune / comd_autotune)
     int ncu, max_lds;
@@ -507,6 +509,7 @@ static void free_all(comd_ctx *c)
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (c->stage_h) hipHostFree(c->stage_h);
+    if (c->xf_stream) hipStreamDestroy(c->xf_stream);
     for (Replica &r : c->reps)
         for (void *p : r.owned)
             if (p) hipFree(p);
@@ -515,6 +518,10 @@ static void free_all(comd_ctx *c)
     for (auto e : c->pool) hipEventDestroy(e);
     if (c->stream) hipStreamDestroy(c->stream);
 }
+
+// Contexts of the process: the transfers' staging (transfer, below) is kept
+// between transfers while there is one.
+static void count_context(int change);
 
 // Per-interval coefficients of the table formula (src-flat/eam.c:418-433):
 // on interval i the value is c0 + t(c1 + t c2) and the derivative d0 + t d1
@@ -904,6 +911,7 @@ static int ctx_create(int nrep, const comd_params *prms, comd_ctx **out)
         delete c;
         return set_err(nullptr, COMD_ERR_HIP, "initialisation failed");
     }
+    count_context(1);
     *out = c;
     return COMD_OK;
 }
@@ -1234,13 +1242,189 @@ static int nl_setup(comd_ctx *c)
 
 // ---- state transfer of one replica
 
+// Chunks of a state transfer.  A chunk's packing over PCIe (57 GB/s) runs
+// while the host copies the one before it out of its buffer; one thread does
+// that at about 28 GB/s, two at 48 (r, p and ids of 12.5 M slots, 650 MB: 23
+// and 13.4 ms), more gain nothing.  A second thread costs about 0.03 ms to
+// start and pays from 64 MB on.  Below that 1 MB chunks overlap better (8 MB:
+// 25 GB/s against 22) and need less pinned memory.
+#define CM_XF_LARGE ((size_t)64 << 20)
+#define CM_XF_CHUNK_SMALL ((size_t)1 << 20)
+#define CM_XF_CHUNK_LARGE ((size_t)4 << 20)
+
+// Pinned staging buffers, shared by the process's contexts (allocating 16 MB
+// takes about 4 ms, as long as the transfer of 200 MB): each is one
+// transfer's while it runs, at most CM_XF_POOL are kept between transfers,
+// and all are freed with the last context.
+#define CM_XF_POOL 2
+struct XferStage {
+    char *h;
+    size_t cap;
+};
+static std::mutex g_xf_mu;
+static XferStage g_xf_free[CM_XF_POOL];
+static int g_xf_nfree, g_contexts;
+
+static XferStage xfer_acquire(size_t bytes)
+{
+    XferStage s = {nullptr, 0};
+    {
+        // one that is large enough; else, with the pool full, one to replace
+        std::lock_guard<std::mutex> lock(g_xf_mu);
+        int k = 0;
+        while (k < g_xf_nfree && g_xf_free[k].cap < bytes) k++;
+        if (k == g_xf_nfree && k == CM_XF_POOL) k = 0;
+        if (k < g_xf_nfree) {
+            s = g_xf_free[k];
+            g_xf_free[k] = g_xf_free[--g_xf_nfree];
+        }
+    }
+    if (s.cap >= bytes) return s;
+    if (s.h) hipHostFree(s.h);
+    s = {nullptr, 0};
+    if (hipHostMalloc((void **)&s.h, bytes, hipHostMallocPortable) == hipSuccess) s.cap = bytes;
+    else s.h = nullptr;
+    return s;
+}
+
+static void xfer_release(const XferStage &s)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_xf_mu);
+        if (g_contexts > 0 && g_xf_nfree < CM_XF_POOL) {
+            g_xf_free[g_xf_nfree++] = s;
+            return;
+        }
+    }
+    hipHostFree(s.h);
+}
+
+static void count_context(int change)
+{
+    XferStage gone[CM_XF_POOL];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> lock(g_xf_mu);
+        g_contexts += change;
+        if (g_contexts == 0)
+            while (g_xf_nfree > 0) gone[n++] = g_xf_free[--g_xf_nfree];
+    }
+    while (n > 0) hipHostFree(gone[--n].h);
+}
+
+// The state of grid g's cells into the caller's slot arrays (upload = false)
+// or from them; null fields are left out (upload: zeros).  The stream is idle
+// on entry and on return.
+static int transfer(comd_ctx *c, const Grid &g, const CmSlots &user, bool upload)
+{
+    struct Field {
+        char *at;
+        size_t bytes;  // per cell
+    };
+    const Field field[8] = {{(char *)user.natoms, 4},
+                            {(char *)user.id, CM_SLOTS * 4},
+                            {(char *)user.itype, CM_SLOTS * 4},
+                            {(char *)user.r, CM_SLOTS * 24},
+                            {(char *)user.p, CM_SLOTS * 24},
+                            {(char *)user.f, CM_SLOTS * 32},
+                            {(char *)user.rho, CM_SLOTS * 8},
+                            {(char *)user.fi, CM_SLOTS * 8}};
+    size_t per = 0;
+    for (const Field &f : field)
+        if (f.at) per += f.bytes;
+    if (per == 0 || g.ncells < 1) return COMD_OK;
+    const bool large = per * g.ncells >= CM_XF_LARGE;
+    const int most = (int)((large ? CM_XF_CHUNK_LARGE : CM_XF_CHUNK_SMALL) / per);
+    const int nchunk = (g.ncells + most - 1) / most;
+    const int span = nchunk > 1 ? most : g.ncells;  // cells per chunk
+    const size_t size = (per * span + 255) / 256 * 256;
+    int nthr = large ? 2 : 1;
+    // two buffers a thread
+    const XferStage stage = xfer_acquire(size * (nchunk > 1 ? 2 * nthr : 1));
+    if (!stage.h) return set_err(c, COMD_ERR_NOMEM, "transfer staging");
+    if (nthr == 2 && !c->xf_stream && hipStreamCreateWithFlags(&c->xf_stream, hipStreamNonBlocking) != hipSuccess) {
+        c->xf_stream = nullptr;
+        nthr = 1;
+    }
+    const DevState d = dev_state(c);
+    // thread t takes chunks t, t + nthr, ... through its own two buffers
+    auto copy = [&](int t, hipStream_t st) -> bool {
+        char *buf[2] = {stage.h + (nchunk > 1 ? 2 * t : 0) * size, nullptr};
+        buf[1] = nchunk > 1 ? buf[0] + size : buf[0];
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        bool ok = true;
+        for (hipEvent_t &e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        auto cells = [&](int k) { return std::min(span, g.ncells - k * span); };
+        auto launch = [&](int k, char *b) {
+            const int n = cells(k);
+            char *at[8];
+            size_t off = 0;
+            // the counts last: any number of 4-byte values, the others whole 256-byte lines
+            for (int j = 7; j >= 0; j--) {
+                at[j] = field[j].at ? b + off : nullptr;
+                if (field[j].at) off += field[j].bytes * n;
+            }
+            const CmSlots h = {(int *)at[0], (int *)at[1], (int *)at[2], (double *)at[3],
+                               (double *)at[4], (double *)at[5], (double *)at[6], (double *)at[7]};
+            if (upload) cm_launch_unpack(d, h, g.cell_base + k * span, n, st);
+            else cm_launch_pack(d, h, g.cell_base + k * span, n, st);
+            return hipGetLastError() == hipSuccess;
+        };
+        auto host = [&](int k, char *b) {
+            const int n = cells(k);
+            size_t off = 0;
+            for (int j = 7; j >= 0; j--) {
+                if (!field[j].at) continue;
+                const size_t bytes = field[j].bytes * n;
+                char *u = field[j].at + field[j].bytes * (size_t)k * span;
+                if (upload) memcpy(b + off, u, bytes);
+                else memcpy(u, b + off, bytes);
+                off += bytes;
+            }
+        };
+        int s = 0;
+        if (ok && !upload && t < nchunk) ok = launch(t, buf[0]) && hipEventRecord(ev[0], st) == hipSuccess;
+        for (int k = t; ok && k < nchunk; k += nthr, s ^= 1) {
+            if (upload) {
+                // the buffer's last chunk read by its kernel, then filled again
+                if (k >= t + 2 * nthr) ok = hipEventSynchronize(ev[s]) == hipSuccess;
+                if (!ok) break;
+                host(k, buf[s]);
+                ok = launch(k, buf[s]) && hipEventRecord(ev[s], st) == hipSuccess;
+            } else {
+                const int kn = k + nthr;
+                if (kn < nchunk) ok = launch(kn, buf[s ^ 1]) && hipEventRecord(ev[s ^ 1], st) == hipSuccess;
+                if (ok) ok = hipEventSynchronize(ev[s]) == hipSuccess;
+                if (ok) host(k, buf[s]);
+            }
+        }
+        if (hipStreamSynchronize(st) != hipSuccess) ok = false;
+        for (hipEvent_t e : ev)
+            if (e) hipEventDestroy(e);
+        return ok;
+    };
+    bool ok0, ok1 = true;
+    std::thread other;
+    if (nthr == 2) {
+        try {
+            other = std::thread([&] { ok1 = hipSetDevice(c->device) == hipSuccess && copy(1, c->xf_stream); });
+        } catch (...) {  // no thread to be had: this one takes both halves
+        }
+    }
+    ok0 = copy(0, c->stream);
+    if (other.joinable()) other.join();
+    else if (nthr == 2) ok1 = copy(1, c->stream);
+    xfer_release(stage);
+    if (!ok0 || !ok1) return set_err(c, COMD_ERR_HIP, "state transfer failed");
+    return COMD_OK;
+}
+
 static int upload_rep(comd_ctx *c, int r, const int *natoms, const int *id, const int *itype, const double *rr,
                       const double *p)
 {
     if (!natoms || !id || !rr) return set_err(c, COMD_ERR_ARG, "null argument");
     const Grid &g = c->reps[r].g;
-    const size_t C = (size_t)g.ncells, S = C * CM_SLOTS;
-    const size_t c0 = (size_t)g.cell_base, s0 = c0 * CM_SLOTS;
+    const size_t C = (size_t)g.ncells;
     int tot = 0;
     long nids = 0;
     for (size_t b = 0; b < C; b++) {
@@ -1263,21 +1447,11 @@ static int upload_rep(comd_ctx *c, int r, const int *natoms, const int *id, cons
                 seen[a] = 1;
             }
     }
-    std::vector<double> buf(S);
-    std::vector<int> it(S, 0);
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(c->natoms + c0, natoms, C * 4, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->id + s0, id, S * 4, hipMemcpyHostToDevice));
-    if (itype) memcpy(it.data(), itype, S * 4);
-    HIPCHK(c, hipMemcpy(c->itype + s0, it.data(), S * 4, hipMemcpyHostToDevice));
-    double *dst[6] = {c->rx, c->ry, c->rz, c->px, c->py, c->pz};
-    for (int k = 0; k < 6; k++) {
-        const double *src = k < 3 ? rr : p;
-        if (!src) std::fill(buf.begin(), buf.end(), 0.0);
-        else
-            for (size_t s = 0; s < S; s++) buf[s] = src[3 * s + (k % 3)];
-        HIPCHK(c, hipMemcpy(dst[k] + s0, buf.data(), S * 8, hipMemcpyHostToDevice));
-    }
+    const CmSlots user = {const_cast<int *>(natoms), const_cast<int *>(id), const_cast<int *>(itype),
+                          const_cast<double *>(rr), const_cast<double *>(p), nullptr, nullptr, nullptr};
+    int rc = transfer(c, g, user, true);
+    if (rc) return rc;
     c->ntot += tot - c->reps[r].ntot;
     c->reps[r].ntot = tot;
     c->have_atoms = 1;
@@ -1288,40 +1462,8 @@ static int upload_rep(comd_ctx *c, int r, const int *natoms, const int *id, cons
 static int download_rep(comd_ctx *c, int r, int *natoms, int *id, int *itype, double *rr, double *p, double *f,
                         double *rho, double *fi)
 {
-    const Grid &g = c->reps[r].g;
-    const size_t C = (size_t)g.ncells, S = C * CM_SLOTS;
-    const size_t c0 = (size_t)g.cell_base, s0 = c0 * CM_SLOTS;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (natoms) HIPCHK(c, hipMemcpy(natoms, c->natoms + c0, C * 4, hipMemcpyDeviceToHost));
-    if (id) HIPCHK(c, hipMemcpy(id, c->id + s0, S * 4, hipMemcpyDeviceToHost));
-    if (itype) HIPCHK(c, hipMemcpy(itype, c->itype + s0, S * 4, hipMemcpyDeviceToHost));
-    std::vector<double> buf(S);
-    auto gather = [&](double *dst, int stride, int k, const double *src) -> int {
-        if (hipMemcpy(buf.data(), src + s0, S * 8, hipMemcpyDeviceToHost) != hipSuccess) return COMD_ERR_HIP;
-        for (size_t s = 0; s < S; s++) dst[stride * s + k] = buf[s];
-        return COMD_OK;
-    };
-    int rc = COMD_OK;
-    if (rr) {
-        rc |= gather(rr, 3, 0, c->rx);
-        rc |= gather(rr, 3, 1, c->ry);
-        rc |= gather(rr, 3, 2, c->rz);
-    }
-    if (p) {
-        rc |= gather(p, 3, 0, c->px);
-        rc |= gather(p, 3, 1, c->py);
-        rc |= gather(p, 3, 2, c->pz);
-    }
-    if (f) {
-        rc |= gather(f, 4, 0, c->fx);
-        rc |= gather(f, 4, 1, c->fy);
-        rc |= gather(f, 4, 2, c->fz);
-        rc |= gather(f, 4, 3, c->fe);
-    }
-    if (rho) HIPCHK(c, hipMemcpy(rho, c->rho + s0, S * 8, hipMemcpyDeviceToHost));
-    if (fi) HIPCHK(c, hipMemcpy(fi, c->fi + s0, S * 8, hipMemcpyDeviceToHost));
-    if (rc) return set_err(c, COMD_ERR_HIP, "download failed");
-    return COMD_OK;
+    return transfer(c, c->reps[r].g, CmSlots{natoms, id, itype, rr, p, f, rho, fi}, false);
 }
 
 static int bin_rep_device(comd_ctx *c, int r, int n, const double *d_xyz, const double *d_pxyz, int itype)
@@ -1411,6 +1553,7 @@ int comd_destroy(comd_ctx *ctx)
     hipStreamSynchronize(ctx->stream);
     free_all(ctx);
     delete ctx;
+    count_context(-1);
     return COMD_OK;
 }
 

@@ -132,6 +132,16 @@ void cm_launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, i
 void cm_launch_rebox(const DevState &d, hipStream_t st);
 void cm_launch_bin(const DevState &d, const Grid &g, hipStream_t st, int n, const double *xyz, const double *pxyz,
                    int itype, int *cnt, int *tmp);
+// Slot arrays in the reference's layout (r, p 3 and f 4 doubles per slot);
+// a null field is not transferred.
+struct CmSlots {
+    int *natoms, *id, *itype;
+    double *r, *p, *f, *rho, *fi;
+};
+// Cells [c0, c0 + nc) of the state into h, and from h (whose itype and p may
+// be null: zeros); h lies in pinned host memory (transfer.hip).
+void cm_launch_pack(const DevState &d, const CmSlots &h, int c0, int nc, hipStream_t st);
+void cm_launch_unpack(const DevState &d, const CmSlots &h, int c0, int nc, hipStream_t st);
 void cm_launch_fill_int(int *p, int v, long n, hipStream_t st);
 void cm_launch_force(const DevState &d, const PotDev &pot, int kind, int mixed, const ForceCfg &cfg, hipStream_t st);
 // All replicas of a batch in one launch (pass 1: EAM density or LJ; pass 3:
