@@ -108,8 +108,9 @@ struct comd_ctx {
     int use_plist;
     double *partials;
     int nparts;
-    // observables and the energy monitor (allocated on first use)
+    // observables, the energy monitor and centrosymmetry (allocated on first use)
     double *obs_part, *mon;
+    double *cs_out;        // centrosymmetry, one double per slot
     comd_observables *obs_out;
     long mon_cap;
     double *red_out;       // 3 doubles, device
@@ -504,7 +505,7 @@ static void free_all(comd_ctx *c)
                     c->perm, c->flags, c->mh, c->plist, c->pcount, c->pvalid,
                     c->partials, c->red_out, c->d_grids, c->d_cell_grid, c->d_pots,
                     c->adj_g[0], c->adj_g[1], c->adj_g[2], c->adj_lam, c->adj_mu,
-                    c->adj_ft, c->adj_f2, c->adj_part, c->adj_out, c->adj_rep, c->obs_part, c->obs_out, c->mon,
+                    c->adj_ft, c->adj_f2, c->adj_part, c->adj_out, c->adj_rep, c->obs_part, c->obs_out, c->mon, c->cs_out,
                     c->adj_gb, c->adj_part_nl, c->adj_E, c->adj_epart, c->stage_d};
     for (void *p : ptrs)
         if (p) hipFree(p);
@@ -1312,10 +1313,10 @@ static void count_context(int change)
     while (n > 0) hipHostFree(gone[--n].h);
 }
 
-// The state of grid g's cells into the caller's slot arrays (upload = false)
-// or from them; null fields are left out (upload: zeros).  The stream is idle
+// The state d of grid g's cells into the caller's slot arrays (upload =
+// false) or from them; null fields are left out (upload: zeros).  The stream is idle
 // on entry and on return.
-static int transfer(comd_ctx *c, const Grid &g, const CmSlots &user, bool upload)
+static int transfer(comd_ctx *c, const DevState &d, const Grid &g, const CmSlots &user, bool upload)
 {
     struct Field {
         char *at;
@@ -1346,7 +1347,6 @@ static int transfer(comd_ctx *c, const Grid &g, const CmSlots &user, bool upload
         c->xf_stream = nullptr;
         nthr = 1;
     }
-    const DevState d = dev_state(c);
     // thread t takes chunks t, t + nthr, ... through its own two buffers
     auto copy = [&](int t, hipStream_t st) -> bool {
         char *buf[2] = {stage.h + (nchunk > 1 ? 2 * t : 0) * size, nullptr};
@@ -1450,7 +1450,7 @@ static int upload_rep(comd_ctx *c, int r, const int *natoms, const int *id, cons
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const CmSlots user = {const_cast<int *>(natoms), const_cast<int *>(id), const_cast<int *>(itype),
                           const_cast<double *>(rr), const_cast<double *>(p), nullptr, nullptr, nullptr};
-    int rc = transfer(c, g, user, true);
+    int rc = transfer(c, dev_state(c), g, user, true);
     if (rc) return rc;
     c->ntot += tot - c->reps[r].ntot;
     c->reps[r].ntot = tot;
@@ -1463,7 +1463,7 @@ static int download_rep(comd_ctx *c, int r, int *natoms, int *id, int *itype, do
                         double *rho, double *fi)
 {
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    return transfer(c, c->reps[r].g, CmSlots{natoms, id, itype, rr, p, f, rho, fi}, false);
+    return transfer(c, dev_state(c), c->reps[r].g, CmSlots{natoms, id, itype, rr, p, f, rho, fi}, false);
 }
 
 static int bin_rep_device(comd_ctx *c, int r, int n, const double *d_xyz, const double *d_pxyz, int itype)
@@ -2195,20 +2195,18 @@ static int centro_rep(comd_ctx *c, int r, double *out)
     if (!out) return set_err(c, COMD_ERR_ARG, "null argument");
     if (!c->have_atoms) return set_err(c, COMD_ERR_STATE, "no atoms");
     const Grid &g = c->reps[r].g;
-    const size_t n = (size_t)g.ncells * CM_SLOTS;
-    double *dev = nullptr;
-    if (hipMalloc((void **)&dev, n * 8) != hipSuccess) return set_err(c, COMD_ERR_NOMEM, "centrosymmetry buffer");
-    int rc = COMD_OK;
-    if (hipMemsetAsync(dev, 0, n * 8, c->stream) != hipSuccess) rc = set_err(c, COMD_ERR_HIP, "memset failed");
-    if (!rc) {
-        cm_launch_centro(dev_state(c), g, dev, c->stream);
-        if (hipGetLastError() != hipSuccess) rc = set_err(c, COMD_ERR_HIP, "centrosymmetry launch failed");
+    if (!c->cs_out && hipMalloc((void **)&c->cs_out, (size_t)c->nslots * 8) != hipSuccess) {
+        c->cs_out = nullptr;
+        return set_err(c, COMD_ERR_NOMEM, "centrosymmetry buffer");
     }
-    if (!rc && (hipMemcpyAsync(out, dev, n * 8, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-                hipStreamSynchronize(c->stream) != hipSuccess))
-        rc = set_err(c, COMD_ERR_HIP, "centrosymmetry copy failed");
-    hipFree(dev);
-    return rc;
+    double *dev = c->cs_out + (size_t)g.cell_base * CM_SLOTS;
+    HIPCHK(c, hipMemsetAsync(dev, 0, (size_t)g.ncells * CM_SLOTS * 8, c->stream));
+    DevState d = dev_state(c);
+    cm_launch_centro(d, g, dev, c->stream);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    d.rho = c->cs_out;  // copied out as the field of one double per slot
+    return transfer(c, d, g, CmSlots{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, out, nullptr}, false);
 }
 
 int comd_centrosymmetry(comd_ctx *c, double *out)

@@ -73,3 +73,14 @@ def test_batch_centrosymmetry_equals_single(gpu, cu500):
         assert np.array_equal(gs, gb)
         assert np.array_equal(s.download()["id"], b.download(r)["id"])
         s.close()
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_centrosymmetry_of_a_gas_equals_oracle(gpu, cu500, ocu500, seed):
+    """Random positions: no pairing stands out, so the search's bound cuts
+    least; momenta play no part."""
+    rng = np.random.default_rng(seed)
+    bounds = (21.0, 26.0, 33.0)
+    xyz = rng.uniform(0.0, 1.0, (1200, 3)) * bounds
+    g, o = both(cu500, ocu500, xyz, np.zeros_like(xyz), bounds)
+    assert np.array_equal(g, o)
