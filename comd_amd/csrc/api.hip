@@ -150,7 +150,7 @@ struct comd_ctx {
     int nl_rows_lds;    // COMD_TUNE_LIST_ROWS_LDS (-1: whenever they fit)
     int nl_threads_div; // COMD_TUNE_LIST_THREADS_DIV: home atoms per thread of the list passes
     int nl_lanes;       // COMD_TUNE_LIST_LANES: lanes per home atom of the list passes (0: by size)
-    long nl_alloc_n, nl_alloc_k, nl_alloc_aux, nl_alloc_groups, nl_alloc_rep;
+    long nl_alloc_n, nl_alloc_k, nl_alloc_aux, nl_alloc_groups, nl_alloc_rep, nl_alloc_gslot;
     int nl_eam_groups, nl_lj_groups;  // the list groups of the EAM replicas (first), then of the LJ ones
     int nl_eam_rep, nl_lj_rep;        // a replica of each kind (their potentials stand for the kind's)
     // one DKD step captured as a HIP graph (comd_steps)
@@ -486,11 +486,12 @@ static void free_nl(comd_ctx *c)
                  c->nl.nbl,      c->nl.ncnt,     c->nl.aux_cnt,   c->nl.aux_n,   c->nl.aux_start,
                  c->nl.aux_mem,  c->nl.gstart,   c->nl.nonempty,  c->nl.count,   c->nl.flags,
                  (void *)c->nl.cell_order, (void *)c->nl.group_q0, (void *)c->nl.group_rep,
-                 (void *)c->nl.aux_group, (void *)c->nl.rep};
+                 (void *)c->nl.aux_group, (void *)c->nl.rep, c->nl.gtab, c->nl.gslot};
     for (void *q : p)
         if (q) hipFree(q);
     memset(&c->nl, 0, sizeof c->nl);
     c->nl_alloc_n = c->nl_alloc_k = c->nl_alloc_aux = c->nl_alloc_groups = c->nl_alloc_rep = 0;
+    c->nl_alloc_gslot = 0;
     c->nl_active = 0;
 }
 
@@ -692,7 +693,8 @@ static bool setup_pot(const comd_params *p, Replica &R)
             f[1] = b[1];
         }
         // mixed density rows: phi d0 d1 (double), then 6 floats (40 bytes)
-        std::vector<float> dm((size_t)10 * (n + 1));
+        // padded to whole 16-byte words, as the passes stage them
+        std::vector<float> dm(((size_t)10 * (n + 1) + 3) / 4 * 4, 0.0f);
         for (int i = 0; i <= n; i++) {
             memcpy(&dm[10 * i], &d64[8 * i], 2 * sizeof(double));
             for (int q = 0; q < 6; q++) dm[10 * i + 4 + q] = (float)d64[8 * i + 2 + q];
@@ -1088,8 +1090,10 @@ static int nl_setup(comd_ctx *c)
             if ((c->reps[r].prm.potential == COMD_POT_LJ) == (pass == 1)) gorder.push_back(r);
     long nids = 0;
     for (int r = 0; r < nrep; r++) nids += c->reps[r].nl_ids;
+    const long pass_threads = std::min<long>(768, threads), gwords = (hcap + 4 * pass_threads - 1) / (4 * pass_threads);
+    const long ngslot = ngroups * gwords * pass_threads;
     if (nids > c->nl_alloc_n || kmax > c->nl_alloc_k || naux > c->nl_alloc_aux || ngroups > c->nl_alloc_groups ||
-        nrep > c->nl_alloc_rep) {
+        nrep > c->nl_alloc_rep || ngslot > c->nl_alloc_gslot) {
         free_nl(c);
         bool ok = true;
         auto alloc = [&](void **ptr, size_t bytes) {
@@ -1114,6 +1118,8 @@ static int nl_setup(comd_ctx *c)
         alloc((void **)&c->nl.group_rep, (size_t)ngroups * 4);
         alloc((void **)&c->nl.aux_group, (size_t)naux * 4);
         alloc((void **)&c->nl.rep, (size_t)nrep * sizeof(NlRep));
+        alloc((void **)&c->nl.gtab, (size_t)ngroups * CM_NL_GTAB * 4);
+        alloc((void **)&c->nl.gslot, (size_t)ngslot * 4);
         alloc((void **)&c->nl.nonempty, (size_t)c->ncells * 4);
         alloc((void **)&c->nl.count, 16);
         alloc((void **)&c->nl.flags, 16);
@@ -1126,6 +1132,7 @@ static int nl_setup(comd_ctx *c)
         c->nl_alloc_aux = naux;
         c->nl_alloc_groups = ngroups;
         c->nl_alloc_rep = nrep;
+        c->nl_alloc_gslot = ngslot;
     }
     CmList &l = c->nl;
     l.n = (int)nids;
@@ -1138,7 +1145,8 @@ static int nl_setup(comd_ctx *c)
     l.rows_lds = c->nl_rows_lds;
     l.pass_blocks = (int)ngroups;
     // threads per pass block: a group's home atoms with 10 % to spare
-    l.pass_threads = (int)std::min<long>(768, threads);
+    l.pass_threads = (int)pass_threads;
+    l.gwords = (int)gwords;
     l.lanes = lanes;
     l.tailq = cm_nl_pick_tailq(l);
     std::vector<NlRep> reps(nrep);
@@ -2317,6 +2325,7 @@ int comd_snapshot_load(comd_ctx *c, const char *path)
         for (auto &b : snap_list_buffers(c)) ok = ok && snap_io(fp, b.first, b.second, false);
     fclose(fp);
     if (!ok) return set_err(c, COMD_ERR_ARG, "%s is truncated", path);
+    if (c->nl_active) cm_nl_tables(c->nl, c->stream);  // not in the file: they follow from the cells' offsets
     c->nl_stale = 0;
     c->nl_invalid_seen = 0;
     invalidate_graph(c);

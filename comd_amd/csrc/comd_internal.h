@@ -265,6 +265,9 @@ struct CmList {
     int *aux_start;          // first atom of each auxiliary cell in build order
     int *aux_mem;            // [cell][CM_NL_AUXCAP] member ids
     int *gstart;             // [ngroups + 1]: first atom of each group in build order
+    int *gtab;               // [ngroups][CM_NL_GTAB]: the groups' halo tables (nlist.hip, group_store)
+    unsigned *gslot;         // [ngroups][gwords][pass_threads]: slots of the halo entries
+    int gwords;              // words of four entries per thread: ceil(hcap / (4 pass_threads))
     int *nonempty;           // per link cell: non-empty stencil cells (Lennard-Jones virial)
     int *count;              // [0]: atoms in build order, [1]: builds so far, [2]: build blocks done,
                              // [3]: group-sum blocks done
@@ -272,11 +275,13 @@ struct CmList {
 };
 #define CM_NL_AUXCAP 64
 #define CM_NL_SLOTS 180                 // halo cells of a group, at most (4 + 2) x (4 + 2) x (3 + 2)
+#define CM_NL_GTAB (CM_NL_SLOTS + 4)    // words of a group's halo table
 #define CM_NL_STATIC_LDS (6 << 10)      // static LDS of the list kernels, rounded up
 __host__ __device__ inline size_t nl_entry(int k, int t, int n) { return ((size_t)(k >> 3) * n + t) * 8 + (k & 7); }
 void cm_nl_init(const DevState &d, const CmList &l, hipStream_t st);
 void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st);
 void cm_nl_sync(const DevState &d, const CmList &l, hipStream_t st);
+void cm_nl_tables(const CmList &l, hipStream_t st);
 size_t cm_nl_build_lds(const CmList &l);
 // Entries per thread of the build's tail queue: the most (16, 12, 8 or 4)
 // that fit without fewer resident build blocks per CU than with none.

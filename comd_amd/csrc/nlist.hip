@@ -217,6 +217,73 @@ __device__ __forceinline__ void group_setup(const CmList &l, const NlRep &R, con
     }
 }
 
+// A group's halo table as the passes read it, written at the build: per halo
+// slot its first atom in build order less the slot's offset in the halo (entry
+// h of slot s is atom base[s] + h), the halo's size, and per entry its slot (a
+// byte, four of a thread's entries to a word: entries t + 4 w bd + k bd, k =
+// 0..3, of thread t in a block of bd).  The passes then start from three
+// coalesced loads.  Before, every pass formed the table again (two dependent
+// gathers, the scan, the byte map filled slot by slot) and copied the table
+// rows through registers, with nothing else to run on a CU that holds one or
+// two blocks.  With this and stage_rows: 2 048 000 atoms density 0.246 ->
+// 0.222 ms mixed, 0.422 -> 0.400 FP64, embedding force 0.193 -> 0.184 and
+// 0.299 -> 0.278; 256 000 atoms FP64 87 -> 69 and 57 -> 52 us.
+__device__ __forceinline__ void group_store(const CmList &l, const GroupLds &S, const CM_LDS uint8_t *slot_of, int g)
+{
+    int *gt = l.gtab + (size_t)g * CM_NL_GTAB;
+    const int H = S.off[S.ns], bd = blockDim.x;
+    for (int s = threadIdx.x; s < S.ns; s += bd) gt[s] = S.start[s] - S.off[s];
+    if (threadIdx.x == 0) gt[CM_NL_SLOTS] = H;
+    for (int w = 0; w < l.gwords; w++) {
+        unsigned v = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int h = (int)threadIdx.x + (4 * w + k) * bd;
+            if (h < min(H, l.hcap)) v |= (unsigned)slot_of[h] << (8 * k);
+        }
+        l.gslot[((size_t)g * l.gwords + w) * bd + threadIdx.x] = v;
+    }
+}
+
+// The same in a pass's LDS: base per slot, and the slots' coordinates (ux | uy
+// << 8 | uz << 16).  No barrier: the caller's follows.  Returns the halo's
+// size (never above hcap while the lists are valid).
+struct PassLds {
+    int base[CM_NL_SLOTS], uxyz[CM_NL_SLOTS];
+};
+
+__device__ __forceinline__ int group_load(const CmList &l, const GroupGeo &G, int g, PassLds &S)
+{
+    const int *gt = l.gtab + (size_t)g * CM_NL_GTAB;
+    const int hx = G.lx + 2, hy = G.ly + 2, ns = hx * hy * (G.lz + 2);
+    for (int s = threadIdx.x; s < ns; s += blockDim.x) {
+        S.base[s] = gt[s];
+        S.uxyz[s] = s % hx | ((s / hx) % hy) << 8 | (s / (hx * hy)) << 16;
+    }
+    return min(gt[CM_NL_SLOTS], l.hcap);
+}
+
+// Word w of this thread's halo slots (group_store).
+__device__ __forceinline__ unsigned group_slots(const CmList &l, int g, int w)
+{
+    return ((const CM_GLOBAL unsigned *)l.gslot)[((size_t)g * l.gwords + min(w, l.gwords - 1)) * blockDim.x + threadIdx.x];
+}
+
+// bytes (a multiple of 16) of global memory straight into LDS, 16 bytes a
+// lane, in flight until the caller's wait (vmcnt) and barrier: table rows need
+// no registers on the way and their wait is shared with the halo's.
+__device__ __forceinline__ void stage_rows(CM_LDS char *dst, const void *src, int bytes)
+{
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const CM_GLOBAL char *s = (const CM_GLOBAL char *)src;
+    for (int o = w * 1024; o < bytes; o += (int)blockDim.x * 16)
+        if (o + lane * 16 < bytes)
+            __builtin_amdgcn_global_load_lds((const CM_GLOBAL unsigned *)(s + o + lane * 16), (CM_LDS unsigned *)(dst + o), 16, 0, 0);
+}
+
+// Every vector-memory load of this wave has arrived (stage_rows' among them).
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v3u __attribute__((ext_vector_type(3)));
 
@@ -423,6 +490,7 @@ __global__ __launch_bounds__(1024) void k_nl_build(DevState d, CmList l)
     // the group's replica: the grid of every atom it stages
     const Grid gr = d.ngrids == 1 ? d.g0 : d.grids[l.group_rep[g]];
     group_setup(l, R, G, g, S, slot_of);
+    group_store(l, S, slot_of, g);
     const int H = S.off[S.ns];
     if (H > l.hcap) {  // the same in every thread of the block
         ovf = true;
@@ -534,6 +602,19 @@ __global__ __launch_bounds__(1024) void k_nl_build(DevState d, CmList l)
         else atomicAnd(l.flags, ~(unsigned)CM_NL_INVALID);
         atomicAnd(l.flags, ~(unsigned)(CM_NL_OVERFLOW | CM_NL_REBUILD));
     }
+}
+
+// The groups' halo tables from the cells' counts and offsets, for lists that
+// were not built here (a snapshot's).
+__global__ __launch_bounds__(1024) void k_nl_tables(CmList l)
+{
+    extern __shared__ float4 hl4[];  // [hcap] the slot map
+    __shared__ GroupLds S;
+    const int g = blockIdx.x;
+    const NlRep R = nl_rep(l, l.group_rep[g]);
+    CM_LDS uint8_t *slot_of = (CM_LDS uint8_t *)hl4;
+    group_setup(l, R, group_geo(R, g - R.group_base), g, S, slot_of);
+    group_store(l, S, slot_of, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -991,8 +1072,7 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
 // at the centre of the group's cells), then each thread takes home atoms.
 // TLDS: the compact table rows are staged in LDS (1), or the full tables are
 // read from global memory (0); a compile-time choice, so the row reads are
-// LDS or global loads.  Dynamic LDS: [rows (TLDS)] [halo, hcap atoms]
-// [slot of each halo entry, hcap bytes].
+// LDS or global loads.  Dynamic LDS: [rows (TLDS)] [halo, hcap atoms].
 // Blocks of at most 768 threads (a group's home atoms); the Chebyshev passes
 // declare that bound, so that their four-pair recurrences (cheb64_n) get the
 // registers three waves per SIMD allow.
@@ -1002,29 +1082,19 @@ __attribute__((amdgpu_waves_per_eu(MIXED && KIND != CM_KIND_LJ && TLDS ? 6 : 1))
 void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase)
 {
     extern __shared__ __align__(16) char nls[];
-    __shared__ GroupLds S;
+    __shared__ PassLds S;
     if (l.flags[0] & CM_NL_INVALID) return;
     CM_LDS char *halo = (CM_LDS char *)nls + tab_bytes;
-    CM_LDS uint8_t *slot_of = (CM_LDS uint8_t *)(halo + (size_t)l.hcap * nl_halo_bytes(KIND, MIXED));
     CM_LDS v4u *hq = (CM_LDS v4u *)halo;
     CM_LDS double *hx = (CM_LDS double *)halo, *hy = hx + l.hcap, *hz = hy + l.hcap, *hf = hz + l.hcap;
     CompactLds TL;
     TL.d64 = TL.r64 = nullptr;
     TL.dm = nullptr;
     if (TLDS) {
-        if (MIXED && KIND == CM_KIND_EAM1) {
-            const int nv = (P.n[0] + 1) * 10;
-            CM_LDS float *dst = (CM_LDS float *)nls;
-            for (int k = threadIdx.x; k < nv; k += blockDim.x) dst[k] = P.cdm[k];
-            TL.dm = dst;
-            TL.d64 = (CM_LDS double *)dst;
-        } else {
-            const int nv = (P.n[0] + 1) * (KIND == CM_KIND_EAM1 ? 8 : 2);
-            const double *src = KIND == CM_KIND_EAM1 ? P.cd64 : P.cr64;
-            CM_LDS double *dst = (CM_LDS double *)nls;
-            for (int k = threadIdx.x; k < nv; k += blockDim.x) dst[k] = src[k];
-            TL.d64 = TL.r64 = dst;
-        }
+        const void *rows = KIND == CM_KIND_EAM1 ? (MIXED ? (const void *)P.cdm : (const void *)P.cd64) : (const void *)P.cr64;
+        stage_rows((CM_LDS char *)nls, rows, tab_bytes);
+        TL.dm = (CM_LDS float *)nls;
+        TL.d64 = TL.r64 = (CM_LDS double *)nls;
     }
     const TabsGlobal TG = global_tabs(P);
     // one group per block (the dispatcher balances the groups' uneven work
@@ -1045,26 +1115,28 @@ void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase)
         const int ta = l.gstart[g] + (int)threadIdx.x / lanes, tb = l.gstart[g + 1];
         NlHead hd = {0, 0, 0, {0u, 0u, 0u, 0u}};
         if (ta < tb) hd = nl_head(l, ta, sub);
-        group_setup(l, R, G, g, S, slot_of);  // its first barrier also covers the table staging
+        const int H = group_load(l, G, g, S);
+        unsigned word = group_slots(l, g, 0);
         const double ox = (G.x0 + 0.5 * G.lx) * R.ab0, oy = (G.y0 + 0.5 * G.ly) * R.ab1,
                      oz = (G.z0 + 0.5 * G.lz) * R.ab2;
-        const int H = min(S.off[S.ns], l.hcap);  // never above hcap while the lists are valid
-        // up to SB entries per thread in flight: their id and position loads
-        // are issued together (a thread stages about hcap / blockDim of
-        // them, up to 3.8 with 4 x 4 x 3 groups; one at a time in the mixed
-        // embedding-force pass and four in the other mixed table and
-        // Lennard-Jones passes, which keep to 80 registers for six waves
-        // per SIMD with the atom's head held meanwhile)
-        constexpr int SB = MIXED ? (KIND == CM_KIND_EAM3 ? 1 : EVAL == COMD_EVAL_CHEB ? 6 : 4) : 6;
-        for (int h0 = threadIdx.x; h0 < H; h0 += SB * blockDim.x) {
-            // slots first, then the position loads (build order: a
-            // halo slot's atoms are consecutive)
+        __syncthreads();
+        // up to SB entries per thread in flight: their position loads are
+        // issued together (a thread stages about hcap / blockDim of them, up
+        // to 3.8 with 4 x 4 x 3 groups; one at a time in the mixed table
+        // passes, which keep to 80 registers for six waves per SIMD with the
+        // atom's head held meanwhile: two or four at a time spill, density
+        // pass 0.222 -> 0.27 ms)
+        constexpr int SB = MIXED && KIND == CM_KIND_EAM3 ? 1 : MIXED && TLDS ? 1 : 4;
+        const int bd = (int)blockDim.x;
+        for (int h0 = threadIdx.x, n = 0; h0 < H; h0 += SB * bd, n += SB) {
+            if (n > 0 && (n & 3) == 0) word = group_slots(l, g, n >> 2);
             int sl[SB], q[SB];
 #pragma unroll
             for (int k = 0; k < SB; k++) {
-                const int h = min(h0 + k * (int)blockDim.x, H - 1);
-                sl[k] = slot_of[h];
-                q[k] = S.start[sl[k]] + (h - S.off[sl[k]]);
+                sl[k] = (int)((word >> (8 * ((n + k) & 3))) & 0xffu);
+                q[k] = S.base[sl[k]] + h0 + k * bd;
+                // past the halo's end: the first entry again, not used
+                if (h0 + k * bd >= H) sl[k] = sl[0], q[k] = q[0];
             }
             CmPos p[SB];
             double fp[SB];
@@ -1102,6 +1174,7 @@ void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase)
                 }
             }
         }
+        wait_loads();  // the rows (older than the positions just waited for)
         __syncthreads();
         // the first atom with its head read above, then any further ones
         // (more home atoms than threads) with theirs read in turn
@@ -1152,7 +1225,7 @@ template <int PASS, int MIXED>
 __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, CmAdjNl A, int pbase)
 {
     extern __shared__ __align__(16) char nls[];
-    __shared__ GroupLds S;
+    __shared__ PassLds S;
     __shared__ double red[12][ANMOM];
     double *hx = (double *)nls, *hy = hx + l.hcap, *hz = hy + l.hcap;
     CM_LDS uint8_t *slot_of = (CM_LDS uint8_t *)(nls + (size_t)l.hcap * 24);
@@ -1172,13 +1245,17 @@ __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, 
     const int g = nb < 8 ? (int)blockIdx.x : xcd * qb + min(xcd, rem) + idx;
     const NlRep R = nl_rep(l, l.group_rep[g]);
     const GroupGeo G = group_geo(R, g - R.group_base);
-    group_setup(l, R, G, g, S, slot_of);
+    const int H = group_load(l, G, g, S);
+    unsigned word = group_slots(l, g, 0);
+    const int t0 = l.gstart[g], t1 = l.gstart[g + 1];
     const double ox = (G.x0 + 0.5 * G.lx) * R.ab0, oy = (G.y0 + 0.5 * G.ly) * R.ab1,
                  oz = (G.z0 + 0.5 * G.lz) * R.ab2;
-    const int H = min(S.off[S.ns], l.hcap);
-    for (int h = threadIdx.x; h < H; h += blockDim.x) {
-        const int sl = slot_of[h];
-        const CmPos p = load_pos(l.pos, S.start[sl] + (h - S.off[sl]));
+    __syncthreads();
+    for (int h = threadIdx.x, n = 0; h < H; h += blockDim.x, n++) {
+        if (n > 0 && (n & 3) == 0) word = group_slots(l, g, n >> 2);
+        const int sl = (int)((word >> (8 * (n & 3))) & 0xffu);
+        slot_of[h] = (uint8_t)sl;
+        const CmPos p = load_pos(l.pos, S.base[sl] + h);
         frame_pos(R, G, S.uxyz[sl], p, ox, oy, oz, hx[h], hy[h], hz[h]);
     }
     __syncthreads();
@@ -1187,7 +1264,7 @@ __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, 
     // moments through the derivative operator)
     const double de = PASS == 1 ? 0.5 * A.dlde[l.group_rep[g]] : 0.0;
     const double inv_ba = 1.0 / (cb - ca);
-    for (int t = S.t0 + threadIdx.x; t < S.t1; t += blockDim.x) {
+    for (int t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
         const int s = l.slot[l.order[t]];
         const int self = l.selfh[t];
         const double xi = hx[self], yi = hy[self], zi = hz[self];
@@ -1218,8 +1295,7 @@ __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, 
                     add_basis<MIXED, 0>(y, m, wi, 0.0, m0, m0);
                     continue;
                 }
-                const int sl = slot_of[h];
-                const int q = S.start[sl] + (h - S.off[sl]);
+                const int q = S.base[slot_of[h]] + h;
                 const double w = ((gix - A.gb[3L * q + 0]) * dx + (giy - A.gb[3L * q + 1]) * dy +
                                   (giz - A.gb[3L * q + 2]) * dz) / r;
                 if (PASS == 1) {
@@ -1296,7 +1372,7 @@ size_t cm_nl_tab_bytes(const PotDev &P, int kind, int mixed)
 
 size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int *tables_in_lds)
 {
-    const size_t halo = (size_t)l.hcap * nl_halo_bytes(kind, mixed) + nl_slotmap_bytes(l.hcap);
+    const size_t halo = (size_t)l.hcap * nl_halo_bytes(kind, mixed);
     size_t tab = 0;
     if (P.eval == COMD_EVAL_TABLE && kind != CM_KIND_LJ && P.cd64) tab = nl_tab_bytes(P, kind, mixed);
     // rows in LDS whenever they fit beside the halo (unless tuned off)
@@ -1380,6 +1456,11 @@ void cm_nl_force(const DevState &d, const PotDev &P, const CmList &l, int kind, 
         if (kind == CM_KIND_EAM1) nl_launch2<CM_KIND_EAM1, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng);
         else nl_launch2<CM_KIND_EAM3, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng);
     }
+}
+
+void cm_nl_tables(const CmList &l, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_nl_tables, dim3(l.ngroups), dim3(l.pass_threads), nl_slotmap_bytes(l.hcap), st, l);
 }
 
 size_t cm_adj_nl_lds(const CmList &l) { return (size_t)l.hcap * 24 + nl_slotmap_bytes(l.hcap); }

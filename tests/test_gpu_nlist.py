@@ -264,3 +264,23 @@ def test_autotune_tunes_list_passes(gpu, cu500, precision):
     a.nsteps(10)
     b.nsteps(10)
     assert_same(a, b, f"autotuned {precision}, 10 steps", tol=1e-10 if precision == "fp64" else 1e-5)
+
+
+@pytest.mark.parametrize("groups,div,precision", [(4, 4, "fp64"), (3, 3, "mixed"), (4, 4, "mixed"), (0, 4, "fp64")])
+@pytest.mark.parametrize("n", [5, 9])
+def test_halo_tables_of_small_blocks(gpu, cu500, groups, div, precision, n):
+    """Blocks with few threads stage many halo entries each, so their halo
+    slots take several words per thread; across a rebuild."""
+    a, b = pair_of_sims(cu500, n, 3.615, 900.0, 0.1, 17, precision=precision)
+    b.set_precision("fp64")
+    a.tune(list_groups=groups, list_threads_div=div)
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    for s in (a, b):
+        s.force()
+    assert a.list_info()["valid"] == 1
+    assert_same(a, b, f"groups {groups} div {div} {precision}", tol=tol)
+    for s in (a, b):
+        s.nsteps(25)
+    assert a.list_info()["builds"] > 1
+    if precision == "fp64":  # mixed trajectories differ by their rounding
+        assert_same(a, b, "after a rebuild", tol=1e-9)
