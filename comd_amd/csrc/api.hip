@@ -93,8 +93,9 @@ struct comd_ctx {
     double *fx, *fy, *fz, *fe, *rho, *fi, *vir;
     int *nnb;
     // rebin scratch
-    unsigned long long *leave;
+    unsigned long long *leave, *leave_b;  // _b: the second pass of a fused pair of half drifts
     int *mvidx, *meta, *counts, *touched, *tc, *arr_cnt, *arr;
+    int *touched_b, *tc_b, *arr_cnt_b, *arr_b;
     int *mv_slot, *mv_rank, *mv_id, *mv_itype;
     float4 *mv_nlr, *nlr;
     double *mv_rx, *mv_ry, *mv_rz, *mv_px, *mv_py, *mv_pz;
@@ -153,10 +154,11 @@ struct comd_ctx {
     long nl_alloc_n, nl_alloc_k, nl_alloc_aux, nl_alloc_groups, nl_alloc_rep, nl_alloc_gslot;
     int nl_eam_groups, nl_lj_groups;  // the list groups of the EAM replicas (first), then of the LJ ones
     int nl_eam_rep, nl_lj_rep;        // a replica of each kind (their potentials stand for the kind's)
-    // one DKD step captured as a HIP graph (comd_steps)
+    // the repeated part of comd_steps captured as a HIP graph
     int use_graph;
     hipGraphExec_t graph;
     double graph_dt;
+    int graph_fused;  // the graph holds a fused middle (run_steps), not a whole step
     // timing
     int timing;
     std::vector<TimedEvent> events;
@@ -201,13 +203,10 @@ static DevState dev_state(const comd_ctx *c)
     d.fx = c->fx; d.fy = c->fy; d.fz = c->fz; d.fe = c->fe;
     d.rho = c->rho; d.fi = c->fi; d.vir = c->vir;
     d.nnb = c->nnb;
-    d.leave = c->leave;
+    d.ra = RebinSet{c->leave, c->touched, c->tc, c->counts + 1, c->arr_cnt, c->arr};
+    d.rb = RebinSet{c->leave_b, c->touched_b, c->tc_b, c->counts + 2, c->arr_cnt_b, c->arr_b};
     d.mvidx = c->mvidx;
     d.counts = c->counts;
-    d.touched = c->touched;
-    d.tc = c->tc;
-    d.arr_cnt = c->arr_cnt;
-    d.arr = c->arr;
     d.mv_slot = c->mv_slot; d.mv_rank = c->mv_rank; d.mv_id = c->mv_id; d.mv_itype = c->mv_itype;
     d.mv_nlr = c->mv_nlr;
     d.nlr = c->nlr;
@@ -394,7 +393,7 @@ static void op_force(comd_ctx *c)
 }
 
 // One velocity-Verlet step of src-flat/timestep.c:114-135 without the
-// trailing force: half drift, rebin, force, kick + half drift, rebin.
+// trailing force: half drift, rebin, force, kick, half drift, rebin.
 static void op_step(comd_ctx *c, double dt)
 {
     op_move(c, 0.0, dt / 2.0, 0, 1);
@@ -404,33 +403,60 @@ static void op_step(comd_ctx *c, double dt)
     op_rebox(c);
 }
 
-// n steps: replays of the captured step graph when graphs are on and the
-// kernels are not being timed, else launched one by one.
+// A step's force and the rest of it, with the first half drift and rebin of
+// the step after (cm_launch_move_two).
+static void op_middle(comd_ctx *c, double dt)
+{
+    op_force(c);
+    hipEvent_t ev = nullptr;
+    tbegin(c, COMD_K_REBIN, &ev);
+    cm_launch_move_two(dev_state(c), c->stream, dt, dt / 2.0);
+    tend(c, COMD_K_REBIN, ev);
+    c->nl_stale = 0;
+}
+
+// n steps.  Two and more: a first half drift, n - 1 fused middles, a force and
+// the last kick and half drift, when two mover records per atom have room
+// (cells at most half full on average: all but the densest input); else step
+// by step.  The repeated part is replayed from its captured graph when graphs
+// are on and the kernels are not being timed.
 static int run_steps(comd_ctx *c, int n, double dt)
 {
+    const bool fused = n >= 2 && 2L * c->ntot <= c->nslots;
+    const int repeat = fused ? n - 1 : n;
+    if (fused) {
+        op_move(c, 0.0, dt / 2.0, 0, 1);
+        op_rebox(c);
+    }
     if (!c->use_graph || c->timing || n < 2) {
-        for (int i = 0; i < n; i++) op_step(c, dt);
-        HIPCHK(c, hipGetLastError());
-        return COMD_OK;
-    }
-    if (c->graph && c->graph_dt != dt) invalidate_graph(c);
-    if (!c->graph) {
-        hipGraph_t g = nullptr;
-        HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
-        op_step(c, dt);
-        HIPCHK(c, hipStreamEndCapture(c->stream, &g));
-        const hipError_t e = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
-        hipGraphDestroy(g);
-        if (e != hipSuccess) {
-            c->graph = nullptr;
-            return set_err(c, COMD_ERR_HIP, "graph instantiation: %s", hipGetErrorString(e));
+        for (int i = 0; i < repeat; i++) fused ? op_middle(c, dt) : op_step(c, dt);
+    } else {
+        if (c->graph && (c->graph_dt != dt || c->graph_fused != (int)fused)) invalidate_graph(c);
+        if (!c->graph) {
+            hipGraph_t g = nullptr;
+            HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
+            fused ? op_middle(c, dt) : op_step(c, dt);
+            HIPCHK(c, hipStreamEndCapture(c->stream, &g));
+            const hipError_t e = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
+            hipGraphDestroy(g);
+            if (e != hipSuccess) {
+                c->graph = nullptr;
+                return set_err(c, COMD_ERR_HIP, "graph instantiation: %s", hipGetErrorString(e));
+            }
+            c->graph_dt = dt;
+            c->graph_fused = fused;
         }
-        c->graph_dt = dt;
+        for (int i = 0; i < repeat; i++) HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
+        // a whole step ends with a drift that leaves the list positions stale
+        // (the capture recorded that on the host once; replays must too)
+        if (c->nl_active) c->nl_stale = !fused;
     }
-    for (int i = 0; i < n; i++) HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
-    // each step ends with a drift that leaves the list positions stale (the
-    // capture recorded that on the host once; replays must too)
-    if (c->nl_active) c->nl_stale = 1;
+    if (fused) {
+        op_force(c);
+        op_move(c, dt, dt / 2.0, 1, 1, 1, 0);
+        op_rebox(c);
+    }
+    HIPCHK(c, hipGetLastError());
     return COMD_OK;
 }
 
@@ -501,7 +527,7 @@ static void free_all(comd_ctx *c)
     free_nl(c);
     void *ptrs[] = {c->natoms, c->id, c->itype, c->rx, c->ry, c->rz, c->px, c->py, c->pz,
                     c->fx, c->fy, c->fz, c->fe, c->rho, c->fi, c->vir, c->nnb, c->leave, c->mvidx, c->meta,
-                    c->counts, c->touched, c->tc, c->arr_cnt, c->arr, c->mv_slot, c->mv_rank, c->mv_id, c->mv_nlr, c->nlr,
+                    c->counts, c->touched, c->tc, c->arr_cnt, c->arr, c->leave_b, c->touched_b, c->tc_b, c->arr_cnt_b, c->arr_b, c->mv_slot, c->mv_rank, c->mv_id, c->mv_nlr, c->nlr,
                     c->mv_itype, c->mv_rx, c->mv_ry, c->mv_rz, c->mv_px, c->mv_py, c->mv_pz,
                     c->perm, c->flags, c->mh, c->plist, c->pcount, c->pvalid,
                     c->partials, c->red_out, c->d_grids, c->d_cell_grid, c->d_pots,
@@ -813,6 +839,11 @@ static int ctx_create(int nrep, const comd_params *prms, comd_ctx **out)
     alloc((void **)&c->tc, C * 4);
     alloc((void **)&c->arr_cnt, C * 4);
     alloc((void **)&c->arr, S * 4);
+    alloc((void **)&c->leave_b, C * 8);
+    alloc((void **)&c->touched_b, C * 4);
+    alloc((void **)&c->tc_b, C * 4);
+    alloc((void **)&c->arr_cnt_b, C * 4);
+    alloc((void **)&c->arr_b, S * 4);
     // one mover record per slot at most
     alloc((void **)&c->mv_slot, S * 4);
     alloc((void **)&c->mv_rank, S * 4);

@@ -20,27 +20,104 @@
 // that case for the atom's replica, whose cells the parallel kernels then
 // leave alone, and a serial kernel (one block per flagged replica) redoes
 // that replica's pass exactly as the reference does.
+//
+// Fused half drifts.  Inside a multi-step call a step's second half drift and
+// rebin (pass A) are followed at once by the next step's first half drift and
+// rebin (pass B), with nothing between that reads the state.  The move kernels
+// are bound by HBM (4.7 TB/s over the sparse slot rows), so one pass over the
+// atoms does the kick and both half drifts: 232 bytes per atom become 160 and
+// two launches one.  An atom that stays in pass A gets its position after
+// both drifts, and its move in pass B, if any, is recorded with its slot of
+// before A; A's gather, which rewrites the slots of the cells A touches,
+// renames those records' slots and finds the moves in B of the atoms that
+// arrive.  Pass B then scans and gathers its own lists.  When a replica needs
+// A's serial replay, its departing atoms still hold the position of between
+// the drifts (slot) and are known (leave); the serial kernel moves them, drifts
+// them and replays B.  Slot order, positions and flags are those of the two
+// passes, bit for bit.  2 048 000 atoms: two move passes of 68 us -> one of
+// 100, with one launch of the serial kernel in place of two; a step of 256 000
+// atoms FP64 216 -> 190 us, of 864 atoms 62 -> 49 us.
 #include "comd_internal.h"
 
 #define CM_ACAP 64  // arrivals recorded per cell and pass
 
-__device__ static inline void mark_touched(const DevState &d, int c)
+__device__ static inline void mark_touched(const RebinSet &p, int c)
 {
-    if (atomicExch(&d.touched[c], 1) == 0) {
-        const int i = atomicAdd(&d.counts[1], 1);
-        d.tc[i] = c;
+    if (atomicExch(&p.touched[c], 1) == 0) {
+        const int i = atomicAdd(p.ntc, 1);
+        p.tc[i] = c;
     }
+}
+
+// Destination cell of an atom of cell c = (ix, iy, iz) at (x, y, z) by the
+// rules of reBoxAll (domains.c:356-377), -1 when it stays, and its position
+// in that cell.
+__device__ __forceinline__ int hop(const Grid &g, int c, int ix, int iy, int iz, double x, double y, double z,
+                                   double &ax, double &ay, double &az)
+{
+    int nx = ix, ny = iy, nz = iz;
+    ax = x;
+    ay = y;
+    az = z;
+    if (x < 0.0) { nx = ix - 1; ax = x + g.bs0; } else if (x >= g.bs0) { nx = ix + 1; ax = x - g.bs0; }
+    if (y < 0.0) { ny = iy - 1; ay = y + g.bs1; } else if (y >= g.bs1) { ny = iy + 1; ay = y - g.bs1; }
+    if (z < 0.0) { nz = iz - 1; az = z + g.bs2; } else if (z >= g.bs2) { nz = iz + 1; az = z - g.bs2; }
+    const int j = cell_wrap(g, nx, ny, nz);
+    return j == c ? -1 : j;
+}
+
+// An arrival in dst (above c) that is still outside it is moved again in the
+// same pass (it is examined again when dst is scanned).
+__device__ __forceinline__ bool hops_again(const Grid &g, int c, int dst, double ax, double ay, double az)
+{
+    if (dst < c) return false;
+    int jx, jy, jz;
+    cell_xyz(g, dst, jx, jy, jz);
+    double bx, by, bz;
+    return hop(g, dst, jx, jy, jz, ax, ay, az, bx, by, bz) >= 0;
+}
+
+struct Mover {
+    double x, y, z, px, py, pz;  // position in the destination cell, momentum
+    float4 nlr;
+    int id, itype;
+};
+
+// Records the departure of slot s (cell c) to dst in pass P; the caller sets
+// the slot's bit in P.leave.
+__device__ __forceinline__ void put_mover(const DevState &d, const RebinSet &P, int c, int s, int dst, const Mover &v)
+{
+    const int m = atomicAdd(&d.counts[0], 1);  // capacity: one record per slot
+    d.mv_slot[m] = s;
+    d.mv_id[m] = v.id;
+    d.mv_nlr[m] = v.nlr;
+    d.mv_itype[m] = v.itype;
+    d.mv_rx[m] = v.x;
+    d.mv_ry[m] = v.y;
+    d.mv_rz[m] = v.z;
+    d.mv_px[m] = v.px;
+    d.mv_py[m] = v.py;
+    d.mv_pz[m] = v.pz;
+    d.mvidx[s] = m;
+    const int k = atomicAdd(&P.arr_cnt[dst], 1);
+    if (k < CM_ACAP) P.arr[dst * CM_ACAP + k] = m;
+    mark_touched(P, c);
+    mark_touched(P, dst);
 }
 
 // ---------------------------------------------------------------------------
 // kick (p -= dtk f, src-flat/timestep.c:62-74), drift (r += (dtd p)/rmass,
 // timestep.c:76-104) and the per-atom destination of reBoxAll
 // (domains.c:356-377) of the atom in slot s of cell c = (ix, iy, iz);
-// departing atoms are recorded as movers.
+// departing atoms are recorded as movers.  TWO: the kick, both half drifts and
+// the destinations of both passes (see above); kick, drift and rebin are then
+// taken as 1.
+template <int TWO>
 __device__ __forceinline__ void move_atom(const DevState &d, const Grid &g, int c, int ix, int iy, int iz, int s,
                                           double dtk, double dtd, int kick, int drift, int rebin)
 {
     const double rmass = g.rmass;
+    if (TWO) kick = drift = rebin = 1;
     // every load first (the arrays may alias as far as the compiler can
     // tell, so a load after a store would wait for it)
     double x = d.rx[s], y = d.ry[s], z = d.rz[s];
@@ -62,21 +139,39 @@ __device__ __forceinline__ void move_atom(const DevState &d, const Grid &g, int 
         d.py[s] = py;
         d.pz[s] = pz;
     }
+    double ux = 0.0, uy = 0.0, uz = 0.0;
     if (drift) {
-        x = x + dtd * px / rmass;
-        y = y + dtd * py / rmass;
-        z = z + dtd * pz / rmass;
-        d.rx[s] = x;
-        d.ry[s] = y;
-        d.rz[s] = z;
+        ux = dtd * px / rmass;
+        uy = dtd * py / rmass;
+        uz = dtd * pz / rmass;
+        x = x + ux;
+        y = y + uy;
+        z = z + uz;
+    }
+    double ax = x, ay = y, az = z;
+    int dst = -1;  // of pass A
+    if (rebin) dst = hop(g, c, ix, iy, iz, x, y, z, ax, ay, az);
+    // the position kept in the slot: a departing atom's is its mover record's,
+    // the slot's own serves the serial replay alone
+    int hx = ix, hy = iy, hz = iz;  // the cell that (wx, wy, wz) is relative to
+    double wx = x, wy = y, wz = z;
+    if (TWO) {
+        if (dst >= 0) cell_xyz(g, dst, hx, hy, hz), wx = ax + ux, wy = ay + uy, wz = az + uz;
+        else wx = x + ux, wy = y + uy, wz = z + uz;
+    }
+    if (drift) {
+        const bool first = TWO && dst >= 0;
+        d.rx[s] = first ? x : wx;
+        d.ry[s] = first ? y : wy;
+        d.rz[s] = first ? z : wz;
         if (upkeep) {
             // absolute position for the neighbour lists, and the rebuild
             // request once the atom has moved half the skin (nearest image)
             double cx, cy, cz;
-            corner_of(g, ix, iy, iz, cx, cy, cz);
-            const double ax = cx + x, ay = cy + y, az = cz + z;
-            d.nl_pos[__float_as_int(q.w)] = CmPos{ax, ay, az};
-            double ex = ax - q.x, ey = ay - q.y, ez = az - q.z;
+            corner_of(g, hx, hy, hz, cx, cy, cz);
+            const double bx = cx + wx, by = cy + wy, bz = cz + wz;
+            d.nl_pos[__float_as_int(q.w)] = CmPos{bx, by, bz};
+            double ex = bx - q.x, ey = by - q.y, ez = bz - q.z;
             ex -= g.L0 * rint(ex * g.iL0);
             ey -= g.L1 * rint(ey * g.iL1);
             ez -= g.L2 * rint(ez * g.iL2);
@@ -88,48 +183,29 @@ __device__ __forceinline__ void move_atom(const DevState &d, const Grid &g, int 
         }
     }
     if (!rebin) return;
-    int nx = ix, ny = iy, nz = iz;
-    double ax = x, ay = y, az = z;
-    if (x < 0.0) { nx = ix - 1; ax = x + g.bs0; } else if (x >= g.bs0) { nx = ix + 1; ax = x - g.bs0; }
-    if (y < 0.0) { ny = iy - 1; ay = y + g.bs1; } else if (y >= g.bs1) { ny = iy + 1; ay = y - g.bs1; }
-    if (z < 0.0) { nz = iz - 1; az = z + g.bs2; } else if (z >= g.bs2) { nz = iz + 1; az = z - g.bs2; }
-    const int j = cell_wrap(g, nx, ny, nz);
-    if (j < 0 || j == c) return;
-    const int dst = j;
-    if (dst > c) {
-        // the arrival is examined again when dst is scanned
-        int jx, jy, jz;
-        cell_xyz(g, dst, jx, jy, jz);
-        int mx = jx, my = jy, mz = jz;
-        if (ax < 0.0) mx = jx - 1; else if (ax >= g.bs0) mx = jx + 1;
-        if (ay < 0.0) my = jy - 1; else if (ay >= g.bs1) my = jy + 1;
-        if (az < 0.0) mz = jz - 1; else if (az >= g.bs2) mz = jz + 1;
-        const int j2 = cell_wrap(g, mx, my, mz);
-        if (j2 >= 0 && j2 != dst) atomicOr(&d.mh[g.pot], 1);
+    if (TWO && dst < 0) {
+        // stays in pass A; a move of pass B, under its slot of before A
+        double bx, by, bz;
+        const int dstb = hop(g, c, ix, iy, iz, wx, wy, wz, bx, by, bz);
+        if (dstb < 0) return;
+        if (hops_again(g, c, dstb, bx, by, bz)) atomicOr(&d.mh[g.pot], 2);
+        put_mover(d, d.rb, c, s, dstb, Mover{bx, by, bz, px, py, pz, d.nlr[s], d.id[s], d.itype[s]});
+        atomicOr(&d.rb.leave[c], 1ull << (s - c * CM_SLOTS));
+        return;
     }
-    const int m = atomicAdd(&d.counts[0], 1);  // capacity: one record per slot
-    d.mv_slot[m] = s;
-    d.mv_id[m] = d.id[s];
-    d.mv_nlr[m] = d.nlr[s];
-    d.mv_itype[m] = d.itype[s];
-    d.mv_rx[m] = ax;
-    d.mv_ry[m] = ay;
-    d.mv_rz[m] = az;
-    d.mv_px[m] = px;
-    d.mv_py[m] = py;
-    d.mv_pz[m] = pz;
-    d.mvidx[s] = m;
-    atomicOr(&d.leave[c], 1ull << (s - c * CM_SLOTS));
-    const int k = atomicAdd(&d.arr_cnt[dst], 1);
-    if (k < CM_ACAP) d.arr[dst * CM_ACAP + k] = m;
-    mark_touched(d, c);
-    mark_touched(d, dst);
+    if (dst < 0) return;
+    if (hops_again(g, c, dst, ax, ay, az)) atomicOr(&d.mh[g.pot], 1);
+    const Mover v = TWO ? Mover{wx, wy, wz, px, py, pz, d.nlr[s], d.id[s], d.itype[s]}
+                        : Mover{ax, ay, az, px, py, pz, d.nlr[s], d.id[s], d.itype[s]};
+    put_mover(d, d.ra, c, s, dst, v);
+    atomicOr(&d.ra.leave[c], 1ull << (s - c * CM_SLOTS));
 }
 
 // Any number of replicas: four consecutive global cells per wave, 16 lanes
 // each (a cell's atoms beyond 16 taken in further rounds).  Held to 96
-// registers for five waves per SIMD instead of four (no spills; the
-// 64-replica batch step 0.462 -> 0.459 ms).
+// registers for five waves per SIMD instead of four (the 64-replica batch
+// step 0.462 -> 0.459 ms).
+template <int TWO>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5)))
 void k_move(DevState d, double dtk, double dtd, int kick, int drift, int rebin)
 {
@@ -140,11 +216,13 @@ void k_move(DevState d, double dtk, double dtd, int kick, int drift, int rebin)
     const Grid g = grid_of(d, c);
     int ix, iy, iz;
     cell_xyz(g, c, ix, iy, iz);
-    for (int t = threadIdx.x & 15; t < n; t += 16) move_atom(d, g, c, ix, iy, iz, c * CM_SLOTS + t, dtk, dtd, kick, drift, rebin);
+    for (int t = threadIdx.x & 15; t < n; t += 16)
+        move_atom<TWO>(d, g, c, ix, iy, iz, c * CM_SLOTS + t, dtk, dtd, kick, drift, rebin);
 }
 
 // One replica: four cells per wave, 16 lanes each, cell coordinates from the
 // 3-D grid (x: groups of four cells).
+template <int TWO>
 __global__ __launch_bounds__(64) void k_move4(DevState d, double dtk, double dtd, int kick, int drift, int rebin)
 {
     const Grid &g = d.g0;
@@ -154,7 +232,7 @@ __global__ __launch_bounds__(64) void k_move4(DevState d, double dtk, double dtd
     const int c = ix + g.nbx0 * (iy + g.nbx1 * iz);
     const int n = d.natoms[c];
     for (int t = threadIdx.x & 15; t < n; t += 16)
-        move_atom(d, g, c, ix, iy, iz, c * CM_SLOTS + t, dtk, dtd, kick, drift, rebin);
+        move_atom<TWO>(d, g, c, ix, iy, iz, c * CM_SLOTS + t, dtk, dtd, kick, drift, rebin);
 }
 
 // Per touched cell (one wave each): count arrivals from lower/higher cells,
@@ -162,26 +240,28 @@ __global__ __launch_bounds__(64) void k_move4(DevState d, double dtk, double dtd
 // placeholders appended, recording each departure's rank and the resulting
 // arrangement.  The lanes load the arrivals and the departing atoms' mover
 // records together; lane 0 runs the scan in LDS.
-__global__ __launch_bounds__(64) void k_rebox_scan(DevState d)
+// second: pass B of a fused pair (P: its lists).  A replica with a flag of the
+// pass or an earlier one is left out.
+__global__ __launch_bounds__(64) void k_rebox_scan(DevState d, RebinSet P, int second)
 {
     __shared__ uint8_t perm[128];
     __shared__ int rank_of[CM_SLOTS];
     const int L = threadIdx.x;
-    const int ntc = d.counts[1];
+    const int ntc = *P.ntc, replay = second ? 3 : 1;
     for (int i = blockIdx.x; i < ntc; i += gridDim.x) {
-        const int c = d.tc[i];
-        if (d.mh[rep_of(d, c)]) continue;  // the same in every lane: replayed serially
+        const int c = P.tc[i];
+        if (d.mh[rep_of(d, c)] & replay) continue;  // the same in every lane: replayed serially
         const int n0 = d.natoms[c];
-        int na = d.arr_cnt[c];
+        int na = P.arr_cnt[c];
         // which of the cell's own atoms leave (set by k_move per departure)
-        const unsigned long long leaves = d.leave[c];
+        const unsigned long long leaves = P.leave[c];
         unsigned fl = 0;
         if (na > CM_ACAP) {
             fl |= CM_FLAG_OVERFLOW;
             na = CM_ACAP;
         }
         bool low = false;
-        if (L < na) low = (d.mv_slot[d.arr[c * CM_ACAP + L]] / CM_SLOTS) < c;
+        if (L < na) low = (d.mv_slot[P.arr[c * CM_ACAP + L]] / CM_SLOTS) < c;
         const bool leaving = L < n0 && ((leaves >> L) & 1ull);
         const int mv = leaving ? d.mvidx[c * CM_SLOTS + L] : -1;
         const int nlow = __popcll(__ballot(low));
@@ -225,23 +305,27 @@ __global__ __launch_bounds__(64) void k_rebox_scan(DevState d)
 // (source cell, rank), then write survivors and low arrivals in the scanned
 // arrangement followed by the high arrivals.  All lanes read before any lane
 // writes, so the cell is updated in place.  Clears the cell's pass state.
-__global__ __launch_bounds__(64) void k_rebox_gather(DevState d)
+// FIRST: pass A of a fused pair; the moves of pass B by the cell's atoms are
+// put under their new slots, and those of its arrivals recorded.
+template <int FIRST>
+__global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int second)
 {
     __shared__ int sm[2][CM_SLOTS];  // movers by low / high arrival order
     const int L = threadIdx.x;
-    const int ntc = d.counts[1];
+    const int ntc = *P.ntc, replay = second ? 3 : 1;
     for (int i = blockIdx.x; i < ntc; i += gridDim.x) {
-        const int c = d.tc[i];
+        const int c = P.tc[i];
         // cells of a replica whose pass is replayed serially are left as the
         // move kernel left them (the same in every lane)
-        if (!d.mh[rep_of(d, c)]) {
+        const bool serial = (d.mh[rep_of(d, c)] & replay) != 0;
+        if (!serial) {
             const int len = d.meta[4 * c + 0];
             const int nhigh = d.meta[4 * c + 2];
-            int na = d.arr_cnt[c];
+            int na = P.arr_cnt[c];
             na = na < CM_ACAP ? na : CM_ACAP;
             int m = -1, src = 0, rk = 0;
             if (L < na) {
-                m = d.arr[c * CM_ACAP + L];
+                m = P.arr[c * CM_ACAP + L];
                 src = d.mv_slot[m] / CM_SLOTS;
                 rk = d.mv_rank[m];
             }
@@ -263,8 +347,8 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d)
             int gid = 0, git = 0;
             float4 gq = {0.0f, 0.0f, 0.0f, 0.0f};
             double gx = 0, gy = 0, gz = 0, gpx = 0, gpy = 0, gpz = 0;
+            int mv = -1, own = -1, mb = -1;
             if (L < nout) {
-                int mv = -1, own = -1;
                 if (L < keep) {
                     const int e = d.perm[c * CM_SLOTS + L];
                     if (e < CM_SLOTS) own = c * CM_SLOTS + e;
@@ -273,6 +357,7 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d)
                     mv = sm[1][(L - len) & (CM_SLOTS - 1)];
                 }
                 if (own >= 0) {
+                    if (FIRST && ((d.rb.leave[c] >> (own - c * CM_SLOTS)) & 1ull)) mb = d.mvidx[own];
                     gid = d.id[own];
                     gq = d.nlr[own];
                     git = d.itype[own];
@@ -309,11 +394,34 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d)
                 d.pz[o] = gpz;
             }
             if (L == 0) d.natoms[c] = nout;
+            if (FIRST) {
+                // pass B: the cell's own movers renamed, its arrivals' found
+                const int o = c * CM_SLOTS + L;
+                if (mb >= 0) {
+                    d.mvidx[o] = mb;
+                    d.mv_slot[mb] = o;
+                }
+                const Grid g = grid_of(d, c);
+                double bx = 0, by = 0, bz = 0;
+                int dstb = -1;
+                if (mv >= 0) {
+                    int ix, iy, iz;
+                    cell_xyz(g, c, ix, iy, iz);
+                    dstb = hop(g, c, ix, iy, iz, gx, gy, gz, bx, by, bz);
+                }
+                const unsigned long long leave = __ballot(mb >= 0 || dstb >= 0);
+                if (L == 0) d.rb.leave[c] = leave;
+                if (dstb >= 0) {
+                    if (hops_again(g, c, dstb, bx, by, bz)) atomicOr(&d.mh[g.pot], 2);
+                    put_mover(d, d.rb, c, o, dstb, Mover{bx, by, bz, gpx, gpy, gpz, gq, gid, git});
+                }
+            }
         }
         if (L == 0) {
-            d.arr_cnt[c] = 0;
-            d.touched[c] = 0;
-            d.leave[c] = 0;
+            P.arr_cnt[c] = 0;
+            P.touched[c] = 0;
+            // pass A's replay of a fused pair reads which atoms leave
+            if (!(FIRST && serial)) P.leave[c] = 0;
         }
         __syncthreads();
     }
@@ -337,31 +445,43 @@ __device__ static void serial_copy(const DevState &d, int from, int to)
     d.pz[to] = d.pz[from];
 }
 
-__global__ void k_rebox_serial(DevState d)
+// One pass over the cells of grid g.  FIRST: pass A of a fused pair: the atoms
+// of ra.leave hold their position of before the second drift and are
+// examined, with their arrivals in cells yet to come; each is drifted (by dtd)
+// where it ends.  The others have moved on already and stay.
+template <int FIRST>
+__device__ static unsigned serial_pass(const DevState &d, const Grid &g, double dtd)
 {
-    if (threadIdx.x != 0) return;
-    const int r = blockIdx.x;
-    if (r == 0) {
-        d.counts[0] = 0;
-        d.counts[1] = 0;
-    }
-    if (!d.mh[r]) return;
-    const Grid g = d.ngrids == 1 ? d.g0 : d.grids[r];
     unsigned fl = 0;
+    unsigned long long *leave = d.ra.leave;
+    auto settle = [&](int s, int ix, int iy, int iz) {
+        double x = d.rx[s], y = d.ry[s], z = d.rz[s];
+        x = x + dtd * d.px[s] / g.rmass;
+        y = y + dtd * d.py[s] / g.rmass;
+        z = z + dtd * d.pz[s] / g.rmass;
+        d.rx[s] = x;
+        d.ry[s] = y;
+        d.rz[s] = z;
+        if (d.nl_pos) {
+            double cx, cy, cz;
+            corner_of(g, ix, iy, iz, cx, cy, cz);
+            d.nl_pos[__float_as_int(d.nlr[s].w)] = CmPos{cx + x, cy + y, cz + z};
+        }
+    };
     for (int c = g.cell_base; c < g.cell_base + g.ncells; c++) {
         int ix, iy, iz;
         cell_xyz(g, c, ix, iy, iz);
         int i = 0;
         while (i < d.natoms[c]) {
             const int o = c * CM_SLOTS + i;
-            const double x = d.rx[o], y = d.ry[o], z = d.rz[o];
-            int nx = ix, ny = iy, nz = iz;
-            double ax = x, ay = y, az = z;
-            if (x < 0.0) { nx = ix - 1; ax = x + g.bs0; } else if (x >= g.bs0) { nx = ix + 1; ax = x - g.bs0; }
-            if (y < 0.0) { ny = iy - 1; ay = y + g.bs1; } else if (y >= g.bs1) { ny = iy + 1; ay = y - g.bs1; }
-            if (z < 0.0) { nz = iz - 1; az = z + g.bs2; } else if (z >= g.bs2) { nz = iz + 1; az = z - g.bs2; }
-            const int j = cell_wrap(g, nx, ny, nz);
-            if (j < 0 || j == c) {
+            if (FIRST && !((leave[c] >> i) & 1ull)) {
+                i++;
+                continue;
+            }
+            double ax, ay, az;
+            const int j = hop(g, c, ix, iy, iz, d.rx[o], d.ry[o], d.rz[o], ax, ay, az);
+            if (j < 0) {
+                if (FIRST) settle(o, ix, iy, iz);
                 i++;
                 continue;
             }
@@ -374,16 +494,50 @@ __global__ void k_rebox_serial(DevState d)
                 i++;
                 continue;
             }
-            serial_copy(d, o, j * CM_SLOTS + nj);
+            const int t = j * CM_SLOTS + nj;
+            serial_copy(d, o, t);
             d.natoms[j] = nj + 1;
             if (nj + 1 >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
+            if (FIRST) {
+                if (j > c) {
+                    leave[j] |= 1ull << nj;  // examined when its cell is
+                } else {
+                    int jx, jy, jz;
+                    cell_xyz(g, j, jx, jy, jz);
+                    settle(t, jx, jy, jz);
+                }
+            }
             // the cell's last atom fills the hole; none to move when the
             // departed atom was the last (a self-copy would point its id ->
             // slot entry back at the slot it left)
             const int ni = --d.natoms[c];
-            if (ni > i) serial_copy(d, c * CM_SLOTS + ni, o);
+            if (ni > i) {
+                serial_copy(d, c * CM_SLOTS + ni, o);
+                if (FIRST && !((leave[c] >> ni) & 1ull)) leave[c] &= ~(1ull << i);
+            }
+            if (FIRST && ni < CM_SLOTS) leave[c] &= ~(ni > i ? 1ull << ni : 1ull << i);
         }
+        if (FIRST) leave[c] = 0;
     }
+    return fl;
+}
+
+// fused: after a fused pair of half drifts (dtd: a half drift's time)
+__global__ void k_rebox_serial(DevState d, int fused, double dtd)
+{
+    if (threadIdx.x != 0) return;
+    const int r = blockIdx.x;
+    if (r == 0) {
+        d.counts[0] = 0;
+        d.counts[1] = 0;
+        d.counts[2] = 0;
+    }
+    const int mh = d.mh[r];
+    if (!mh) return;
+    const Grid g = d.ngrids == 1 ? d.g0 : d.grids[r];
+    unsigned fl = 0;
+    if (fused && (mh & 1)) fl |= serial_pass<1>(d, g, dtd);
+    fl |= serial_pass<0>(d, g, 0.0);
     d.mh[r] = 0;
     if (fl) atomicOr(d.flags, fl);
 }
@@ -460,23 +614,40 @@ __global__ void k_fill_int(int *p, int v, long n)
 // ---------------------------------------------------------------------------
 // host launchers
 
-void cm_launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, int kick, int drift, int rebin)
+template <int TWO>
+static void launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, int kick, int drift, int rebin)
 {
     if (d.ngrids == 1 && d.g0.cell_base == 0) {
         const dim3 grid((unsigned)((d.g0.nbx0 + 3) / 4), (unsigned)d.g0.nbx1, (unsigned)d.g0.nbx2);
-        hipLaunchKernelGGL(k_move4, grid, dim3(64), 0, st, d, dtk, dtd, kick, drift, rebin);
+        hipLaunchKernelGGL(k_move4<TWO>, grid, dim3(64), 0, st, d, dtk, dtd, kick, drift, rebin);
     } else {
-        hipLaunchKernelGGL(k_move, dim3((d.ncells + 3) / 4), dim3(64), 0, st, d, dtk, dtd, kick, drift, rebin);
+        hipLaunchKernelGGL(k_move<TWO>, dim3((d.ncells + 3) / 4), dim3(64), 0, st, d, dtk, dtd, kick, drift, rebin);
     }
 }
 
+void cm_launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, int kick, int drift, int rebin)
+{
+    launch_move<0>(d, st, dtk, dtd, kick, drift, rebin);
+}
+
+static int scan_blocks(const DevState &d) { return d.ncells < 8192 ? d.ncells : 8192; }
+static int gather_blocks(const DevState &d) { return d.ncells < 4096 ? d.ncells : 4096; }
+
 void cm_launch_rebox(const DevState &d, hipStream_t st)
 {
-    const int ns = d.ncells < 8192 ? d.ncells : 8192;
-    hipLaunchKernelGGL(k_rebox_scan, dim3(ns), dim3(64), 0, st, d);
-    const int ng = d.ncells < 4096 ? d.ncells : 4096;
-    hipLaunchKernelGGL(k_rebox_gather, dim3(ng), dim3(64), 0, st, d);
-    hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d);
+    hipLaunchKernelGGL(k_rebox_scan, dim3(scan_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
+    hipLaunchKernelGGL(k_rebox_gather<0>, dim3(gather_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
+    hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d, 0, 0.0);
+}
+
+void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd)
+{
+    launch_move<1>(d, st, dtk, dtd, 1, 1, 1);
+    hipLaunchKernelGGL(k_rebox_scan, dim3(scan_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
+    hipLaunchKernelGGL(k_rebox_gather<1>, dim3(gather_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
+    hipLaunchKernelGGL(k_rebox_scan, dim3(scan_blocks(d)), dim3(64), 0, st, d, d.rb, 1);
+    hipLaunchKernelGGL(k_rebox_gather<0>, dim3(gather_blocks(d)), dim3(64), 0, st, d, d.rb, 1);
+    hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d, 1, dtd);
 }
 
 void cm_launch_fill_int(int *p, int v, long n, hipStream_t st)

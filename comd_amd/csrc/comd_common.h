@@ -34,6 +34,16 @@ struct CmPos {
     double x, y, z;
 };
 
+// Bookkeeping of one rebin pass.
+struct RebinSet {
+    unsigned long long *leave;  // per cell: bit k set when slot k departs (cleared with touched)
+    int *touched;               // per cell: 1 while listed in tc
+    int *tc;                    // touched cells of the pass
+    int *ntc;                   // their number
+    int *arr_cnt;               // per cell: arrivals of the pass
+    int *arr;                   // per cell: up to 64 arriving mover indices
+};
+
 struct DevState {
     int ncells;              // cells of all replicas
     int ngrids;              // replicas
@@ -51,24 +61,21 @@ struct DevState {
     int *nnb;           // per slot: neighbours inside the cutoff (last density/LJ pass)
     float4 *nlr;        // per slot: the atom's FP32 position at the last list build (x, y, z)
                         // and its build position (w, int bits); moved with the atom
-    // rebin scratch
-    unsigned long long *leave;  // per cell: bit k set when slot k departs (cleared with touched)
+    // rebin scratch: the pass, and the second one of a fused pair of half
+    // drifts (rb)
+    RebinSet ra, rb;
     int *mvidx;         // per slot: index of its mover record (departing atoms)
     uint8_t *perm;      // per cell: arrangement after the cell's own scan
     int *meta;          // per cell: (len, nlow, nhigh, n0)
-    int *counts;        // [0] movers, [1] touched cells of the current pass
-    int *touched;       // per cell: 1 while listed in tc
-    int *tc;            // touched cells of the current pass
-    int *arr_cnt;       // per cell: arrivals of the current pass
-    int *arr;           // per cell: up to 64 arriving mover indices
+    int *counts;        // [0] movers of both passes, [1] and [2] touched cells of each
     // mover records: source slot, departure rank, and the atom with its
     // shifted coordinates
     int *mv_slot, *mv_rank, *mv_id, *mv_itype;
     float4 *mv_nlr;
     double *mv_rx, *mv_ry, *mv_rz, *mv_px, *mv_py, *mv_pz;
     unsigned *flags;    // error flag word
-    int *mh;            // per replica: an arrival of the current rebin pass would move again (the
-                        // replica's pass is then replayed serially)
+    int *mh;            // per replica: an arrival of the pass (bit 0), of a fused pair's second
+                        // pass (bit 1), would move again (the pass is then replayed serially)
     // pair lists of the EAM density pass, replayed by the embedding-force
     // pass (null when not kept): per cell CM_PLIST x 64 halo indices
     // ([entry][lane]), per slot-lane the entry count, per cell 1 when no

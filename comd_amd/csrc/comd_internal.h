@@ -130,6 +130,10 @@ int cm_force_lds_bytes(const PotDev &P, int kind, int mixed, int waves, int tab_
 
 void cm_launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, int kick, int drift, int rebin);
 void cm_launch_rebox(const DevState &d, hipStream_t st);
+// Kick, half drift, rebin, half drift, rebin in one pass over the atoms
+// (bin_rebox.hip); needs room for two mover records per atom (2 atoms <=
+// slots).
+void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd);
 void cm_launch_bin(const DevState &d, const Grid &g, hipStream_t st, int n, const double *xyz, const double *pxyz,
                    int itype, int *cnt, int *tmp);
 // Slot arrays in the reference's layout (r, p 3 and f 4 doubles per slot);
