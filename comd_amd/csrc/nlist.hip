@@ -537,42 +537,67 @@ __global__ __launch_bounds__(1024) void k_nl_build(DevState d, CmList l)
             l.selfh[t] = (uint16_t)self;
             const float4 pi = hl4[self];
             // the 27 stencil cells as 9 runs of three x-adjacent halo slots,
-            // whose atoms are contiguous in the halo; entries gathered 8 at a
-            // time and stored as one 16-byte group
+            // whose atoms are contiguous in the halo.  A run is tested 32
+            // atoms at a time into bit masks (first atom in the top bit), and
+            // the set bits then taken one by one: a list entry costs some 15
+            // instructions, and taken where it is found, in the loop over
+            // candidates, some lane of the wave has one nearly every time
+            // (build of 2 048 000 atoms 0.92 -> 0.75 ms, of which 0.56 are the
+            // candidate tests; 32 000 Lennard-Jones atoms 139 -> 96 us).  Entries are
+            // gathered 8 at a time in a 128-bit shift register (the first in
+            // the lowest bits) and stored as one 16-byte group
             int k = 0, nt = 0;
-            unsigned long long lo = 0, hi = 0;
+            unsigned w0 = 0, w1 = 0, w2 = 0, w3 = 0;
+            auto shift_in = [&](unsigned h) {
+                w0 = __builtin_amdgcn_alignbit(w1, w0, 16);
+                w1 = __builtin_amdgcn_alignbit(w2, w1, 16);
+                w2 = __builtin_amdgcn_alignbit(w3, w2, 16);
+                w3 = __builtin_amdgcn_alignbit(h, w3, 16);
+            };
             auto push = [&](int h) {
-                const int c8 = k & 7;
-                if (c8 < 4) lo |= (unsigned long long)h << (16 * c8);
-                else hi |= (unsigned long long)h << (16 * (c8 - 4));
-                if (c8 == 7 && k < l.kmax) {
-                    ulonglong2 w;
-                    w.x = lo;
-                    w.y = hi;
-                    *(ulonglong2 *)&l.nbl[nl_entry(k - 7, t, l.n)] = w;
-                    lo = hi = 0;
-                }
+                shift_in((unsigned)h);
                 k++;
+                if ((k & 7) == 0 && k <= l.kmax) *(v4u *)&l.nbl[nl_entry(k - 8, t, l.n)] = v4u{w0, w1, w2, w3};
             };
             for (int e = 0; e < 9; e++) {
                 const int s0 = (cx - 1) + shx * ((cy + e / 3 - 1) + shy * (cz + e % 3 - 1));
                 const int h1 = S.off[s0 + 3];
-                for (int h = S.off[s0]; h < h1; h++) {
-                    const float4 qh = hl4[h];
-                    const float dx = pi.x - qh.x, dy = pi.y - qh.y, dz = pi.z - qh.z;
-                    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                    if (r2 <= rl2 && h != self) {
-                        if (r2 > rc2 && nt < l.tailq) tq[(nt++) * blockDim.x] = (uint16_t)h;
-                        else push(h);
+                for (int hb = S.off[s0]; hb < h1; hb += 32) {
+                    // in: within cutoff + skin, far: beyond the cutoff (found
+                    // again per entry below instead: 8 % slower)
+                    unsigned in = 0, far = 0;
+#pragma unroll 1
+                    for (int j = 0; j < 32; j += 8) {
+                        if (hb + j >= h1) {
+                            in <<= 8;
+                            far <<= 8;
+                            continue;
+                        }
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            // (up to 7 entries past the run: within the block's LDS, masked below)
+                            const float4 qh = hl4[hb + j + u];
+                            const float dx = pi.x - qh.x, dy = pi.y - qh.y, dz = pi.z - qh.z;
+                            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                            in = in << 1 | (r2 <= rl2 ? 1u : 0u);
+                            far = far << 1 | (r2 > rc2 ? 1u : 0u);
+                        }
+                    }
+                    if (h1 - hb < 32) in &= ~0u << (32 - (h1 - hb));
+                    if ((unsigned)(self - hb) < 32u) in &= ~(0x80000000u >> (self - hb));
+                    while (in) {
+                        const int b = __builtin_clz(in);
+                        const unsigned bit = 0x80000000u >> b;
+                        in ^= bit;
+                        if ((far & bit) && nt < l.tailq) tq[(nt++) * blockDim.x] = (uint16_t)(hb + b);
+                        else push(hb + b);
                     }
                 }
             }
             for (int j = 0; j < nt; j++) push(tq[j * blockDim.x]);
             if ((k & 7) != 0 && k <= l.kmax) {
-                ulonglong2 w;
-                w.x = lo;
-                w.y = hi;
-                *(ulonglong2 *)&l.nbl[nl_entry(k & ~7, t, l.n)] = w;
+                for (int j = k & 7; j < 8; j++) shift_in(0u);
+                *(v4u *)&l.nbl[nl_entry(k & ~7, t, l.n)] = v4u{w0, w1, w2, w3};
             }
             l.ncnt[t] = min(k, l.kmax);
             ovf |= k > l.kmax;
@@ -1334,7 +1359,8 @@ void cm_nl_sync(const DevState &d, const CmList &l, hipStream_t st)
 
 size_t cm_nl_build_lds(const CmList &l)
 {
-    return (size_t)l.hcap * 16 + nl_slotmap_bytes(l.hcap) + (size_t)l.tailq * l.pass_threads * 2;
+    // (128: the search reads up to 7 entries past the halo)
+    return (size_t)l.hcap * 16 + nl_slotmap_bytes(l.hcap) + (size_t)l.tailq * l.pass_threads * 2 + 128;
 }
 
 int cm_nl_pick_tailq(CmList l)

@@ -284,3 +284,30 @@ def test_halo_tables_of_small_blocks(gpu, cu500, groups, div, precision, n):
     assert a.list_info()["builds"] > 1
     if precision == "fp64":  # mixed trajectories differ by their rounding
         assert_same(a, b, "after a rebuild", tol=1e-9)
+
+
+@pytest.mark.parametrize("per_cell", [1, 6, 10, 11, 18, 21, 30])
+def test_runs_of_every_length(gpu, per_cell):
+    """Runs of three cells of a few to some ninety atoms (the build tests 32
+    at a time, 8 by 8), uneven from cell to cell: the lists hold every pair
+    that the link cells find, each once."""
+    pot = CA.LJPotential(sigma=0.1, epsilon=1e-12, cutoff=2.0, mass=1.0)
+    rng = np.random.default_rng(per_cell)
+    bounds = np.array([14.6, 12.2, 10.1])
+    xyz = rng.uniform(0.0, 1.0, (int(per_cell * 210), 3)) * bounds
+    xyz[:: 3, 0] *= 0.7  # denser on one side
+    out = []
+    for skin in (0.4, 0.0):
+        s = CA.Simulation(pot, bounds)
+        s.tune(skin=skin)
+        s.bin_atoms(xyz)
+        s.force()
+        out.append(s)
+    a, b = out
+    assert a.list_info()["active"] == 1 and b.list_info()["active"] == 0
+    # from 21 on an auxiliary cell passes 64 atoms: the link cells take over
+    assert a.list_info()["valid"] == (1 if per_cell < 21 else 0)
+    m = np.arange(64)[None, :] < a.download()["natoms"][:, None]
+    na, nb = (s.download_aux()[0].reshape(-1, 64)[m] for s in out)
+    assert np.array_equal(na, nb)
+    assert a.pair_count() == b.pair_count()
