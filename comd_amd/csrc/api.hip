@@ -316,72 +316,65 @@ static bool any_eam(const comd_ctx *c)
     return false;
 }
 
-static void op_force(comd_ctx *c)
+// replay_dtd: after a fused pair of half drifts whose serial replay is still
+// to be checked for (op_middle), a half drift's time
+static void op_force(comd_ctx *c, double replay_dtd = 0.0)
 {
     DevState d = dev_state(c);
     const int mixed = c->precision == COMD_PREC_MIXED;
     hipEvent_t ev = nullptr;
     // with neighbour lists: the (usually skipped) list build, then each pass
-    // over the lists; the link-cell kernels run only if the lists are invalid
+    // over the lists.  Should they be invalid, the link cells do the pass,
+    // inside the list passes' launches (cells) until the host has seen it, by
+    // the link-cell kernels from then on.  With mixed Lennard-Jones passes,
+    // which do not hold that code, those kernels run beside the passes every
+    // time, on a small grid (idle beside valid lists) until then
     const bool nl = c->nl_active != 0;
+    const bool cells = !c->nl_invalid_seen && (c->nl_lj_groups == 0 || cm_nl_cells_inside(CM_KIND_LJ, mixed));
+    auto cfg_of = [&](int kind) {
+        ForceCfg cfg = force_cfg(c, kind, mixed);
+        if (nl && !c->nl_invalid_seen && cfg.blocks > c->ncu) cfg.blocks = c->ncu;
+        return cfg;
+    };
     if (nl) {
         tbegin(c, COMD_K_LIST_BUILD, &ev);
         if (c->nl_stale) {
             cm_nl_sync(d, c->nl, c->stream);
             c->nl_stale = 0;
         }
-        cm_nl_build(d, c->nl, c->stream);
+        cm_nl_build(d, c->nl, c->stream, c->nl_lj_groups > 0 ? c->nl_eam_groups : -1, replay_dtd);
         tend(c, COMD_K_LIST_BUILD, ev);
     }
+    auto lists = [&](int rep, int kind, int cls, int g0, int ng) {
+        tbegin(c, cls, &ev);
+        if (ng > 0) cm_nl_force(d, c->reps[rep].pot, c->nl, kind, mixed, c->stream, g0, ng, cells);
+        tend(c, cls, ev);
+    };
     if (c->nrep > 1) {
-        // lists: the EAM replicas' groups (density, then embedding force)
-        // and the LJ replicas' groups, each kind with its shared potential;
-        // then the link-cell passes over all replicas, which do the work
-        // when there are no lists and return at once beside valid ones
+        // the EAM replicas' groups (density, then embedding force) and the LJ
+        // replicas' groups, each kind with its shared potential
         if (nl) {
-            tbegin(c, COMD_K_DENSITY, &ev);
-            if (c->nl_eam_groups > 0)
-                cm_nl_force(d, c->reps[c->nl_eam_rep].pot, c->nl, CM_KIND_EAM1, mixed, c->stream, 0,
-                            c->nl_eam_groups);
-            if (c->nl_lj_groups > 0)
-                cm_nl_force(d, c->reps[c->nl_lj_rep].pot, c->nl, CM_KIND_LJ, mixed, c->stream, c->nl_eam_groups,
-                            c->nl_lj_groups);
-            tend(c, COMD_K_DENSITY, ev);
-            if (c->nl_eam_groups > 0) {
-                tbegin(c, COMD_K_EMBED_FORCE, &ev);
-                cm_nl_force(d, c->reps[c->nl_eam_rep].pot, c->nl, CM_KIND_EAM3, mixed, c->stream, 0,
-                            c->nl_eam_groups);
-                tend(c, COMD_K_EMBED_FORCE, ev);
-            }
+            lists(c->nl_eam_rep, CM_KIND_EAM1, COMD_K_DENSITY, 0, c->nl_eam_groups);
+            lists(c->nl_lj_rep, CM_KIND_LJ, COMD_K_DENSITY, c->nl_eam_groups, c->nl_lj_groups);
+            lists(c->nl_eam_rep, CM_KIND_EAM3, COMD_K_EMBED_FORCE, 0, c->nl_eam_groups);
+            if (cells) return;
         }
-        auto cells = [&](int pass, int kind, int cls) {
+        auto all = [&](int pass, int kind, int cls) {
             tbegin(c, nl ? COMD_K_CELL_FALLBACK : cls, &ev);
-            ForceCfg cfg = force_cfg(c, kind, mixed);
-            if (nl && !c->nl_invalid_seen && cfg.blocks > c->ncu) cfg.blocks = c->ncu;
-            cm_launch_force_batch(d, c->d_pots, pass, mixed, cfg, c->stream);
+            cm_launch_force_batch(d, c->d_pots, pass, mixed, cfg_of(kind), c->stream);
             tend(c, nl ? COMD_K_CELL_FALLBACK : cls, ev);
         };
-        cells(1, CM_KIND_EAM1, COMD_K_DENSITY);
-        if (any_eam(c)) cells(3, CM_KIND_EAM3, COMD_K_EMBED_FORCE);
+        all(1, CM_KIND_EAM1, COMD_K_DENSITY);
+        if (any_eam(c)) all(3, CM_KIND_EAM3, COMD_K_EMBED_FORCE);
         return;
     }
     const PotDev &P = c->reps[0].pot;
-    // one pass: the list kernel, then the link-cell kernel (which does the
-    // work when there are no lists, and returns at once while they are valid)
     auto pass = [&](int kind, int cls) {
-        if (nl) {
-            tbegin(c, cls, &ev);
-            cm_nl_force(d, P, c->nl, kind, mixed, c->stream, 0, c->nl.ngroups);
-            tend(c, cls, ev);
-        }
+        if (nl) lists(0, kind, cls, 0, c->nl.ngroups);
+        if (nl && cells) return;
         const int ccls = nl ? COMD_K_CELL_FALLBACK : cls;
         tbegin(c, ccls, &ev);
-        ForceCfg cfg = force_cfg(c, kind, mixed);
-        // beside valid lists the link-cell pass returns at once: a small grid
-        // keeps that cheap (the full grid once the host has seen the lists
-        // invalid)
-        if (nl && !c->nl_invalid_seen && cfg.blocks > c->ncu) cfg.blocks = c->ncu;
-        cm_launch_force(d, P, kind, mixed, cfg, c->stream);
+        cm_launch_force(d, P, kind, mixed, cfg_of(kind), c->stream);
         tend(c, ccls, ev);
     };
     if (P.kind == COMD_POT_LJ) {
@@ -404,13 +397,14 @@ static void op_step(comd_ctx *c, double dt)
 }
 
 // A step's force and the rest of it, with the first half drift and rebin of
-// the step after (cm_launch_move_two).
+// the step after (cm_launch_move_two).  With lists the force that follows, in
+// every case, checks for the serial replay in its first kernel.
 static void op_middle(comd_ctx *c, double dt)
 {
-    op_force(c);
+    op_force(c, dt / 2.0);
     hipEvent_t ev = nullptr;
     tbegin(c, COMD_K_REBIN, &ev);
-    cm_launch_move_two(dev_state(c), c->stream, dt, dt / 2.0);
+    cm_launch_move_two(dev_state(c), c->stream, dt, dt / 2.0, !c->nl_active);
     tend(c, COMD_K_REBIN, ev);
     c->nl_stale = 0;
 }
@@ -452,7 +446,7 @@ static int run_steps(comd_ctx *c, int n, double dt)
         if (c->nl_active) c->nl_stale = !fused;
     }
     if (fused) {
-        op_force(c);
+        op_force(c, dt / 2.0);
         op_move(c, dt, dt / 2.0, 1, 1, 1, 0);
         op_rebox(c);
     }

@@ -38,6 +38,7 @@
 // 100, with one launch of the serial kernel in place of two; a step of 256 000
 // atoms FP64 216 -> 190 us, of 864 atoms 62 -> 49 us.
 #include "comd_internal.h"
+#include "rebox_serial.h"
 
 #define CM_ACAP 64  // arrivals recorded per cell and pass
 
@@ -49,23 +50,6 @@ __device__ static inline void mark_touched(const RebinSet &p, int c)
     }
 }
 
-// Destination cell of an atom of cell c = (ix, iy, iz) at (x, y, z) by the
-// rules of reBoxAll (domains.c:356-377), -1 when it stays, and its position
-// in that cell.
-__device__ __forceinline__ int hop(const Grid &g, int c, int ix, int iy, int iz, double x, double y, double z,
-                                   double &ax, double &ay, double &az)
-{
-    int nx = ix, ny = iy, nz = iz;
-    ax = x;
-    ay = y;
-    az = z;
-    if (x < 0.0) { nx = ix - 1; ax = x + g.bs0; } else if (x >= g.bs0) { nx = ix + 1; ax = x - g.bs0; }
-    if (y < 0.0) { ny = iy - 1; ay = y + g.bs1; } else if (y >= g.bs1) { ny = iy + 1; ay = y - g.bs1; }
-    if (z < 0.0) { nz = iz - 1; az = z + g.bs2; } else if (z >= g.bs2) { nz = iz + 1; az = z - g.bs2; }
-    const int j = cell_wrap(g, nx, ny, nz);
-    return j == c ? -1 : j;
-}
-
 // An arrival in dst (above c) that is still outside it is moved again in the
 // same pass (it is examined again when dst is scanned).
 __device__ __forceinline__ bool hops_again(const Grid &g, int c, int dst, double ax, double ay, double az)
@@ -75,6 +59,14 @@ __device__ __forceinline__ bool hops_again(const Grid &g, int c, int dst, double
     cell_xyz(g, dst, jx, jy, jz);
     double bx, by, bz;
     return hop(g, dst, jx, jy, jz, ax, ay, az, bx, by, bz) >= 0;
+}
+
+// The replica's pass (bit 1) or a fused pair's second one (bit 2) is to be
+// replayed serially.
+__device__ __forceinline__ void request_replay(const DevState &d, const Grid &g, int bit)
+{
+    atomicOr(&d.mh[g.pot], bit);
+    atomicOr(&d.counts[3], 1);
 }
 
 struct Mover {
@@ -188,13 +180,13 @@ __device__ __forceinline__ void move_atom(const DevState &d, const Grid &g, int 
         double bx, by, bz;
         const int dstb = hop(g, c, ix, iy, iz, wx, wy, wz, bx, by, bz);
         if (dstb < 0) return;
-        if (hops_again(g, c, dstb, bx, by, bz)) atomicOr(&d.mh[g.pot], 2);
+        if (hops_again(g, c, dstb, bx, by, bz)) request_replay(d, g, 2);
         put_mover(d, d.rb, c, s, dstb, Mover{bx, by, bz, px, py, pz, d.nlr[s], d.id[s], d.itype[s]});
         atomicOr(&d.rb.leave[c], 1ull << (s - c * CM_SLOTS));
         return;
     }
     if (dst < 0) return;
-    if (hops_again(g, c, dst, ax, ay, az)) atomicOr(&d.mh[g.pot], 1);
+    if (hops_again(g, c, dst, ax, ay, az)) request_replay(d, g, 1);
     const Mover v = TWO ? Mover{wx, wy, wz, px, py, pz, d.nlr[s], d.id[s], d.itype[s]}
                         : Mover{ax, ay, az, px, py, pz, d.nlr[s], d.id[s], d.itype[s]};
     put_mover(d, d.ra, c, s, dst, v);
@@ -412,7 +404,7 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int
                 const unsigned long long leave = __ballot(mb >= 0 || dstb >= 0);
                 if (L == 0) d.rb.leave[c] = leave;
                 if (dstb >= 0) {
-                    if (hops_again(g, c, dstb, bx, by, bz)) atomicOr(&d.mh[g.pot], 2);
+                    if (hops_again(g, c, dstb, bx, by, bz)) request_replay(d, g, 2);
                     put_mover(d, d.rb, c, o, dstb, Mover{bx, by, bz, gpx, gpy, gpz, gq, gid, git});
                 }
             }
@@ -427,119 +419,13 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int
     }
 }
 
-// Serial pass of the replicas in which k_move found an arrival that would
-// move again (one block each, its first thread walking the replica's cells):
-// reBoxAll exactly as the reference runs it, in place.  Block 0 also clears
-// the pass counters.
-__device__ static void serial_copy(const DevState &d, int from, int to)
-{
-    if (d.nl_slot) d.nl_slot[grid_of(d, to / CM_SLOTS).nl_id_base + d.id[from]] = to;
-    d.id[to] = d.id[from];
-    d.nlr[to] = d.nlr[from];
-    d.itype[to] = d.itype[from];
-    d.rx[to] = d.rx[from];
-    d.ry[to] = d.ry[from];
-    d.rz[to] = d.rz[from];
-    d.px[to] = d.px[from];
-    d.py[to] = d.py[from];
-    d.pz[to] = d.pz[from];
-}
-
-// One pass over the cells of grid g.  FIRST: pass A of a fused pair: the atoms
-// of ra.leave hold their position of before the second drift and are
-// examined, with their arrivals in cells yet to come; each is drifted (by dtd)
-// where it ends.  The others have moved on already and stay.
-template <int FIRST>
-__device__ static unsigned serial_pass(const DevState &d, const Grid &g, double dtd)
-{
-    unsigned fl = 0;
-    unsigned long long *leave = d.ra.leave;
-    auto settle = [&](int s, int ix, int iy, int iz) {
-        double x = d.rx[s], y = d.ry[s], z = d.rz[s];
-        x = x + dtd * d.px[s] / g.rmass;
-        y = y + dtd * d.py[s] / g.rmass;
-        z = z + dtd * d.pz[s] / g.rmass;
-        d.rx[s] = x;
-        d.ry[s] = y;
-        d.rz[s] = z;
-        if (d.nl_pos) {
-            double cx, cy, cz;
-            corner_of(g, ix, iy, iz, cx, cy, cz);
-            d.nl_pos[__float_as_int(d.nlr[s].w)] = CmPos{cx + x, cy + y, cz + z};
-        }
-    };
-    for (int c = g.cell_base; c < g.cell_base + g.ncells; c++) {
-        int ix, iy, iz;
-        cell_xyz(g, c, ix, iy, iz);
-        int i = 0;
-        while (i < d.natoms[c]) {
-            const int o = c * CM_SLOTS + i;
-            if (FIRST && !((leave[c] >> i) & 1ull)) {
-                i++;
-                continue;
-            }
-            double ax, ay, az;
-            const int j = hop(g, c, ix, iy, iz, d.rx[o], d.ry[o], d.rz[o], ax, ay, az);
-            if (j < 0) {
-                if (FIRST) settle(o, ix, iy, iz);
-                i++;
-                continue;
-            }
-            d.rx[o] = ax;
-            d.ry[o] = ay;
-            d.rz[o] = az;
-            const int nj = d.natoms[j];
-            if (nj >= CM_SLOTS) {  // no room: the reference aborts here
-                fl |= CM_FLAG_OVERFLOW;
-                i++;
-                continue;
-            }
-            const int t = j * CM_SLOTS + nj;
-            serial_copy(d, o, t);
-            d.natoms[j] = nj + 1;
-            if (nj + 1 >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
-            if (FIRST) {
-                if (j > c) {
-                    leave[j] |= 1ull << nj;  // examined when its cell is
-                } else {
-                    int jx, jy, jz;
-                    cell_xyz(g, j, jx, jy, jz);
-                    settle(t, jx, jy, jz);
-                }
-            }
-            // the cell's last atom fills the hole; none to move when the
-            // departed atom was the last (a self-copy would point its id ->
-            // slot entry back at the slot it left)
-            const int ni = --d.natoms[c];
-            if (ni > i) {
-                serial_copy(d, c * CM_SLOTS + ni, o);
-                if (FIRST && !((leave[c] >> ni) & 1ull)) leave[c] &= ~(1ull << i);
-            }
-            if (FIRST && ni < CM_SLOTS) leave[c] &= ~(ni > i ? 1ull << ni : 1ull << i);
-        }
-        if (FIRST) leave[c] = 0;
-    }
-    return fl;
-}
-
 // fused: after a fused pair of half drifts (dtd: a half drift's time)
 __global__ void k_rebox_serial(DevState d, int fused, double dtd)
 {
     if (threadIdx.x != 0) return;
-    const int r = blockIdx.x;
-    if (r == 0) {
-        d.counts[0] = 0;
-        d.counts[1] = 0;
-        d.counts[2] = 0;
-    }
-    const int mh = d.mh[r];
-    if (!mh) return;
-    const Grid g = d.ngrids == 1 ? d.g0 : d.grids[r];
-    unsigned fl = 0;
-    if (fused && (mh & 1)) fl |= serial_pass<1>(d, g, dtd);
-    fl |= serial_pass<0>(d, g, 0.0);
-    d.mh[r] = 0;
-    if (fl) atomicOr(d.flags, fl);
+    if (blockIdx.x == 0)
+        for (int k = 0; k < 4; k++) d.counts[k] = 0;
+    replay_replica(d, blockIdx.x, fused, dtd);
 }
 
 // ---------------------------------------------------------------------------
@@ -640,14 +526,14 @@ void cm_launch_rebox(const DevState &d, hipStream_t st)
     hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d, 0, 0.0);
 }
 
-void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd)
+void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd, int serial)
 {
     launch_move<1>(d, st, dtk, dtd, 1, 1, 1);
     hipLaunchKernelGGL(k_rebox_scan, dim3(scan_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
     hipLaunchKernelGGL(k_rebox_gather<1>, dim3(gather_blocks(d)), dim3(64), 0, st, d, d.ra, 0);
     hipLaunchKernelGGL(k_rebox_scan, dim3(scan_blocks(d)), dim3(64), 0, st, d, d.rb, 1);
     hipLaunchKernelGGL(k_rebox_gather<0>, dim3(gather_blocks(d)), dim3(64), 0, st, d, d.rb, 1);
-    hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d, 1, dtd);
+    if (serial) hipLaunchKernelGGL(k_rebox_serial, dim3((unsigned)d.ngrids), dim3(64), 0, st, d, 1, dtd);
 }
 
 void cm_launch_fill_int(int *p, int v, long n, hipStream_t st)

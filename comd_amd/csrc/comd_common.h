@@ -67,7 +67,8 @@ struct DevState {
     int *mvidx;         // per slot: index of its mover record (departing atoms)
     uint8_t *perm;      // per cell: arrangement after the cell's own scan
     int *meta;          // per cell: (len, nlow, nhigh, n0)
-    int *counts;        // [0] movers of both passes, [1] and [2] touched cells of each
+    int *counts;        // [0] movers of both passes, [1] and [2] touched cells of each,
+                        // [3] a replica's pass is to be replayed (any bit of mh)
     // mover records: source slot, departure rank, and the atom with its
     // shifted coordinates
     int *mv_slot, *mv_rank, *mv_id, *mv_itype;

@@ -132,8 +132,9 @@ void cm_launch_move(const DevState &d, hipStream_t st, double dtk, double dtd, i
 void cm_launch_rebox(const DevState &d, hipStream_t st);
 // Kick, half drift, rebin, half drift, rebin in one pass over the atoms
 // (bin_rebox.hip); needs room for two mover records per atom (2 atoms <=
-// slots).
-void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd);
+// slots).  serial 0: the replay and the counters' reset are left to the list
+// check that follows (cm_nl_build with this dtd).
+void cm_launch_move_two(const DevState &d, hipStream_t st, double dtk, double dtd, int serial);
 void cm_launch_bin(const DevState &d, const Grid &g, hipStream_t st, int n, const double *xyz, const double *pxyz,
                    int itype, int *cnt, int *tmp);
 // Slot arrays in the reference's layout (r, p 3 and f 4 doubles per slot);
@@ -274,7 +275,7 @@ struct CmList {
     int gwords;              // words of four entries per thread: ceil(hcap / (4 pass_threads))
     int *nonempty;           // per link cell: non-empty stencil cells (Lennard-Jones virial)
     int *count;              // [0]: atoms in build order, [1]: builds so far, [2]: build blocks done,
-                             // [3]: group-sum blocks done
+                             // [3]: k_nl_key blocks done
     unsigned *flags;         // CM_NL_REBUILD, CM_NL_INVALID, CM_NL_OVERFLOW (during a build)
 };
 #define CM_NL_AUXCAP 64
@@ -283,7 +284,7 @@ struct CmList {
 #define CM_NL_STATIC_LDS (6 << 10)      // static LDS of the list kernels, rounded up
 __host__ __device__ inline size_t nl_entry(int k, int t, int n) { return ((size_t)(k >> 3) * n + t) * 8 + (k & 7); }
 void cm_nl_init(const DevState &d, const CmList &l, hipStream_t st);
-void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st);
+void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st, int lj_g0, double dtd);
 void cm_nl_sync(const DevState &d, const CmList &l, hipStream_t st);
 void cm_nl_tables(const CmList &l, hipStream_t st);
 size_t cm_nl_build_lds(const CmList &l);
@@ -292,11 +293,14 @@ size_t cm_nl_build_lds(const CmList &l);
 int cm_nl_pick_tailq(CmList l);
 size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int *tables_in_lds);
 size_t cm_nl_tab_bytes(const PotDev &P, int kind, int mixed);
+// Whether a pass can do the link cells' work itself (nlist.hip).
+bool cm_nl_cells_inside(int kind, int mixed);
 // The list pass of one kind over groups [g0, g0 + ng) (a single
 // simulation: all of them; a batch: the groups of its EAM or of its LJ
-// replicas, which share one potential).
+// replicas, which share one potential).  cells: the launch does the pass over
+// the link cells itself if the lists are invalid.
 void cm_nl_force(const DevState &d, const PotDev &P, const CmList &l, int kind, int mixed, hipStream_t st, int g0,
-                 int ng);
+                 int ng, int cells);
 // Resident blocks per CU of a list pass (-1 if the runtime cannot tell) and
 // its dynamic LDS bytes.
 int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int *lds_bytes);

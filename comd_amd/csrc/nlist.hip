@@ -30,7 +30,8 @@
 // link-cell kernels otherwise.
 #include "comd_internal.h"
 #include "adj_basis.h"
-#include "pair_terms.h"
+#include "pair_cell.h"
+#include "rebox_serial.h"
 
 #include <type_traits>
 
@@ -313,18 +314,17 @@ __device__ __forceinline__ void frame_pos(const NlRep &R, const GroupGeo &G, int
 // launches that find no request cost only their dispatch: their grids are
 // kept small, with strided loops)
 
-// Each atom into its auxiliary cell (counts start at zero: the previous
-// build's last block cleared them).  Atoms taken in slot order, 16 lanes per
-// link cell (its atoms beyond 16 in further rounds), so that the positions
-// and ids are read in whole lines; the order within an auxiliary cell is
-// set by k_nl_sort.  Ids outside the replica's range are left out, as
-// k_nl_from_slots leaves them out of the id -> slot map (and marks the
-// lists invalid).
-__global__ __launch_bounds__(256) void k_nl_key(DevState d, CmList l)
+// The cells' work of k_nl_key for blocks b of nb: each atom into its auxiliary
+// cell (counts start at zero: the previous build's last block cleared them).
+// Atoms taken in slot order, 16 lanes per link cell (its atoms beyond 16 in
+// further rounds), so that the positions and ids are read in whole lines; the
+// order within an auxiliary cell is set by k_nl_sort.  Ids outside the
+// replica's range are left out, as k_nl_from_slots leaves them out of the
+// id -> slot map (and marks the lists invalid).
+__device__ static void key_cells(const DevState &d, const CmList &l, int b, int nb)
 {
-    if (!nl_rebuild(l)) return;
     const int sub = threadIdx.x & 15;
-    const int c0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 4), dc = (int)((gridDim.x * blockDim.x) >> 4);
+    const int c0 = (int)((b * blockDim.x + threadIdx.x) >> 4), dc = (int)((nb * blockDim.x) >> 4);
     for (int c = c0; c < d.ncells; c += dc) {
         const int n = d.natoms[c];
         if (sub >= n) continue;
@@ -344,44 +344,76 @@ __global__ __launch_bounds__(256) void k_nl_key(DevState d, CmList l)
     }
 }
 
-// Per group (one wave each; a group has at most 64 cells): its cells' atom
-// counts (capped) and their exclusive offsets within the group in build
-// order; the block that finishes last then turns the group totals into each
-// group's first atom (an exclusive prefix sum, gstart) and count[0].
-__global__ __launch_bounds__(256) void k_nl_gsum(CmList l)
+// Non-empty stencil cells of each link cell, for blocks b of nb: the reference
+// adds the kinetic virial term once per non-empty neighbour cell
+// (src-flat/ljForce.c:175).  Cells of the replicas whose groups start at g0 or
+// later (the Lennard-Jones ones); the 27 entries of stencil_cell, duplicates
+// included, their loads in flight together.
+__device__ static void nonempty_cells(const DevState &d, const CmList &l, int g0, int b, int nb)
 {
-    if (!nl_rebuild(l)) return;
-    __shared__ int wsum[4];
-    __shared__ int carry_s, last;
-    const int t = threadIdx.x, L = t & 63, w = t >> 6;
-    for (int g = blockIdx.x * 4 + w; g < l.ngroups; g += gridDim.x * 4) {
-        const int q0 = l.group_q0[g], nq = l.group_q0[g + 1] - q0;
-        int a = 0, v = 0;
-        if (L < nq) {
-            a = l.cell_order[q0 + L];
-            v = min(l.aux_cnt[a], CM_NL_AUXCAP);
+    for (int c = b * blockDim.x + threadIdx.x; c < d.ncells; c += nb * blockDim.x) {
+        if (g0 > 0 && l.rep[rep_of(d, c)].group_base < g0) continue;
+        const Grid g = grid_of(d, c);
+        int n = 0;
+        if (g.ncells == 1) {
+            n = d.natoms[c] > 0;
+        } else {
+            int ix, iy, iz;
+            cell_xyz(g, c, ix, iy, iz);
+#pragma unroll
+            for (int ox = -1; ox <= 1; ox++)
+#pragma unroll
+                for (int oy = -1; oy <= 1; oy++)
+#pragma unroll
+                    for (int oz = -1; oz <= 1; oz++) {
+                        const int j = cell_wrap(g, ix + ox, iy + oy, iz + oz);
+                        n += d.natoms[j < 0 ? c : j] > 0 && j >= 0;
+                    }
         }
-        int incl = v;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int u = __shfl_up(incl, o, 64);
-            if (L >= o) incl += u;
+        l.nonempty[c] = n;
+    }
+}
+
+// Per group (one wave each, eight groups' loads in flight; a group has at most
+// 64 cells): its cells' atom counts (capped) and their exclusive offsets within
+// the group in build order; then each group's first atom (an exclusive prefix
+// sum, gstart) and count[0].  One block; the counts are read as the other
+// blocks' atomics left them.
+__device__ static void group_starts(const CmList &l)
+{
+    __shared__ int wsum[16];
+    __shared__ int carry_s;
+    const int t = threadIdx.x, L = t & 63, w = t >> 6, nw = blockDim.x >> 6;
+    constexpr int GB = 8;
+    for (int gb = GB * w; gb < l.ngroups; gb += GB * nw) {
+        int nq[GB], a[GB], v[GB];
+#pragma unroll
+        for (int k = 0; k < GB; k++) {
+            const int g = min(gb + k, l.ngroups - 1), q0 = l.group_q0[g];
+            nq[k] = l.group_q0[g + 1] - q0;
+            a[k] = l.cell_order[q0 + min(L, nq[k] - 1)];
         }
-        if (L < nq) {
-            l.aux_start[a] = incl - v;
-            l.aux_n[a] = v;
+#pragma unroll
+        for (int k = 0; k < GB; k++) v[k] = __hip_atomic_load(&l.aux_cnt[a[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int k = 0; k < GB; k++) {
+            if (gb + k >= l.ngroups) break;
+            const int n = L < nq[k] ? min(v[k], CM_NL_AUXCAP) : 0;
+            int incl = n;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(incl, o, 64);
+                if (L >= o) incl += u;
+            }
+            if (L < nq[k]) {
+                l.aux_start[a[k]] = incl - n;
+                l.aux_n[a[k]] = n;
+            }
+            if (L == 63) l.gstart[gb + k] = incl;  // the group's total, for now
         }
-        if (L == 63) l.gstart[g] = incl;  // the group's total, for now
     }
     __syncthreads();
-    if (t == 0) {
-        __threadfence();
-        last = atomicAdd(&l.count[3], 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
     int carry = 0;
-    for (int base = 0; base < l.ngroups; base += 4 * 256) {
+    for (int base = 0; base < l.ngroups; base += 4 * (int)blockDim.x) {
         int v[4], s = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -398,7 +430,7 @@ __global__ __launch_bounds__(256) void k_nl_gsum(CmList l)
         __syncthreads();
         if (t == 0) {
             int run = 0;
-            for (int k = 0; k < 4; k++) {
+            for (int k = 0; k < nw; k++) {
                 const int x = wsum[k];
                 wsum[k] = run;
                 run += x;
@@ -419,8 +451,47 @@ __global__ __launch_bounds__(256) void k_nl_gsum(CmList l)
     if (t == 0) {
         l.count[0] = carry;
         l.gstart[l.ngroups] = carry;
-        l.count[3] = 0;
     }
+}
+
+// The first kernel of every force call over lists: the serial replay of a
+// fused pair of half drifts, where one asked for it; the Lennard-Jones virial's
+// cell counts (lj_g0 >= 0); and, when a rebuild was requested, the atoms'
+// auxiliary cells and, by the block that finishes last, the groups' first
+// atoms.  One launch: an idle one costs 2 us (a small system) to 4.5 us (the
+// TLBs and caches turned over by the passes between), and apart these were
+// four.  With the link cells' code inside the passes (cells_instead) a step's
+// launches are ten in place of fifteen: 864 atoms 53 -> 46 us, 32 000
+// Lennard-Jones atoms 71 -> 64, 256 000 atoms FP64 181 -> 175.  No fence per block
+// is needed: the last block reads only what atomics wrote, except after a
+// replay (rare: its blocks fence, and the last one does the cells' work alone,
+// once every replica is settled).
+#define CM_KEY_BLOCKS 256
+#define CM_KEY_THREADS 1024
+__global__ __launch_bounds__(CM_KEY_THREADS) void k_nl_key(DevState d, CmList l, int lj_g0, double dtd)
+{
+    __shared__ int last;
+    const bool replay = d.counts[3] != 0, build = nl_rebuild(l);
+    if (!replay) {
+        if (lj_g0 >= 0) nonempty_cells(d, l, lj_g0, blockIdx.x, gridDim.x);
+        if (!build) return;
+        key_cells(d, l, blockIdx.x, gridDim.x);
+    } else if (threadIdx.x == 0) {
+        for (int r = blockIdx.x; r < d.ngrids; r += gridDim.x) replay_replica(d, r, 1, dtd);
+        __threadfence();
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&l.count[3], 1) == (int)gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    if (replay) {
+        __threadfence();
+        if (lj_g0 >= 0) nonempty_cells(d, l, lj_g0, 0, 1);
+        if (build) key_cells(d, l, 0, 1);
+        __syncthreads();
+    }
+    if (build) group_starts(l);
+    if (threadIdx.x == 0) l.count[3] = 0;
 }
 
 // Members of each auxiliary cell in id order (deterministic lists), placed in
@@ -472,6 +543,8 @@ __host__ __device__ constexpr int nl_slotmap_bytes(int hcap) { return (hcap + 15
 // for the next build.
 __global__ __launch_bounds__(1024) void k_nl_build(DevState d, CmList l)
 {
+    // the rebin's counters, read by k_nl_key just before
+    if (blockIdx.x == 0 && threadIdx.x < 4) d.counts[threadIdx.x] = 0;
     if (!nl_rebuild(l)) return;
     extern __shared__ float4 hl4[];  // [hcap] frame x, y, z; then the slot map
     CM_LDS uint8_t *slot_of = (CM_LDS uint8_t *)((CM_LDS char *)hl4 + (size_t)l.hcap * 16);
@@ -643,35 +716,11 @@ __global__ __launch_bounds__(1024) void k_nl_tables(CmList l)
 }
 
 // ---------------------------------------------------------------------------
-// force passes over the lists (return at once when the lists are invalid;
-// the link-cell kernels then run instead)
-
-// Non-empty stencil cells of each link cell: the reference adds the kinetic
-// virial term once per non-empty neighbour cell (src-flat/ljForce.c:175).
-// Cells of the replicas whose groups start at g0 or later (the
-// Lennard-Jones ones); the 27 entries of stencil_cell, duplicates included.
-__global__ void k_nl_nonempty(DevState d, CmList l, int g0)
-{
-    if (l.flags[0] & CM_NL_INVALID) return;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= d.ncells) return;
-    if (g0 > 0 && l.rep[rep_of(d, c)].group_base < g0) return;
-    const Grid g = grid_of(d, c);
-    int n = 0;
-    if (g.ncells == 1) {
-        n = d.natoms[c] > 0;
-    } else {
-        int ix, iy, iz;
-        cell_xyz(g, c, ix, iy, iz);
-        for (int ox = -1; ox <= 1; ox++)
-            for (int oy = -1; oy <= 1; oy++)
-                for (int oz = -1; oz <= 1; oz++) {
-                    const int b = cell_wrap(g, ix + ox, iy + oy, iz + oz);
-                    n += b >= 0 && d.natoms[b] > 0;
-                }
-    }
-    l.nonempty[c] = n;
-}
+// force passes over the lists.  When the lists are invalid the link cells do
+// the pass instead: inside the same launch until the host has seen it
+// (cells_instead), by their own kernels on a full grid from then on.  Launched
+// beside the list passes every time, those kernels' idle launches took 4.6 us
+// each (256 000 atoms and more; 3 us at 864).
 
 // Chebyshev passes: N pairs of a list chunk evaluated together, each series
 // as N interleaved Clenshaw recurrences (src-flat/cheby.c:276-310) that
@@ -1093,6 +1142,43 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
     }
 }
 
+__host__ __device__ constexpr bool nl_cells_inside(int kind, int mixed) { return !(kind == CM_KIND_LJ && mixed); }
+
+// The link cells' work of a pass whose lists are invalid, dealt to the waves
+// that the block's LDS has room for.  Replicas of the launch's kind: those with
+// groups in [gbase, gbase + gridDim.x).
+template <int KIND, int EVAL, int MIXED>
+__device__ __forceinline__ void cells_instead(const DevState &d, const PotDev &P, const CmList &l, char *lds, int lds_bytes,
+                                              int gbase)
+{
+    const int W = min((int)blockDim.x >> 6, lds_bytes / wave_lds_bytes(KIND)), wv = (int)threadIdx.x >> 6;
+    if (wv >= W) return;
+    const WaveLds w = carve(lds + wv * wave_lds_bytes(KIND), KIND);
+    for (int c = (int)blockIdx.x * W + wv; c < d.ncells; c += (int)gridDim.x * W) {
+        if (d.ngrids > 1) {
+            const int b = l.rep[rep_of(d, c)].group_base;
+            if (b < gbase || b >= gbase + (int)gridDim.x) continue;
+        }
+        pair_cell<KIND, EVAL, MIXED>(d, grid_of(d, c), P, w, c, (int)threadIdx.x & 63);
+    }
+}
+
+// The passes that hold the link cells' code: all but the mixed Lennard-Jones
+// pass, whose 71 registers its 104 would raise past six waves per SIMD, or
+// spill (64 replicas, the pass 103 -> 131 us).
+bool cm_nl_cells_inside(int kind, int mixed) { return nl_cells_inside(kind, mixed); }
+
+// Waves per SIMD that a pass keeps registers for: as many as it has room for
+// without the link cells' code (cells_instead: 104 to 114 registers, spilled
+// there where that is more), and two blocks of 12 waves per CU in the mixed
+// table passes.
+constexpr int nl_pass_waves(int kind, int eval, int mixed, int lanes)
+{
+    if (kind == CM_KIND_LJ) return mixed ? 1 : 5;
+    if (!mixed) return 1;
+    return eval == COMD_EVAL_CHEB && kind == CM_KIND_EAM1 ? 5 - lanes : 6;
+}
+
 // A block per group: the halo is staged in LDS in the group's frame (origin
 // at the centre of the group's cells), then each thread takes home atoms.
 // TLDS: the compact table rows are staged in LDS (1), or the full tables are
@@ -1103,12 +1189,17 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
 // registers three waves per SIMD allow.
 template <int KIND, int EVAL, int MIXED, int TLDS, int LANES>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, EVAL == COMD_EVAL_CHEB ? 768 : 1024)))
-__attribute__((amdgpu_waves_per_eu(MIXED && KIND != CM_KIND_LJ && TLDS ? 6 : 1)))
-void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase)
+__attribute__((amdgpu_waves_per_eu(nl_pass_waves(KIND, EVAL, MIXED, LANES))))
+void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase, int cells_lds)
 {
     extern __shared__ __align__(16) char nls[];
     __shared__ PassLds S;
-    if (l.flags[0] & CM_NL_INVALID) return;
+    if (l.flags[0] & CM_NL_INVALID) {
+        if constexpr (nl_cells_inside(KIND, MIXED)) {
+            if (cells_lds) cells_instead<KIND, EVAL, MIXED>(d, P, l, nls, cells_lds, gbase);
+        }
+        return;
+    }
     CM_LDS char *halo = (CM_LDS char *)nls + tab_bytes;
     CM_LDS v4u *hq = (CM_LDS v4u *)halo;
     CM_LDS double *hx = (CM_LDS double *)halo, *hy = hx + l.hcap, *hz = hy + l.hcap, *hf = hz + l.hcap;
@@ -1383,10 +1474,10 @@ int cm_nl_pick_tailq(CmList l)
     return 0;
 }
 
-void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st)
+void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st, int lj_g0, double dtd)
 {
-    hipLaunchKernelGGL(k_nl_key, dim3(1024), dim3(256), 0, st, d, l);
-    hipLaunchKernelGGL(k_nl_gsum, dim3((unsigned)std::min(4096, (l.ngroups + 3) / 4)), dim3(256), 0, st, l);
+    const unsigned blocks = (unsigned)std::min<long>(CM_KEY_BLOCKS, ((long)d.ncells * 16 + CM_KEY_THREADS - 1) / CM_KEY_THREADS);
+    hipLaunchKernelGGL(k_nl_key, dim3(blocks), dim3(CM_KEY_THREADS), 0, st, d, l, lj_g0, dtd);
     hipLaunchKernelGGL(k_nl_sort, dim3(1024), dim3(256), 0, st, l);
     hipLaunchKernelGGL(k_nl_build, dim3(l.pass_blocks), dim3(l.pass_threads), cm_nl_build_lds(l), st, d, l);
 }
@@ -1408,21 +1499,23 @@ size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int
 }
 
 template <int KIND, int EVAL, int MIXED>
-static void nl_launch(const DevState &d, const PotDev &P, const CmList &l, hipStream_t st, int g0, int ng)
+static void nl_launch(const DevState &d, const PotDev &P, const CmList &l, hipStream_t st, int g0, int ng, int cells)
 {
     int tl = 0;
-    const size_t lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
+    size_t lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
     const int tab = tl ? (int)nl_tab_bytes(P, KIND, MIXED) : 0;
+    if (cells) lds = std::max<size_t>(lds, wave_lds_bytes(KIND));
+    const int cl = cells ? (int)lds : 0;
     const dim3 grid(ng), block(l.pass_threads);
     if constexpr (EVAL == COMD_EVAL_TABLE && KIND != CM_KIND_LJ) {
         if (tl) {
-            if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 1>), grid, block, lds, st, d, P, l, tab, g0);
-            else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 0>), grid, block, lds, st, d, P, l, tab, g0);
+            if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 1>), grid, block, lds, st, d, P, l, tab, g0, cl);
+            else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 0>), grid, block, lds, st, d, P, l, tab, g0, cl);
             return;
         }
     }
-    if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 1>), grid, block, lds, st, d, P, l, 0, g0);
-    else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 0>), grid, block, lds, st, d, P, l, 0, g0);
+    if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 1>), grid, block, lds, st, d, P, l, 0, g0, cl);
+    else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 0>), grid, block, lds, st, d, P, l, 0, g0, cl);
 }
 
 // Resident blocks per CU of the pass nl_launch would start, and its dynamic LDS.
@@ -1462,25 +1555,25 @@ int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int *
 }
 
 template <int KIND, int EVAL>
-static void nl_launch2(const DevState &d, const PotDev &P, const CmList &l, int mixed, hipStream_t st, int g0, int ng)
+static void nl_launch2(const DevState &d, const PotDev &P, const CmList &l, int mixed, hipStream_t st, int g0, int ng,
+                       int cells)
 {
-    if (mixed) nl_launch<KIND, EVAL, 1>(d, P, l, st, g0, ng);
-    else nl_launch<KIND, EVAL, 0>(d, P, l, st, g0, ng);
+    if (mixed) nl_launch<KIND, EVAL, 1>(d, P, l, st, g0, ng, cells);
+    else nl_launch<KIND, EVAL, 0>(d, P, l, st, g0, ng, cells);
 }
 
 void cm_nl_force(const DevState &d, const PotDev &P, const CmList &l, int kind, int mixed, hipStream_t st, int g0,
-                 int ng)
+                 int ng, int cells)
 {
     if (ng <= 0) return;
     if (kind == CM_KIND_LJ) {
-        hipLaunchKernelGGL(k_nl_nonempty, dim3(grid_for(d.ncells, 256)), dim3(256), 0, st, d, l, g0);
-        nl_launch2<CM_KIND_LJ, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng);
+        nl_launch2<CM_KIND_LJ, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng, cells);
     } else if (P.eval == COMD_EVAL_CHEB) {
-        if (kind == CM_KIND_EAM1) nl_launch2<CM_KIND_EAM1, COMD_EVAL_CHEB>(d, P, l, mixed, st, g0, ng);
-        else nl_launch2<CM_KIND_EAM3, COMD_EVAL_CHEB>(d, P, l, mixed, st, g0, ng);
+        if (kind == CM_KIND_EAM1) nl_launch2<CM_KIND_EAM1, COMD_EVAL_CHEB>(d, P, l, mixed, st, g0, ng, cells);
+        else nl_launch2<CM_KIND_EAM3, COMD_EVAL_CHEB>(d, P, l, mixed, st, g0, ng, cells);
     } else {
-        if (kind == CM_KIND_EAM1) nl_launch2<CM_KIND_EAM1, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng);
-        else nl_launch2<CM_KIND_EAM3, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng);
+        if (kind == CM_KIND_EAM1) nl_launch2<CM_KIND_EAM1, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng, cells);
+        else nl_launch2<CM_KIND_EAM3, COMD_EVAL_TABLE>(d, P, l, mixed, st, g0, ng, cells);
     }
 }
 

@@ -311,3 +311,50 @@ def test_runs_of_every_length(gpu, per_cell):
     na, nb = (s.download_aux()[0].reshape(-1, 64)[m] for s in out)
     assert np.array_equal(na, nb)
     assert a.pair_count() == b.pair_count()
+
+
+# (a mixed batch takes smaller auxiliary cells, which hold this box)
+@pytest.mark.parametrize("kind,precision", [("table", "fp64"), ("table", "mixed"), ("cheby", "fp64"), ("cheby", "mixed"),
+                                            ("lj", "fp64"), ("lj", "mixed"), ("batch", "fp64")])
+def test_invalid_lists_inside_and_beside_the_passes(gpu, cu500, kind, precision):
+    """Boxes whose auxiliary cells overflow: the link cells' work inside the
+    list passes (until the host has seen it) and by their own kernels (after)
+    is that of a context without lists."""
+    rng = np.random.default_rng(8)
+    lj = CA.LJPotential(sigma=1.9, epsilon=1e-4, cutoff=4.95, mass=63.55)
+    bounds = np.array([29.0, 27.5, 28.1])
+    grid = np.stack(np.meshgrid(*[np.arange(int(b / 1.9)) for b in bounds], indexing="ij"), -1).reshape(-1, 3)
+    xyz = (grid + 0.5) * 1.9 + rng.uniform(-0.1, 0.1, grid.shape)  # 0.146 atoms per A^3: some 30 a cell
+    close = xyz[:, 0] < 7.0
+    xyz = np.concatenate([xyz, xyz[close] + 0.95])  # and twice that in a slab: above 64
+    xyz %= bounds
+
+    def make(skin):
+        if kind == "batch":
+            few = xyz[::9]
+            b = CA.Batch([dict(pot=p, bounds=bounds) for p in (cu500, lj, cu500)], precision=precision)
+            b.tune(skin=skin)
+            for r, x in enumerate((few, few, xyz)):
+                b.bin_atoms(r, x)
+            return b
+        s = CA.Simulation(lj if kind == "lj" else cu500, bounds, precision=precision,
+                          evaluation="cheby" if kind == "cheby" else "table")
+        s.tune(skin=skin)
+        s.bin_atoms(xyz)
+        return s
+
+    def state(s):
+        parts = [s.download(r) for r in range(s.nrep)] if kind == "batch" else [s.download()]
+        parts = [compact(p) for p in parts]
+        return [np.concatenate([p[k] for p in parts]) for k in ("f", "rho", "fi")]
+
+    a, b = make(0.4), make(0.0)
+    b.force()
+    want = state(b)
+    for _ in range(2):
+        a.force()
+        got = state(a)
+        assert a.list_info()["active"] == 1 and a.list_info()["valid"] == 0
+        for g, w in zip(got, want):
+            assert scalar_rel_error(g, w).max() <= 1e-12
+        a.sync()  # the host looks
