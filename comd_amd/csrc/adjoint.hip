@@ -47,21 +47,13 @@ struct AdjDev {
 };
 
 
+// A one-wave block's moments: a[], and b[] or zeros.
 template <int TWO>
-__device__ __forceinline__ void write_moments(const double *a, const double *b, double *part)
+__device__ __forceinline__ void write_moments(double (&a)[AMAX], double (&b)[AMAX], double *part)
 {
-    const int L = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < AMAX; k++) {
-        const double s = wave_sum(a[k]);
-        if (L == 0) part[k] = s;
-        if (TWO) {
-            const double t = wave_sum(b[k]);
-            if (L == 0) part[AMAX + k] = t;
-        } else if (L == 0) {
-            part[AMAX + k] = 0.0;
-        }
-    }
+    const int L = threadIdx.x, k = L >> 1;
+    const double s = wave_sums(a), t = TWO ? wave_sums(b) : 0.0;
+    part[L & 1 ? AMAX + k : k] = L & 1 ? t : s;
 }
 
 // ---------------------------------------------------------------------------
@@ -79,7 +71,7 @@ __device__ __forceinline__ void write_moments(const double *a, const double *b, 
 
 #define AQ 128  // queued pairs: a batch of 64 and up to 63 more
 
-template <int PASS, int MIXED>
+template <int PASS, int MIXED, int NC>
 __global__ __launch_bounds__(64) void k_adj_pair(DevState d, PotDev P, AdjDev A)
 {
     __shared__ double hx[AHMAX], hy[AHMAX], hz[AHMAX];
@@ -100,12 +92,10 @@ __global__ __launch_bounds__(64) void k_adj_pair(DevState d, PotDev P, AdjDev A)
     __shared__ int qh[PASS == 2 ? AQ : 1];
 
     const int L = threadIdx.x;
-    const int m = P.cn;
     const int dom = PASS == 1 ? 0 : 1;
     const double ca = P.ca[dom], cb = P.cb[dom];
     const double rc2 = P.rc2;
-    const int m8 = P.cstride;
-    const double *dser = P.cheb + 4 * m8;      // rho' series
+    const double *dser = P.cheb + 4 * NC;      // rho' series
 
     double m0[AMAX], m1[AMAX];
 #pragma unroll
@@ -120,14 +110,14 @@ __global__ __launch_bounds__(64) void k_adj_pair(DevState d, PotDev P, AdjDev A)
             const double r = sqrt(qr2[L]);
             const double y = cheb_arg(r, ca, cb);
             if (PASS == 3) {
-                add_basis<MIXED, 0>(y, m, qv[L], 0.0, m0, m1);
+                add_basis<MIXED, 0, NC>(y, qv[L], 0.0, m0, m1);
             } else {
                 const double w = qv[L] / r;
                 if (PASS == 1) {
-                    add_basis<MIXED, 1>(y, m, 0.5 * w, 0.5 * de, m0, m1);
+                    add_basis<MIXED, 1, NC>(y, 0.5 * w, 0.5 * de, m0, m1);
                 } else {
                     // rho'(r) from the same basis values (rho's domain)
-                    const double drho = add_basis_sum<MIXED>(y, m, 0.5 * qf[L] * w, m0, dser);
+                    const double drho = add_basis_sum<MIXED, NC>(y, 0.5 * qf[L] * w, m0, dser);
                     v = drho * w;
                     key = qh[L];
                 }
@@ -270,26 +260,28 @@ __global__ __launch_bounds__(64) void k_adj_pair(DevState d, PotDev P, AdjDev A)
 }
 
 // ---------------------------------------------------------------------------
-// atom pass: mu_i, M_F, M_FE
+// atom pass: mu_i, M_F, M_FE.  Four cells per wave, 16 lanes each (their atoms
+// beyond 16 in further rounds): at 10.5 atoms a cell a wave per cell left five
+// lanes in six idle through the basis sums, and each cell ended with its own
+// sums over the lanes (512 000 atoms, mixed: 85 -> 19 us).
 
-template <int MIXED>
+template <int MIXED, int NC>
 __global__ __launch_bounds__(64) void k_adj_atom(DevState d, PotDev P, AdjDev A)
 {
-    const int L = threadIdx.x;
-    const int m = P.cn;
     const double ca = P.ca[2], cb = P.cb[2];
     double m0[AMAX], m1[AMAX];
 #pragma unroll
     for (int k = 0; k < AMAX; k++) m0[k] = m1[k] = 0.0;
-    for (int c = blockIdx.x; c < d.ncells; c += gridDim.x) {
-        if (L < d.natoms[c]) {
-            const int s = c * CM_SLOTS + L;
-            const double de = A.dlde[rep_of(d, c)];
+    for (int c = blockIdx.x * 4 + ((int)threadIdx.x >> 4); c < d.ncells; c += gridDim.x * 4) {
+        const int n = d.natoms[c];
+        const double de = A.dlde[rep_of(d, c)];
+        for (int t = threadIdx.x & 15; t < n; t += 16) {
+            const int s = c * CM_SLOTS + t;
             const double rho = d.rho[s];
             const double lam = A.lam[s];
-            const double f2 = cheb64(A.f2, P.cstride, ca, cb, rho);  // zero-padded as the series
+            const double f2 = cheb64(A.f2, NC, ca, cb, rho);  // zero-padded as the series
             A.mu[s] = lam * f2 + de * d.fi[s];
-            add_basis<MIXED, 1>(cheb_arg(rho, ca, cb), m, lam, de, m0, m1);
+            add_basis<MIXED, 1, NC>(cheb_arg(rho, ca, cb), lam, de, m0, m1);
         }
     }
     write_moments<1>(m0, m1, A.part + (size_t)blockIdx.x * ANMOM);
@@ -297,17 +289,18 @@ __global__ __launch_bounds__(64) void k_adj_atom(DevState d, PotDev P, AdjDev A)
 
 // ---------------------------------------------------------------------------
 // residual: with w the atom's replica weight (1 / (3 N) of its replica),
-// g_i = 2 w (f_i - t_i), and the partial sums of w |f_i - t_i|^2
+// g_i = 2 w (f_i - t_i), and the partial sums of w |f_i - t_i|^2; four cells
+// per wave (empty slots' g is never read)
 
 __global__ __launch_bounds__(64) void k_adj_resid(DevState d, const double *ft, const double *rw, double *gx,
                                                   double *gy, double *gz, double *part)
 {
-    const int L = threadIdx.x;
     double ss = 0.0;
-    for (int c = blockIdx.x; c < d.ncells; c += gridDim.x) {
-        const int s = c * CM_SLOTS + L;
-        if (L < d.natoms[c]) {
-            const double w = rw[rep_of(d, c)];
+    for (int c = blockIdx.x * 4 + ((int)threadIdx.x >> 4); c < d.ncells; c += gridDim.x * 4) {
+        const int n = d.natoms[c];
+        const double w = rw[rep_of(d, c)];
+        for (int t = threadIdx.x & 15; t < n; t += 16) {
+            const int s = c * CM_SLOTS + t;
             const double ex = d.fx[s] - ft[3L * s + 0];
             const double ey = d.fy[s] - ft[3L * s + 1];
             const double ez = d.fz[s] - ft[3L * s + 2];
@@ -315,22 +308,22 @@ __global__ __launch_bounds__(64) void k_adj_resid(DevState d, const double *ft, 
             gy[s] = 2.0 * w * ey;
             gz[s] = 2.0 * w * ez;
             ss += w * (ex * ex + ey * ey + ez * ez);
-        } else {
-            gx[s] = 0.0;
-            gy[s] = 0.0;
-            gz[s] = 0.0;
         }
     }
     const double t = wave_sum(ss);
-    part[(size_t)blockIdx.x * ANMOM + L] = L == 0 ? t : 0.0;
+    part[(size_t)blockIdx.x * ANMOM + threadIdx.x] = threadIdx.x == 0 ? t : 0.0;
 }
 
-// Sums the blocks' partial moments in a fixed order: out[k] = sum_b
-// part[b][k].  Sixteen waves take interleaved runs of 8 blocks (their loads
-// issued together), and their sums are added in wave order.
-__global__ __launch_bounds__(1024) void k_adj_final(const double *part, int nblocks, double *out)
+// Sums the blocks' partial moments of every stage in a fixed order, a block
+// per stage: out[stage][k] = sum_b part[b][k].  Sixteen waves take interleaved
+// runs of 8 blocks (their loads issued together), and their sums are added in
+// wave order.  One launch after all stages (each stage has its own partials):
+// a launch per stage took 5 to 12 us each.
+__global__ __launch_bounds__(1024) void k_adj_final(CmAdjParts J)
 {
     __shared__ double acc[16][ANMOM];
+    const double *part = J.part[blockIdx.x];
+    const int nblocks = J.nblocks[blockIdx.x];
     const int k = threadIdx.x & 63, j = threadIdx.x >> 6;
     double s = 0.0;
     for (int b0 = j * 8; b0 < nblocks; b0 += 16 * 8) {
@@ -345,7 +338,7 @@ __global__ __launch_bounds__(1024) void k_adj_final(const double *part, int nblo
     if (j == 0) {
         double t = 0.0;
         for (int q = 0; q < 16; q++) t += acc[q][k];
-        out[k] = t;
+        J.out[(size_t)blockIdx.x * ANMOM + k] = t;
     }
 }
 
@@ -354,8 +347,8 @@ __global__ __launch_bounds__(1024) void k_adj_final(const double *part, int nblo
 int cm_adjoint_max_coefs() { return AMAX; }
 int cm_adjoint_moments() { return ANMOM; }
 
-template <int MIXED>
-static void launch_all(const DevState &d, const PotDev &P, const CmAdjoint &J, int stage, hipStream_t st)
+template <int MIXED, int NC>
+static void launch_stage(const DevState &d, const PotDev &P, const CmAdjoint &J, int stage, hipStream_t st)
 {
     AdjDev A;
     A.gx = J.gx;
@@ -365,32 +358,41 @@ static void launch_all(const DevState &d, const PotDev &P, const CmAdjoint &J, i
     A.mu = J.mu;
     A.f2 = J.f2;
     A.dlde = J.dlde;
-    A.part = J.part;
-    const dim3 g(J.nblocks), b(64);
-    double *o = J.out + (size_t)stage * ANMOM;
+    A.part = J.parts.part[stage];
+    const dim3 g(J.parts.nblocks[stage]), b(64);
     switch (stage) {
-    case 0: hipLaunchKernelGGL((k_adj_pair<1, MIXED>), g, b, 0, st, d, P, A); break;
-    case 1: hipLaunchKernelGGL((k_adj_pair<2, MIXED>), g, b, 0, st, d, P, A); break;
-    case 2: hipLaunchKernelGGL((k_adj_atom<MIXED>), g, b, 0, st, d, P, A); break;
-    case 3: hipLaunchKernelGGL((k_adj_pair<3, MIXED>), g, b, 0, st, d, P, A); break;
-    default: return;
+    case 0: hipLaunchKernelGGL((k_adj_pair<1, MIXED, NC>), g, b, 0, st, d, P, A); break;
+    case 1: hipLaunchKernelGGL((k_adj_pair<2, MIXED, NC>), g, b, 0, st, d, P, A); break;
+    case 2: hipLaunchKernelGGL((k_adj_atom<MIXED, NC>), g, b, 0, st, d, P, A); break;
+    case 3: hipLaunchKernelGGL((k_adj_pair<3, MIXED, NC>), g, b, 0, st, d, P, A); break;
+    default: break;
     }
-    hipLaunchKernelGGL(k_adj_final, dim3(1), dim3(1024), 0, st, J.part, J.nblocks, o);
+}
+
+template <int NC>
+static void launch_stage2(const DevState &d, const PotDev &P, const CmAdjoint &J, int stage, int mixed, hipStream_t st)
+{
+    if (mixed) launch_stage<1, NC>(d, P, J, stage, st);
+    else launch_stage<0, NC>(d, P, J, stage, st);
 }
 
 void cm_launch_adj_resid(const DevState &d, const CmAdjoint &J, const double *ft, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_adj_resid, dim3(J.nblocks), dim3(64), 0, st, d, ft, J.rw, J.gx, J.gy, J.gz, J.part);
-    hipLaunchKernelGGL(k_adj_final, dim3(1), dim3(1024), 0, st, J.part, J.nblocks, J.out + (size_t)4 * ANMOM);
+    hipLaunchKernelGGL(k_adj_resid, dim3(J.parts.nblocks[4]), dim3(64), 0, st, d, ft, J.rw, J.gx, J.gy, J.gz,
+                       J.parts.part[4]);
 }
 
-void cm_launch_adj_final(const CmAdjoint &J, int nblocks, int stage, hipStream_t st)
+void cm_launch_adj_final(const CmAdjoint &J, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_adj_final, dim3(1), dim3(1024), 0, st, J.part, nblocks, J.out + (size_t)stage * ANMOM);
+    hipLaunchKernelGGL(k_adj_final, dim3(CM_ADJ_STAGES), dim3(1024), 0, st, J.parts);
 }
 
 void cm_launch_adj_stage(const DevState &d, const PotDev &P, const CmAdjoint &J, int stage, int mixed, hipStream_t st)
 {
-    if (mixed) launch_all<1>(d, P, J, stage, st);
-    else launch_all<0>(d, P, J, stage, st);
+    switch (P.cstride) {
+    case 8: launch_stage2<8>(d, P, J, stage, mixed, st); break;
+    case 16: launch_stage2<16>(d, P, J, stage, mixed, st); break;
+    case 24: launch_stage2<24>(d, P, J, stage, mixed, st); break;
+    default: launch_stage2<AMAX>(d, P, J, stage, mixed, st); break;
+    }
 }

@@ -2518,8 +2518,8 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
         alloc((void **)&c->adj_mu, S * 8);
         alloc((void **)&c->adj_ft, S * 3 * 8);
         alloc((void **)&c->adj_f2, 64 * 8);
-        alloc((void **)&c->adj_part, (size_t)c->adj_nblocks * NM * 8);
-        alloc((void **)&c->adj_out, (size_t)5 * NM * 8);
+        alloc((void **)&c->adj_part, (size_t)CM_ADJ_STAGES * c->adj_nblocks * NM * 8);
+        alloc((void **)&c->adj_out, (size_t)CM_ADJ_STAGES * NM * 8);
         alloc((void **)&c->adj_rep, (size_t)2 * c->nrep * 8);
         alloc((void **)&c->adj_E, (size_t)3 * c->nrep * 8);
         alloc((void **)&c->adj_epart, (size_t)3 * c->nrep * c->nparts * 8);
@@ -2588,9 +2588,11 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
     J.f2 = c->adj_f2;
     J.dlde = c->adj_rep;
     J.rw = c->adj_rep + c->nrep;
-    J.part = c->adj_part;
-    J.nblocks = c->adj_nblocks;
-    J.out = c->adj_out;
+    for (int k = 0; k < CM_ADJ_STAGES; k++) {
+        J.parts.part[k] = c->adj_part + (size_t)k * c->adj_nblocks * NM;
+        J.parts.nblocks[k] = c->adj_nblocks;
+    }
+    J.parts.out = c->adj_out;
     PotDev P = R0.pot;  // series, domains and cutoff common to the replicas
     P.eval = COMD_EVAL_CHEB;
     DevState d = dev_state(c);
@@ -2599,64 +2601,68 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
     } else {
         cm_launch_adj_resid(d, J, c->adj_ft, c->stream);
     }
-    // the pair passes over the neighbour lists when the forward pass used
-    // them (valid after it, every group an EAM one, the staged halo in LDS)
-    // and, by default, there is a group per CU at least (a block per group:
-    // fewer groups leave CUs idle, where the link-cell passes, a wave per
-    // cell, measured faster); else over the link cells
-    bool nl = false;
-    if (c->adj_lists && c->nl_active && c->nl_lj_groups == 0 && (c->adj_lists == 2 || c->nl.pass_blocks >= c->ncu)) {
-        unsigned f = 0;
+    // the pair passes over the neighbour lists when the context has them
+    // (every group an EAM one, the staged halo in LDS) and, by default, there
+    // is a group per CU at least (a block per group: fewer groups leave CUs
+    // idle, where the link-cell passes, a wave per cell, measured faster);
+    // else over the link cells.  Whether the forward pass left the lists
+    // valid comes back with the results (waiting for it here left the GPU
+    // idle for some 40 us): if not, the link cells run after all
+    bool nl = c->adj_lists && c->nl_active && !c->nl_invalid_seen && c->nl_lj_groups == 0 &&
+              (c->adj_lists == 2 || c->nl.pass_blocks >= c->ncu) &&
+              cm_adj_nl_lds(c->nl) + (12 << 10) <= (size_t)c->lds_block;
+    std::vector<double> out((size_t)CM_ADJ_STAGES * NM), E3((size_t)3 * nrep);
+    for (;;) {
+        CmAdjoint K = J;
+        if (nl) {
+            const CmList &l = c->nl;
+            const long ng = l.pass_blocks;
+            if ((long)l.n * 3 > c->adj_gb_cap) {
+                if (c->adj_gb) hipFree(c->adj_gb);
+                c->adj_gb = nullptr;
+                c->adj_gb_cap = 0;
+                if (hipMalloc((void **)&c->adj_gb, (size_t)l.n * 3 * 8) != hipSuccess)
+                    return set_err(c, COMD_ERR_NOMEM, "adjoint list buffers");
+                c->adj_gb_cap = (long)l.n * 3;
+            }
+            if (3 * ng > c->adj_part_nl_cap) {
+                if (c->adj_part_nl) hipFree(c->adj_part_nl);
+                c->adj_part_nl = nullptr;
+                c->adj_part_nl_cap = 0;
+                if (hipMalloc((void **)&c->adj_part_nl, (size_t)3 * ng * NM * 8) != hipSuccess)
+                    return set_err(c, COMD_ERR_NOMEM, "adjoint list buffers");
+                c->adj_part_nl_cap = 3 * ng;
+            }
+            CmAdjNl A;
+            A.gb = c->adj_gb;
+            A.gx = J.gx;
+            A.gy = J.gy;
+            A.gz = J.gz;
+            A.mu = J.mu;
+            A.lam = J.lam;
+            A.dlde = J.dlde;
+            const int stage[3] = {0, 1, 3};  // of the passes 1 (the phi gradient's moments, one set), 2, 3
+            cm_launch_adj_nl_gather(l, J.gx, J.gy, J.gz, c->adj_gb, c->stream);
+            for (int q = 0; q < 3; q++) {
+                A.part = K.parts.part[stage[q]] = c->adj_part_nl + (size_t)q * ng * NM;
+                K.parts.nblocks[stage[q]] = (int)ng;
+                if (q == 2) cm_launch_adj_stage(d, P, K, 2, mixed, c->stream);  // the atom pass, per slot
+                cm_launch_adj_nl(d, P, l, A, q + 1, mixed, c->stream);
+            }
+        } else {
+            for (int stage = 0; stage < 4; stage++) cm_launch_adj_stage(d, P, K, stage, mixed, c->stream);
+        }
+        if (emode) K.parts.nblocks[4] = 0;
+        cm_launch_adj_final(K, c->stream);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipMemcpyAsync(out.data(), c->adj_out, out.size() * 8, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(E3.data(), c->adj_E, E3.size() * 8, hipMemcpyDeviceToHost, c->stream));
+        if (nl)
+            HIPCHK(c, hipMemcpyAsync(c->host_flags + 1, c->nl.flags, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(&f, c->nl.flags, 4, hipMemcpyDeviceToHost));
-        nl = !(f & CM_NL_INVALID) && cm_adj_nl_lds(c->nl) + (12 << 10) <= (size_t)c->lds_block;
+        if (!nl || !(c->host_flags[1] & CM_NL_INVALID)) break;
+        nl = false;
     }
-    if (nl) {
-        const CmList &l = c->nl;
-        const long ng = l.pass_blocks;
-        if ((long)l.n * 3 > c->adj_gb_cap) {
-            if (c->adj_gb) hipFree(c->adj_gb);
-            c->adj_gb = nullptr;
-            c->adj_gb_cap = 0;
-            if (hipMalloc((void **)&c->adj_gb, (size_t)l.n * 3 * 8) != hipSuccess)
-                return set_err(c, COMD_ERR_NOMEM, "adjoint list buffers");
-            c->adj_gb_cap = (long)l.n * 3;
-        }
-        if (2 * ng > c->adj_part_nl_cap) {
-            if (c->adj_part_nl) hipFree(c->adj_part_nl);
-            c->adj_part_nl = nullptr;
-            c->adj_part_nl_cap = 0;
-            if (hipMalloc((void **)&c->adj_part_nl, (size_t)2 * ng * NM * 8) != hipSuccess)
-                return set_err(c, COMD_ERR_NOMEM, "adjoint list buffers");
-            c->adj_part_nl_cap = 2 * ng;
-        }
-        CmAdjNl A;
-        A.gb = c->adj_gb;
-        A.gx = J.gx;
-        A.gy = J.gy;
-        A.gz = J.gz;
-        A.mu = J.mu;
-        A.lam = J.lam;
-        A.dlde = J.dlde;
-        A.part = c->adj_part_nl;
-        CmAdjoint Jn = J;
-        Jn.part = c->adj_part_nl;
-        cm_launch_adj_nl_gather(l, J.gx, J.gy, J.gz, c->adj_gb, c->stream);
-        cm_launch_adj_nl(d, P, l, A, 1, mixed, c->stream);  // the phi gradient's moments, one set
-        cm_launch_adj_final(Jn, (int)ng, 0, c->stream);
-        cm_launch_adj_nl(d, P, l, A, 2, mixed, c->stream);
-        cm_launch_adj_final(Jn, (int)ng, 1, c->stream);
-        cm_launch_adj_stage(d, P, J, 2, mixed, c->stream);  // the atom pass, per slot
-        cm_launch_adj_nl(d, P, l, A, 3, mixed, c->stream);
-        cm_launch_adj_final(Jn, (int)ng, 3, c->stream);
-    } else {
-        for (int stage = 0; stage < 4; stage++) cm_launch_adj_stage(d, P, J, stage, mixed, c->stream);
-    }
-    HIPCHK(c, hipGetLastError());
-    std::vector<double> out((size_t)5 * NM), E3((size_t)3 * nrep);
-    HIPCHK(c, hipMemcpyAsync(out.data(), c->adj_out, out.size() * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(E3.data(), c->adj_E, E3.size() * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     double lossE = 0.0;
     for (int r = 0; r < nrep; r++) {
         const double E = E3[(size_t)3 * r];

@@ -170,25 +170,31 @@ void cm_launch_scatter_series(const PotDev *pots, int nrep, const char *src, int
 void cm_launch_adj_rep(const double *E, const double *w, const double *rw, int nrep, int emode, double w_e,
                        double *rep, hipStream_t st);
 
+// Partial moments of the adjoint's stages 0-3 and, as stage 4, of the weighted
+// sum of squared force residuals: per stage its blocks' partials
+// (cm_adjoint_moments() doubles each) and their number; out: their sums.
+#define CM_ADJ_STAGES 5
+struct CmAdjParts {
+    double *part[CM_ADJ_STAGES];
+    int nblocks[CM_ADJ_STAGES];
+    double *out;
+};
 // Device buffers and scalars of the Chebyshev-coefficient adjoint
-// (adjoint.hip).  out holds 5 x cm_adjoint_moments() doubles: the moments of
-// stages 0-3 and, at out[4*64], the weighted sum of squared force residuals.
+// (adjoint.hip).
 struct CmAdjoint {
     double *gx, *gy, *gz;  // per slot: dL/df
     double *lam, *mu;      // per slot
     const double *f2;      // F'' series
     const double *dlde;    // per replica: dL/dE of its energy term
     const double *rw;      // per replica: weight of its force residuals, 1 / (3 N)
-    double *part;          // nblocks x 64 partial moments
-    int nblocks;
-    double *out;
+    CmAdjParts parts;
 };
 int cm_adjoint_max_coefs();
 int cm_adjoint_moments();
 void cm_launch_adj_resid(const DevState &d, const CmAdjoint &J, const double *ft, hipStream_t st);
 void cm_launch_adj_stage(const DevState &d, const PotDev &P, const CmAdjoint &J, int stage, int mixed,
                          hipStream_t st);
-void cm_launch_adj_final(const CmAdjoint &J, int nblocks, int stage, hipStream_t st);
+void cm_launch_adj_final(const CmAdjoint &J, hipStream_t st);
 
 // Observables (observe.hip): per-block partial sums of CM_OBS_N doubles
 // over one replica's cells (at most CM_OBS_MAXBLOCKS blocks, in part), then

@@ -1328,6 +1328,7 @@ void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase, int cel
 __global__ __launch_bounds__(256) void k_adj_nl_gather(CmList l, const double *gx, const double *gy,
                                                        const double *gz, double *gb)
 {
+    if (l.flags[0] & CM_NL_INVALID) return;
     const int n = l.gstart[l.ngroups];
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
         const int s = l.slot[l.order[t]];
@@ -1337,20 +1338,19 @@ __global__ __launch_bounds__(256) void k_adj_nl_gather(CmList l, const double *g
     }
 }
 
-template <int PASS, int MIXED>
-__global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, CmAdjNl A, int pbase)
+template <int PASS, int MIXED, int NC>
+__global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, CmAdjNl A)
 {
+    if (l.flags[0] & CM_NL_INVALID) return;  // the caller finds out with its results
     extern __shared__ __align__(16) char nls[];
     __shared__ PassLds S;
     __shared__ double red[12][ANMOM];
     double *hx = (double *)nls, *hy = hx + l.hcap, *hz = hy + l.hcap;
     CM_LDS uint8_t *slot_of = (CM_LDS uint8_t *)(nls + (size_t)l.hcap * 24);
-    const int m = P.cn;
     const int dom = PASS == 1 ? 0 : 1;  // phi's series domain, else rho's
     const double ca = P.ca[dom], cb = P.cb[dom];
     const double rc2 = P.rc2;
-    const int m8 = P.cstride;
-    const double *dser = P.cheb + 4 * m8;  // rho' series
+    const double *dser = P.cheb + 4 * NC;  // rho' series
     double m0[AMAX];
 #pragma unroll
     for (int k = 0; k < AMAX; k++) m0[k] = 0.0;
@@ -1408,24 +1408,24 @@ __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, 
                 const double r = sqrt(r2);
                 const double y = cheb_arg(r, ca, cb);
                 if (PASS >= 3) {
-                    add_basis<MIXED, 0>(y, m, wi, 0.0, m0, m0);
+                    add_basis<MIXED, 0, NC>(y, wi, 0.0, m0, m0);
                     continue;
                 }
                 const int q = S.base[slot_of[h]] + h;
                 const double w = ((gix - A.gb[3L * q + 0]) * dx + (giy - A.gb[3L * q + 1]) * dy +
                                   (giz - A.gb[3L * q + 2]) * dz) / r;
                 if (PASS == 1) {
-                    add_basis_deriv<MIXED>(y, m, de, w * inv_ba, m0);
+                    add_basis_deriv<MIXED, NC>(y, de, w * inv_ba, m0);
                 } else {
                     // rho'(r) from the same basis values (rho's domain)
-                    const double drho = add_basis_sum<MIXED>(y, m, 0.5 * (wi + l.fq[q]) * w, m0, dser);
+                    const double drho = add_basis_sum<MIXED, NC>(y, 0.5 * (wi + l.fq[q]) * w, m0, dser);
                     lam += drho * w;
                 }
             }
         }
         if (PASS == 2) A.lam[s] = lam;
     }
-    block_moments<0>(m0, red, A.part + (size_t)(pbase + blockIdx.x) * ANMOM);
+    block_moments<0>(m0, red, A.part + (size_t)blockIdx.x * ANMOM);
 }
 
 // ---------------------------------------------------------------------------
@@ -1584,18 +1584,26 @@ void cm_nl_tables(const CmList &l, hipStream_t st)
 
 size_t cm_adj_nl_lds(const CmList &l) { return (size_t)l.hcap * 24 + nl_slotmap_bytes(l.hcap); }
 
-template <int MIXED>
+template <int MIXED, int NC>
 static void adj_nl_launch(const DevState &d, const PotDev &P, const CmList &l, const CmAdjNl &A, int pass,
                           hipStream_t st)
 {
     const dim3 grid(l.pass_blocks), block(l.pass_threads);
     const size_t lds = cm_adj_nl_lds(l);
     switch (pass) {
-    case 1: hipLaunchKernelGGL((k_adj_nl<1, MIXED>), grid, block, lds, st, d, P, l, A, 0); break;
-    case 2: hipLaunchKernelGGL((k_adj_nl<2, MIXED>), grid, block, lds, st, d, P, l, A, 0); break;
-    case 3: hipLaunchKernelGGL((k_adj_nl<3, MIXED>), grid, block, lds, st, d, P, l, A, 0); break;
+    case 1: hipLaunchKernelGGL((k_adj_nl<1, MIXED, NC>), grid, block, lds, st, d, P, l, A); break;
+    case 2: hipLaunchKernelGGL((k_adj_nl<2, MIXED, NC>), grid, block, lds, st, d, P, l, A); break;
+    case 3: hipLaunchKernelGGL((k_adj_nl<3, MIXED, NC>), grid, block, lds, st, d, P, l, A); break;
     default: break;
     }
+}
+
+template <int NC>
+static void adj_nl_launch2(const DevState &d, const PotDev &P, const CmList &l, const CmAdjNl &A, int pass, int mixed,
+                           hipStream_t st)
+{
+    if (mixed) adj_nl_launch<1, NC>(d, P, l, A, pass, st);
+    else adj_nl_launch<0, NC>(d, P, l, A, pass, st);
 }
 
 void cm_launch_adj_nl_gather(const CmList &l, const double *gx, const double *gy, const double *gz, double *gb,
@@ -1607,6 +1615,10 @@ void cm_launch_adj_nl_gather(const CmList &l, const double *gx, const double *gy
 void cm_launch_adj_nl(const DevState &d, const PotDev &P, const CmList &l, const CmAdjNl &A, int pass, int mixed,
                       hipStream_t st)
 {
-    if (mixed) adj_nl_launch<1>(d, P, l, A, pass, st);
-    else adj_nl_launch<0>(d, P, l, A, pass, st);
+    switch (P.cstride) {
+    case 8: adj_nl_launch2<8>(d, P, l, A, pass, mixed, st); break;
+    case 16: adj_nl_launch2<16>(d, P, l, A, pass, mixed, st); break;
+    case 24: adj_nl_launch2<24>(d, P, l, A, pass, mixed, st); break;
+    default: adj_nl_launch2<AMAX>(d, P, l, A, pass, mixed, st); break;
+    }
 }

@@ -394,3 +394,32 @@ def test_batch_16x32k_gradient_at_size(gpu, cu500):
     assert abs(lm32 - loss) <= 1e-5 * loss
     assert (rel <= 1e-4).all()
     b.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [3, 8, 9, 16, 17, 24, 25, 31])
+def test_series_of_every_length_equal_their_zero_padded_32(gpu, cu500, n, precision):
+    """The basis sums have an instance for each stride of the series (8, 16,
+    24, 32 terms).  A series of n terms is the one of 32 with zeros behind,
+    so the loss and the first n components of the gradient are equal; over
+    the lists and over the link cells.  Tolerances: the same operations on
+    the same values, in FP64 to 1e-12 of each function's largest component;
+    in mixed precision to the 1e-6 of the lists against the link cells."""
+    c0 = cu500.cheb[:3].copy()
+    short = np.ascontiguousarray(c0[:, :n])
+    padded = np.zeros_like(c0)
+    padded[:, :n] = short
+    sim, _, _ = config(cu500, 6, 19, precision)
+    ft, et = target_of(sim, perturbed(c0, 6))
+    of_n, _, _ = config(CA.EAMPotential(cu500.name, ncheb=n), 6, 19, precision)
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    for lists in (2, 0):
+        for s in (sim, of_n):
+            s.tune(adjoint_lists=lists)
+        ln, gn = of_n.cheb_grad(short, ft, et, 1e-4)
+        lp, gp = sim.cheb_grad(padded, ft, et, 1e-4)
+        assert gn.shape == (3, n)
+        assert abs(ln - lp) <= tol * abs(lp)
+        err = np.abs(gn - gp[:, :n]).max(axis=1) / np.abs(gp).max(axis=1)
+        print(f"[{n} terms, {precision}, lists={lists}] {err}", flush=True)
+        assert (err <= tol).all()
