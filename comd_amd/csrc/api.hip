@@ -712,6 +712,10 @@ static bool setup_pot(const comd_params *p, Replica &R)
             f[0] = b[0] + b[1];  // rho'
             f[1] = b[1];
         }
+        // the density rows as they are kept: quarters permuted
+        std::vector<double> s64(d64.size());
+        for (int i = 0; i <= n; i++)
+            for (int q = 0; q < 8; q++) s64[(size_t)8 * i + (q ^ compact_swizzle(i))] = d64[(size_t)8 * i + q];
         // mixed density rows: phi d0 d1 (double), then 6 floats (40 bytes)
         // padded to whole 16-byte words, as the passes stage them
         std::vector<float> dm(((size_t)10 * (n + 1) + 3) / 4 * 4, 0.0f);
@@ -722,7 +726,7 @@ static bool setup_pot(const comd_params *p, Replica &R)
         double *a = (double *)alloc(d64.size() * 8), *b = (double *)alloc(r64.size() * 8);
         float *e = (float *)alloc(dm.size() * 4);
         if (ok)
-            ok = hipMemcpy(a, d64.data(), d64.size() * 8, hipMemcpyHostToDevice) == hipSuccess &&
+            ok = hipMemcpy(a, s64.data(), s64.size() * 8, hipMemcpyHostToDevice) == hipSuccess &&
                  hipMemcpy(b, r64.data(), r64.size() * 8, hipMemcpyHostToDevice) == hipSuccess &&
                  hipMemcpy(e, dm.data(), dm.size() * 4, hipMemcpyHostToDevice) == hipSuccess;
         P.cd64 = a;

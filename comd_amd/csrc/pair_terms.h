@@ -113,6 +113,8 @@ __device__ __forceinline__ TabsGlobal global_tabs(const PotDev &P)
     return t;
 }
 
+typedef double v2d __attribute__((ext_vector_type(2)));
+
 struct Acc {
     double x, y, z, e, rho, vir;
 };
@@ -246,9 +248,10 @@ __device__ __forceinline__ void pair_term_compact(const PotDev &P, const CT &T, 
             dphi = fma(t, pd1, pd0);
             rhov = fmaf(f, fmaf(f, rc2, rc1), rc0);
         } else {
-            const double pd0 = T.d64[8 * i + 0], pd1 = T.d64[8 * i + 1], pc0 = T.d64[8 * i + 2],
-                         pc1 = T.d64[8 * i + 3], pc2 = T.d64[8 * i + 4], rc0 = T.d64[8 * i + 5],
-                         rc1 = T.d64[8 * i + 6], rc2 = T.d64[8 * i + 7];
+            const int o = 8 * i + compact_swizzle(i);
+            const v2d a = *(const CM_LDS v2d *)(T.d64 + o), b = *(const CM_LDS v2d *)(T.d64 + (o ^ 2)),
+                      c = *(const CM_LDS v2d *)(T.d64 + (o ^ 4)), e = *(const CM_LDS v2d *)(T.d64 + (o ^ 6));
+            const double pd0 = a.x, pd1 = a.y, pc0 = b.x, pc1 = b.y, pc2 = c.x, rc0 = c.y, rc1 = e.x, rc2 = e.y;
             phiv = fma(t, fma(t, pc2, pc1), pc0);
             dphi = fma(t, pd1, pd0);
             rhov = fma(t, fma(t, rc2, rc1), rc0);
