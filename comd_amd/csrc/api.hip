@@ -1007,15 +1007,40 @@ static int nl_setup(comd_ctx *c)
     const long lds_avail = (long)c->lds_block - CM_NL_STATIC_LDS;
     const long hb = c->precision == COMD_PREC_MIXED ? 16 : 32;
     std::vector<std::array<int, 3>> gd(nrep), na(nrep), ng(nrep);
-    long hcap = 0, naux = 0, ngroups = 0, threads = 64;
+    long hcap = 0, naux = 0, ngroups = 0, threads = 64, build_threads = 64;
     // lanes per home atom in the force passes: as tuned, else two when the
     // atoms would fill fewer than two waves per CU at one lane each (each
     // lane then walks half the list: 32 000 Lennard-Jones atoms, pass
     // 0.034 -> 0.026 ms; at 256 000 atoms and above two lanes measured no
-    // better or slower)
+    // better or slower).  Below that EAM passes are as long as one lane's
+    // list: four lanes below 8 atoms per CU (a step of 864 atoms, tables: 43.8 -> 41.6
+    // us; of 4000 57.4 against 56.8), and eight below 64 per CU for the
+    // Chebyshev passes, whose pairs are some 200 operations each (864 atoms
+    // FP64 79 -> 66 us, mixed 82 -> 64; 4000 atoms mixed 94 -> 84; 32 000
+    // FP64 130 against 116)
     long natoms_all = 0;
-    for (const Replica &R : c->reps) natoms_all += R.ntot;
-    const int lanes = c->nl_lanes > 0 ? c->nl_lanes : (natoms_all < 128L * c->ncu ? 2 : 1);
+    bool lj = false, cheb = true;
+    for (const Replica &R : c->reps) {
+        natoms_all += R.ntot;
+        lj |= R.prm.potential == COMD_POT_LJ;
+        cheb &= R.pot.eval == COMD_EVAL_CHEB;
+    }
+    const int lanes = c->nl_lanes > 0                                ? c->nl_lanes
+                      : natoms_all >= 128L * c->ncu                  ? 1
+                      : lj                                           ? 2
+                      : cheb && natoms_all < 64L * c->ncu            ? 8
+                      : natoms_all < 8L * c->ncu                     ? 4
+                                                                     : 2;
+    // threads of a pass' block for its group's home atoms: 10 % more than
+    // the mean group's; 80 % where the system is small, whose groups of few
+    // cells differ most in their atoms: one atom more than threads and the
+    // block runs a second round (4000 atoms, two lanes, tables 69 -> 56 us a
+    // step, Chebyshev 136 -> 91; 32 000 atoms 69.9 -> 68.8)
+    // The build keeps to 10 % and two lanes' threads: its threads' queues set
+    // the order of the lists (k_nl_build), which should not vary with the
+    // passes' shape
+    const double spare = lanes > 1 ? 1.8 : 1.1;
+    const int build_lanes = natoms_all < 128L * c->ncu ? 2 : 1;
     // o >= 0: that option for every replica; o < 0 (batches): per replica
     // the shape with the fewest groups (then the fewest staged halo atoms)
     // among those whose groups' atoms (10 % spare) fit 768 threads and whose
@@ -1054,9 +1079,9 @@ static int nl_setup(comd_ctx *c)
         }
         return nr;
     };
-    auto shape = [&](int o) {  // fills gd, na, ng, hcap, naux, ngroups, threads
+    auto shape = [&](int o) {  // fills gd, na, ng, hcap, naux, ngroups, threads, build_threads
         hcap = naux = ngroups = 0;
-        threads = 64;
+        threads = build_threads = 64;
         for (int r = 0; r < nrep; r++) {
             long nr;
             if (o >= 0) {
@@ -1083,8 +1108,9 @@ static int nl_setup(comd_ctx *c)
             const long cells = (long)gd[r][0] * gd[r][1] * gd[r][2];
             const long slots = (long)(gd[r][0] + 2) * (gd[r][1] + 2) * (gd[r][2] + 2);
             hcap = std::max<long>(hcap, hcap_of(occ, slots));
-            threads = std::max<long>(
-                threads, ((long)(1.1 * occ * (double)cells * lanes / c->nl_threads_div) + 63) / 64 * 64);
+            const double home = occ * (double)cells / c->nl_threads_div;
+            threads = std::max<long>(threads, ((long)(spare * home * lanes) + 63) / 64 * 64);
+            build_threads = std::max<long>(build_threads, ((long)(1.1 * home * build_lanes) + 63) / 64 * 64);
             naux += nr;
             ngroups += (long)ng[r][0] * ng[r][1] * ng[r][2];
         }
@@ -1175,6 +1201,7 @@ static int nl_setup(comd_ctx *c)
     l.pass_blocks = (int)ngroups;
     // threads per pass block: a group's home atoms with 10 % to spare
     l.pass_threads = (int)pass_threads;
+    l.build_threads = (int)std::min<long>(768, build_threads);
     l.gwords = (int)gwords;
     l.lanes = lanes;
     l.tailq = cm_nl_pick_tailq(l);
@@ -1847,8 +1874,8 @@ int comd_tune(comd_ctx *c, int key, int value)
         if (c->have_atoms) return nl_setup(c);
         break;
     case COMD_TUNE_LIST_LANES:
-        if (value != 0 && value != 1 && value != 2 && value != 4)
-            return set_err(c, COMD_ERR_ARG, "list lanes must be 0 (by size), 1, 2 or 4");
+        if (value < 0 || value > 16 || (value & (value - 1)))
+            return set_err(c, COMD_ERR_ARG, "list lanes must be 0 (by size), 1, 2, 4, 8 or 16");
         c->nl_lanes = value;
         if (c->have_atoms) return nl_setup(c);
         break;
@@ -2312,7 +2339,7 @@ int comd_snapshot_load(comd_ctx *c, const char *path)
     int rc = comd_set_precision(c, hdr[2]);
     if (!rc) rc = comd_set_eval(c, hdr[3]);
     if (!rc && c->nl_skin_milli != hdr[5]) rc = comd_tune(c, COMD_TUNE_SKIN_MILLI, hdr[5]);
-    if (!rc && (hdr[15] == 1 || hdr[15] == 2 || hdr[15] == 4)) c->nl_lanes = hdr[15];
+    if (!rc && hdr[15] > 0 && hdr[15] <= 16 && !(hdr[15] & (hdr[15] - 1))) c->nl_lanes = hdr[15];
     if (!rc && c->reps[0].prm.potential == COMD_POT_LJ) rc = comd_tune(c, COMD_TUNE_LJ_PHYSICAL, hdr[14]);
     if (rc) {
         fclose(fp);

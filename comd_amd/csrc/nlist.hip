@@ -232,17 +232,18 @@ __device__ __forceinline__ void group_setup(const CmList &l, const NlRep &R, con
 __device__ __forceinline__ void group_store(const CmList &l, const GroupLds &S, const CM_LDS uint8_t *slot_of, int g)
 {
     int *gt = l.gtab + (size_t)g * CM_NL_GTAB;
-    const int H = S.off[S.ns], bd = blockDim.x;
-    for (int s = threadIdx.x; s < S.ns; s += bd) gt[s] = S.start[s] - S.off[s];
+    const int H = S.off[S.ns], bd = l.pass_threads;
+    for (int s = threadIdx.x; s < S.ns; s += blockDim.x) gt[s] = S.start[s] - S.off[s];
     if (threadIdx.x == 0) gt[CM_NL_SLOTS] = H;
-    for (int w = 0; w < l.gwords; w++) {
+    for (int t = threadIdx.x; t < bd * l.gwords; t += blockDim.x) {  // word w of thread t - w bd
+        const int h0 = t + 3 * (t / bd) * bd;
         unsigned v = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int h = (int)threadIdx.x + (4 * w + k) * bd;
+            const int h = h0 + k * bd;
             if (h < min(H, l.hcap)) v |= (unsigned)slot_of[h] << (8 * k);
         }
-        l.gslot[((size_t)g * l.gwords + w) * bd + threadIdx.x] = v;
+        l.gslot[(size_t)g * l.gwords * bd + t] = v;
     }
 }
 
@@ -1451,23 +1452,27 @@ void cm_nl_sync(const DevState &d, const CmList &l, hipStream_t st)
 size_t cm_nl_build_lds(const CmList &l)
 {
     // (128: the search reads up to 7 entries past the halo)
-    return (size_t)l.hcap * 16 + nl_slotmap_bytes(l.hcap) + (size_t)l.tailq * l.pass_threads * 2 + 128;
+    return (size_t)l.hcap * 16 + nl_slotmap_bytes(l.hcap) + (size_t)l.tailq * l.build_threads * 2 + 128;
 }
 
+// The tail queue's entries per thread: the most that cost no block per CU.  The
+// 128 bytes above stay out of the choice (they are within the static LDS'
+// allowance): it sets the order of the lists, and with it the rounding of
+// the mixed passes' single-precision sums.
 int cm_nl_pick_tailq(CmList l)
 {
     l.tailq = 0;
     int nb0 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb0, k_nl_build, l.pass_threads, cm_nl_build_lds(l)) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb0, k_nl_build, l.build_threads, cm_nl_build_lds(l) - 128) !=
             hipSuccess ||
         nb0 < 1)
         return 0;
     for (int q = 16; q >= 4; q -= 4) {
         l.tailq = q;
-        const size_t lds = cm_nl_build_lds(l);
+        const size_t lds = cm_nl_build_lds(l) - 128;
         int nb = 0;
         if ((long)lds <= (long)l.lds_avail &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_nl_build, l.pass_threads, lds) == hipSuccess &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_nl_build, l.build_threads, lds) == hipSuccess &&
             nb >= nb0)
             return q;
     }
@@ -1479,7 +1484,7 @@ void cm_nl_build(const DevState &d, const CmList &l, hipStream_t st, int lj_g0, 
     const unsigned blocks = (unsigned)std::min<long>(CM_KEY_BLOCKS, ((long)d.ncells * 16 + CM_KEY_THREADS - 1) / CM_KEY_THREADS);
     hipLaunchKernelGGL(k_nl_key, dim3(blocks), dim3(CM_KEY_THREADS), 0, st, d, l, lj_g0, dtd);
     hipLaunchKernelGGL(k_nl_sort, dim3(1024), dim3(256), 0, st, l);
-    hipLaunchKernelGGL(k_nl_build, dim3(l.pass_blocks), dim3(l.pass_threads), cm_nl_build_lds(l), st, d, l);
+    hipLaunchKernelGGL(k_nl_build, dim3(l.pass_blocks), dim3(l.build_threads), cm_nl_build_lds(l), st, d, l);
 }
 
 size_t cm_nl_tab_bytes(const PotDev &P, int kind, int mixed)

@@ -358,3 +358,29 @@ def test_invalid_lists_inside_and_beside_the_passes(gpu, cu500, kind, precision)
         for g, w in zip(got, want):
             assert scalar_rel_error(g, w).max() <= 1e-12
         a.sync()  # the host looks
+
+
+@pytest.mark.parametrize("lanes", [8, 16])
+@pytest.mark.parametrize("evaluation,precision", [("table", "fp64"), ("cheby", "fp64"), ("table", "mixed"), ("cheby", "mixed")])
+def test_eight_and_sixteen_lanes_equal_one(gpu, cu500, lanes, evaluation, precision):
+    """More lanes than an atom's list has chunks, and fewer: the passes give
+    the forces of one lane per atom, whose sums run in another order: 1e-12;
+    the mixed table passes add 8 pairs' values in single precision before
+    they enter the double sums, and which 8 depends on the block size:
+    7 x 2^-24 = 4e-7, held to 1e-6."""
+    a, b = pair_of_sims(cu500, 8, 3.615, 600.0, 0.1, 5, evaluation, precision)
+    b.tune(skin=0.4, list_lanes=1)
+    a.tune(list_lanes=lanes)
+    for s in (a, b):
+        s.force()
+        assert s.list_info()["active"] == 1 and s.list_info()["valid"] == 1
+    assert a.list_lanes() == lanes and b.list_lanes() == 1
+    assert_same(a, b, f"eam {evaluation} {precision}, {lanes} lanes",
+                tol=1e-6 if (evaluation, precision) == ("table", "mixed") else 1e-12)
+
+
+@pytest.mark.parametrize("evaluation,lanes", [("table", 4), ("cheby", 8)])
+def test_default_lanes_of_small_systems(gpu, cu500, evaluation, lanes):
+    a, _ = pair_of_sims(cu500, 6, 3.615, 600.0, 0.1, 5, evaluation, "fp64")
+    a.force()
+    assert a.list_lanes() == lanes

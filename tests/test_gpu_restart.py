@@ -46,3 +46,9 @@ def test_restart_continues_bit_for_bit(gpu, cu500, tmp_path, precision, lanes):
     for k in ("natoms", "id", "itype", "r", "p", "f", "rho", "fi"):
         assert np.array_equal(ga[k], gb[k]), k
     assert b.energy() == ea
+
+
+@pytest.mark.parametrize("lanes", [8, 16])
+def test_restart_with_more_lanes(gpu, cu500, tmp_path, lanes):
+    """The lanes per atom come from the file for any number there is."""
+    test_restart_continues_bit_for_bit(gpu, cu500, tmp_path, "fp64", lanes)
