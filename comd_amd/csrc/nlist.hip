@@ -723,53 +723,77 @@ __global__ __launch_bounds__(1024) void k_nl_tables(CmList l)
 // beside the list passes every time, those kernels' idle launches took 4.6 us
 // each (256 000 atoms and more; 3 us at 864).
 
-// Chebyshev passes: N pairs of a list chunk evaluated together, each series
-// as N interleaved Clenshaw recurrences (src-flat/cheby.c:276-310) that
-// share every coefficient load: evaluated pair by pair, each pair reloaded
-// all coefficients and ran one serial recurrence at a time.  x[u] is
-// clamped below at a as in cheb64; the series' argument is formed with
-// 1 / (b - a) computed once rather than a division per pair.
-template <int N>
-__device__ __forceinline__ void cheb64_n(const double *cg, int m8, double a, double b, const double (&x)[N],
-                                         double (&out)[N])
+// Chebyshev passes: S series over one domain, at N pairs of a list chunk
+// together (values in the convention of src-flat/cheby.c:290-310: c_0 / 2 +
+// sum of c_k T_k).  The basis is run forward, T_{k+1} = 2y T_k - T_{k-1}, and
+// shared by the series: S + 1 operations a term in place of the 2 S of a
+// Clenshaw sum for each.  Coefficients by scalar loads common to the N pairs, a block ahead of their
+// use; at[s]: the series' first coefficient from cg.  x[u] is clamped below at
+// a as in cheb64; the argument is formed with 1 / (b - a) computed once rather
+// than a division per pair.  The passes are bound by these operations (43 % of
+// the issue slots of 256 000 atoms' FP64 density pass) and by the few waves
+// beside them: 248 -> 162 us, embedding force 118 -> 102; of the mixed passes
+// phi' and rho' alone take this sum: a step 351 -> 326 us, of 48 484 atoms
+// 177 -> 161.
+template <int N, int S>
+__device__ __forceinline__ void cheb_sums(const double *cg, const int (&at)[S], int m8, double a, double b,
+                                          const double (&x)[N], double (&out)[S][N])
 {
+    constexpr int B = S > 1 ? 4 : 8;  // terms per block (m8 is a multiple of 8)
     const CM_CONST double *c = (const CM_CONST double *)cg;
     const double inv = 1.0 / (b - a);
-    double y2[N], d[N], dd[N];
+    double y2[N], tm[N], t[N];  // 2y, T_{k-1}, T_k
 #pragma unroll
     for (int u = 0; u < N; u++) {
         const double xu = x[u] < a ? a : x[u];
-        y2[u] = 2.0 * ((2.0 * xu - a - b) * inv);
-        d[u] = dd[u] = 0.0;
+        tm[u] = 1.0;
+        t[u] = (2.0 * xu - a - b) * inv;
+        y2[u] = 2.0 * t[u];
     }
-    double cc[8];
+    double cc[S][B];
 #pragma unroll
-    for (int k = 0; k < 8; k++) cc[k] = c[m8 - 8 + k];
-    for (int jb = m8 - 8; jb >= 0; jb -= 8) {
-        double cn[8];
-        const int jn = jb >= 8 ? jb - 8 : 0;  // the next block (block 0 again after the last)
+    for (int s = 0; s < S; s++)
 #pragma unroll
-        for (int k = 0; k < 8; k++) cn[k] = c[jn + k];
+        for (int k = 0; k < B; k++) cc[s][k] = c[at[s] + k];
+    auto term = [&](int k) {
 #pragma unroll
-        for (int k = 7; k >= 0; k--) {
-            if (jb + k > 0) {
+        for (int u = 0; u < N; u++) {
 #pragma unroll
-                for (int u = 0; u < N; u++) {
-                    const double sv = d[u];
-                    d[u] = y2[u] * d[u] - dd[u] + cc[k];
-                    dd[u] = sv;
-                }
-            }
+            for (int s = 0; s < S; s++) out[s][u] = fma(cc[s][k], t[u], out[s][u]);
+            const double tn = fma(y2[u], t[u], -tm[u]);
+            tm[u] = t[u];
+            t[u] = tn;
         }
+    };
+    auto block = [&](int jb, auto first) {
+        double cn[S][B];
+        const int jn = jb + B < m8 ? jb + B : jb;  // the next block (the last again after it)
 #pragma unroll
-        for (int k = 0; k < 8; k++) cc[k] = cn[k];
-    }
+        for (int s = 0; s < S; s++)
 #pragma unroll
-    for (int u = 0; u < N; u++) out[u] = 0.5 * y2[u] * d[u] - dd[u] + 0.5 * cc[0];
+            for (int k = 0; k < B; k++) cn[s][k] = c[at[s] + jn + k];
+#pragma unroll
+        for (int k = decltype(first)::value ? 1 : 0; k < B; k++) term(k);
+#pragma unroll
+        for (int s = 0; s < S; s++)
+#pragma unroll
+            for (int k = 0; k < B; k++) {
+                // the loads stay in this block: left alone the compiler moves
+                // them to the top of the next, where each is waited for
+                asm volatile("" : "+s"(cn[s][k]));
+                cc[s][k] = cn[s][k];
+            }
+    };
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int u = 0; u < N; u++) out[s][u] = 0.5 * cc[s][0];
+    block(0, std::true_type());
+    for (int jb = B; jb < m8; jb += B) block(jb, std::false_type());
 }
 
-// The same in single precision (cheb32's recurrence) for the values of the
-// mixed density pass.
+// Clenshaw sums in single precision (cheb32's recurrence) for the values of
+// the mixed density pass.
 template <int N>
 __device__ __forceinline__ void cheb32_n(const float *cg, int m8, float a, float b, const float (&x)[N],
                                          float (&out)[N])
@@ -803,7 +827,10 @@ __device__ __forceinline__ void cheb32_n(const float *cg, int m8, float a, float
             }
         }
 #pragma unroll
-        for (int k = 0; k < 8; k++) cc[k] = cn[k];
+        for (int k = 0; k < 8; k++) {
+            asm volatile("" : "+s"(cn[k]));  // as in cheb_sums
+            cc[k] = cn[k];
+        }
     }
 #pragma unroll
     for (int u = 0; u < N; u++) out[u] = fmaf(0.5f * y2[u], d[u], 0.5f * cc[0] - dd[u]);
@@ -923,17 +950,16 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
             }
         };
         if constexpr (EVAL == COMD_EVAL_CHEB && KIND != CM_KIND_LJ) {
-            // the chunk's pairs NB at a time (cheb64_n): r of each, the
-            // series, then the sums in list order, the separations read
-            // again from the halo.  Four in FP64, two in mixed precision,
-            // where the registers of more recurrences cost more resident
-            // waves than the wider interleave gains (measured, 256 000
-            // atoms: FP64 passes 0.333 + 0.147 -> 0.240 + 0.118 ms, mixed
-            // 0.245 + 0.113 -> 0.186 + 0.096 ms).
+            // the chunk's pairs NB at a time (cheb_sums): r of each, the
+            // series, then the sums in list order.  Four in FP64 (256 000
+            // atoms 325 us a step, two 338), two in mixed precision, whose
+            // passes lose more resident waves to the registers of four than
+            // the wider interleave gains.  Sums without branches over the
+            // pairs outside: no gain
             constexpr int NB = MIXED ? 2 : 4;
 #pragma unroll
             for (int h = 0; h < 8; h += NB) {
-                double rr[NB];
+                double rr[NB], ri[NB];  // r and 1/r
                 unsigned msk = 0;
 #pragma unroll
                 for (int j = 0; j < NB; j++) {
@@ -954,50 +980,52 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
                         in = KIND == CM_KIND_EAM3 ? (r2 < rc2) : (r2 <= rc2);
                     }
                     in = in && (!TAIL || k0 + u < cnt);
-                    rr[j] = in ? r2 * (MIXED ? rsqrt_mixed(r2) : rsqrt64(r2)) : 0.0;  // outside: the lower end
+                    ri[j] = MIXED ? rsqrt_mixed(r2) : rsqrt64(r2);
+                    rr[j] = in ? r2 * ri[j] : 0.0;  // outside: the lower end
                     msk |= (unsigned)in << j;
                 }
                 if (msk == 0) continue;
                 npair += __builtin_popcount(msk);
                 const int m = P.cstride;
-                double v[NB];
                 if constexpr (KIND == CM_KIND_EAM1) {
+                    double v[3][NB];  // phi, phi', rho
                     if constexpr (MIXED) {
-                        float rf[NB], vf[NB];
+                        // values in FP32, the derivative in FP64
+                        float rf[NB], vf[2][NB];
+                        double w[1][NB];
 #pragma unroll
                         for (int j = 0; j < NB; j++) rf[j] = (float)rr[j];
-                        cheb32_n<NB>(P.cheb32 + 0 * m, m, (float)P.ca[0], (float)P.cb[0], rf, vf);
+                        cheb32_n<NB>(P.cheb32 + 0 * m, m, (float)P.ca[0], (float)P.cb[0], rf, vf[0]);
+                        cheb32_n<NB>(P.cheb32 + 1 * m, m, (float)P.ca[1], (float)P.cb[1], rf, vf[1]);
+                        cheb_sums<NB, 1>(P.cheb, {3 * m}, m, P.ca[0], P.cb[0], rr, w);
 #pragma unroll
                         for (int j = 0; j < NB; j++)
-                            if ((msk >> j) & 1u) A.e += 0.5 * (double)vf[j];
-                        cheb32_n<NB>(P.cheb32 + 1 * m, m, (float)P.ca[1], (float)P.cb[1], rf, vf);
+                            v[0][j] = (double)vf[0][j], v[1][j] = w[0][j], v[2][j] = (double)vf[1][j];
+                    } else if (P.ca[0] == P.ca[1] && P.cb[0] == P.cb[1]) {
+                        cheb_sums<NB, 3>(P.cheb, {0, 3 * m, m}, m, P.ca[0], P.cb[0], rr, v);
+                    } else {  // rho apart where its domain is another
+                        double w[2][NB], z[1][NB];
+                        cheb_sums<NB, 2>(P.cheb, {0, 3 * m}, m, P.ca[0], P.cb[0], rr, w);
+                        cheb_sums<NB, 1>(P.cheb, {m}, m, P.ca[1], P.cb[1], rr, z);
 #pragma unroll
-                        for (int j = 0; j < NB; j++)
-                            if ((msk >> j) & 1u) A.rho += (double)vf[j];
-                    } else {
-                        cheb64_n<NB>(P.cheb + 0 * m, m, P.ca[0], P.cb[0], rr, v);
-#pragma unroll
-                        for (int j = 0; j < NB; j++)
-                            if ((msk >> j) & 1u) A.e += 0.5 * v[j];
-                        cheb64_n<NB>(P.cheb + 1 * m, m, P.ca[1], P.cb[1], rr, v);
-#pragma unroll
-                        for (int j = 0; j < NB; j++)
-                            if ((msk >> j) & 1u) A.rho += v[j];
+                        for (int j = 0; j < NB; j++) v[0][j] = w[0][j], v[1][j] = w[1][j], v[2][j] = z[0][j];
                     }
-                    cheb64_n<NB>(P.cheb + 3 * m, m, P.ca[0], P.cb[0], rr, v);  // phi', FP64 in both modes
 #pragma unroll
                     for (int j = 0; j < NB; j++) {
                         if ((msk >> j) & 1u) {
+                            A.e += 0.5 * v[0][j];
+                            A.rho += v[2][j];
                             double dx, dy, dz;
                             sep(h + j, dx, dy, dz);
-                            const double sc = v[j] / rr[j];
+                            const double sc = v[1][j] * ri[j];
                             A.x += sc * dx;
                             A.y += sc * dy;
                             A.z += sc * dz;
                         }
                     }
                 } else {
-                    cheb64_n<NB>(P.cheb + 4 * m, m, P.ca[1], P.cb[1], rr, v);  // rho', FP64 in both modes
+                    double v[1][NB];
+                    cheb_sums<NB, 1>(P.cheb, {4 * m}, m, P.ca[1], P.cb[1], rr, v);  // rho'
 #pragma unroll
                     for (int j = 0; j < NB; j++) {
                         if ((msk >> j) & 1u) {
@@ -1005,7 +1033,7 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
                             sep(h + j, dx, dy, dz);
                             if constexpr (MIXED) fij = (double)__uint_as_float(hq[hj[h + j]].w);
                             else fij = hf[hj[h + j]];
-                            const double g = (fia + fij) * v[j] / rr[j];
+                            const double g = (fia + fij) * v[0][j] * ri[j];
                             A.x += g * dx;
                             A.y += g * dy;
                             A.z += g * dz;
@@ -1107,8 +1135,11 @@ __device__ __forceinline__ void nl_atom(const DevState &d, const PotDev &P, cons
         // pass 2, src-flat/eam.c:576-594
         double fv, fp;
         if (EVAL == COMD_EVAL_CHEB) {
-            fv = cheb64(P.cheb + 2 * P.cstride, P.cstride, P.ca[2], P.cb[2], A.rho);
-            fp = cheb64(P.cheb + 5 * P.cstride, P.cstride, P.ca[2], P.cb[2], A.rho);
+            const double at[1] = {A.rho};
+            double v[2][1];
+            cheb_sums<1, 2>(P.cheb, {2 * P.cstride, 5 * P.cstride}, P.cstride, P.ca[2], P.cb[2], at, v);
+            fv = v[0][0];
+            fp = v[1][0];
         } else {
             interp64(P.tab[2], P.x0[2], P.xn[2], P.invdx[2], P.n[2], A.rho, fv, fp);
         }
@@ -1186,7 +1217,7 @@ constexpr int nl_pass_waves(int kind, int eval, int mixed, int lanes)
 // read from global memory (0); a compile-time choice, so the row reads are
 // LDS or global loads.  Dynamic LDS: [rows (TLDS)] [halo, hcap atoms].
 // Blocks of at most 768 threads (a group's home atoms); the Chebyshev passes
-// declare that bound, so that their four-pair recurrences (cheb64_n) get the
+// declare that bound, so that their four-pair recurrences (cheb_sums) get the
 // registers three waves per SIMD allow.
 template <int KIND, int EVAL, int MIXED, int TLDS, int LANES>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, EVAL == COMD_EVAL_CHEB ? 768 : 1024)))

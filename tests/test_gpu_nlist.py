@@ -384,3 +384,20 @@ def test_default_lanes_of_small_systems(gpu, cu500, evaluation, lanes):
     a, _ = pair_of_sims(cu500, 6, 3.615, 600.0, 0.1, 5, evaluation, "fp64")
     a.force()
     assert a.list_lanes() == lanes
+
+
+@pytest.mark.parametrize("ncheb", [3, 8, 9, 24, 31])
+def test_series_sums_of_the_list_passes(gpu, ncheb):
+    """The list passes share one basis between the FP64 series of phi, phi'
+    and rho where these have one domain; the link cells sum each series by
+    itself.  Equal domains and another one for rho; series of several
+    lengths.  Both sum n terms of size |c_k| with errors of k^2 2^-53 each
+    (the recurrences near the ends of the domain): 1e-12 for n <= 32."""
+    for shift in (0.0, 0.37):
+        pot = CA.EAMPotential("cu500", ncheb=ncheb)
+        pot.cheb_dom[1, 1] += shift
+        a, b = pair_of_sims(pot, 6, 3.615, 600.0, 0.1, 7, evaluation="cheby")
+        for s in (a, b):
+            s.force()
+        assert a.list_info()["valid"] == 1
+        assert_same(a, b, f"{ncheb} terms, shift {shift}", tol=1e-12)
