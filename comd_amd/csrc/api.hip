@@ -147,7 +147,9 @@ struct comd_ctx {
     int nl_active;      // lists allocated and usable for the atoms held
     int nl_stale;       // list positions not updated by the last drift
     int nl_invalid_seen; // the lists were invalid when the host last looked
-    int nl_group_opt;   // COMD_TUNE_LIST_GROUPS (-1: by precision)
+    int nl_group_opt;   // COMD_TUNE_LIST_GROUPS (-1: by size, nl_setup)
+    int nl_two_per_cu;  // the default shape of earlier snapshots: the largest with two groups per CU
+                        // (set by loading one)
     int nl_rows_lds;    // COMD_TUNE_LIST_ROWS_LDS (-1: whenever they fit)
     int nl_threads_div; // COMD_TUNE_LIST_THREADS_DIV: home atoms per thread of the list passes
     int nl_lanes;       // COMD_TUNE_LIST_LANES: lanes per home atom of the list passes (0: by size)
@@ -1007,17 +1009,20 @@ static int nl_setup(comd_ctx *c)
     const long lds_avail = (long)c->lds_block - CM_NL_STATIC_LDS;
     const long hb = c->precision == COMD_PREC_MIXED ? 16 : 32;
     std::vector<std::array<int, 3>> gd(nrep), na(nrep), ng(nrep);
-    long hcap = 0, naux = 0, ngroups = 0, threads = 64, build_threads = 64;
-    // lanes per home atom in the force passes: as tuned, else two when the
-    // atoms would fill fewer than two waves per CU at one lane each (each
-    // lane then walks half the list: 32 000 Lennard-Jones atoms, pass
-    // 0.034 -> 0.026 ms; at 256 000 atoms and above two lanes measured no
-    // better or slower).  Below that EAM passes are as long as one lane's
-    // list: four lanes below 8 atoms per CU (a step of 864 atoms, tables: 43.8 -> 41.6
-    // us; of 4000 57.4 against 56.8), and eight below 64 per CU for the
-    // Chebyshev passes, whose pairs are some 200 operations each (864 atoms
-    // FP64 79 -> 66 us, mixed 82 -> 64; 4000 atoms mixed 94 -> 84; 32 000
-    // FP64 130 against 116)
+    long hcap = 0, naux = 0, ngroups = 0, threads = 64, build_threads = 64, adj_threads = 64;
+    double load = 0.0;  // home atoms and a tenth of the staged ones, over all groups
+    // lanes per home atom in the force passes (each lane walks its share of
+    // the atom's list): as tuned, else by the atoms per CU, since a pass of few
+    // waves per SIMD runs at the latency of a lane's list.  EAM: two lanes
+    // below 2048 per CU (500 000 atoms: tables FP64 249 -> 240 us a step,
+    // mixed 200.6 against 201.3, Chebyshev FP64 483 -> 456; 1 098 500 atoms:
+    // 970 against 1006), four below 64 and for tables below 8 (Chebyshev, 864
+    // atoms 61 -> 53 us, eight lanes 60; 13 500 atoms 72 -> 65, eight 67;
+    // 32 000: 93 both ways; tables, 864 atoms 53.4 -> 51.2, 4000 60.0 against
+    // 61.9).  Lennard-Jones and batches, whose groups are shaped for one
+    // lane's threads: two below 128 per CU (32 000 Lennard-Jones atoms, pass 34 ->
+    // 26 us; 256 000 121 us a step against 130; 3 x 23 328 atoms' gradient 668
+    // against 682)
     long natoms_all = 0;
     bool lj = false, cheb = true;
     for (const Replica &R : c->reps) {
@@ -1025,12 +1030,11 @@ static int nl_setup(comd_ctx *c)
         lj |= R.prm.potential == COMD_POT_LJ;
         cheb &= R.pot.eval == COMD_EVAL_CHEB;
     }
-    const int lanes = c->nl_lanes > 0                                ? c->nl_lanes
-                      : natoms_all >= 128L * c->ncu                  ? 1
-                      : lj                                           ? 2
-                      : cheb && natoms_all < 64L * c->ncu            ? 8
-                      : natoms_all < 8L * c->ncu                     ? 4
-                                                                     : 2;
+    const int lanes = c->nl_lanes > 0                                       ? c->nl_lanes
+                      : natoms_all >= (lj || nrep > 1 ? 128L : 2048L) * c->ncu ? 1
+                      : lj                                                  ? 2
+                      : natoms_all < (cheb ? 64L : 8L) * c->ncu             ? 4
+                                                                            : 2;
     // threads of a pass' block for its group's home atoms: 10 % more than
     // the mean group's; 80 % where the system is small, whose groups of few
     // cells differ most in their atoms: one atom more than threads and the
@@ -1079,9 +1083,10 @@ static int nl_setup(comd_ctx *c)
         }
         return nr;
     };
-    auto shape = [&](int o) {  // fills gd, na, ng, hcap, naux, ngroups, threads, build_threads
+    auto shape = [&](int o) {  // fills gd, na, ng, hcap, naux, ngroups, load and the threads
         hcap = naux = ngroups = 0;
-        threads = build_threads = 64;
+        threads = build_threads = adj_threads = 64;
+        load = 0.0;
         for (int r = 0; r < nrep; r++) {
             long nr;
             if (o >= 0) {
@@ -1111,28 +1116,41 @@ static int nl_setup(comd_ctx *c)
             const double home = occ * (double)cells / c->nl_threads_div;
             threads = std::max<long>(threads, ((long)(spare * home * lanes) + 63) / 64 * 64);
             build_threads = std::max<long>(build_threads, ((long)(1.1 * home * build_lanes) + 63) / 64 * 64);
+            adj_threads = std::max<long>(adj_threads, ((long)(1.1 * home) + 63) / 64 * 64);
             naux += nr;
-            ngroups += (long)ng[r][0] * ng[r][1] * ng[r][2];
+            const long groups = (long)ng[r][0] * ng[r][1] * ng[r][2];
+            ngroups += groups;
+            load += (double)groups * occ * ((double)cells + 0.1 * (double)slots);
         }
     };
+    // One option for all: by default the one with the least work on the
+    // busiest CU, rounds of one group per CU times a group's home atoms and a
+    // tenth of its staged ones (the weight that orders the measured times of
+    // five shapes each at 32 000 to 2 048 000 atoms).  Against the largest
+    // shape with two groups per CU: 48 484 atoms FP64 tables 97 -> 79 us a step
+    // (4 x 2 x 2 cells in place of 2 x 2 x 2), 107 880 atoms 119 -> 98 and
+    // 256 000 181 -> 158 (4 x 4 x 2 in place of 4 x 2 x 2); the same at 2 048 000
     int best = -1;
-    long best_ng = -1;
+    bool per_replica = false;
     if (nrep > 1 && c->nl_group_opt < 0) {
         shape(-1);
-        if (hcap * (hb + 1) <= lds_avail && hcap <= 65535) best = -1, best_ng = 0;
-        else best_ng = -2;  // fall back to one option for all
+        per_replica = hcap * (hb + 1) <= lds_avail && hcap <= 65535;  // else one option for all
     }
-    if (best_ng != 0) {
+    if (!per_replica) {
+        double least = 0.0;
+        long most = -1;
         for (int o = c->nl_group_opt >= 0 ? c->nl_group_opt : 0; o < 5; o++) {
             shape(o);
             if (hcap * (hb + 1) > lds_avail || hcap > 65535) continue;
-            if (c->nl_group_opt >= 0 || ngroups >= 2L * c->ncu) {
+            if (c->nl_group_opt >= 0 || (c->nl_two_per_cu && ngroups >= 2L * c->ncu)) {
                 best = o;
                 break;
             }
-            if (ngroups > best_ng) {
+            const double cost = (double)((ngroups + c->ncu - 1) / c->ncu) * load / (double)ngroups;
+            if (c->nl_two_per_cu ? ngroups > most : best < 0 || cost < least) {
                 best = o;
-                best_ng = ngroups;
+                least = cost;
+                most = ngroups;
             }
         }
         if (best < 0) return COMD_OK;  // too dense for staged halos
@@ -1202,6 +1220,7 @@ static int nl_setup(comd_ctx *c)
     // threads per pass block: a group's home atoms with 10 % to spare
     l.pass_threads = (int)pass_threads;
     l.build_threads = (int)std::min<long>(768, build_threads);
+    l.adj_threads = (int)std::min<long>(768, adj_threads);
     l.gwords = (int)gwords;
     l.lanes = lanes;
     l.tailq = cm_nl_pick_tailq(l);
@@ -2367,9 +2386,26 @@ int comd_snapshot_load(comd_ctx *c, const char *path)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     // ... then the forces, the list words and the lists as they were
     const CmList &l = c->nl;
-    if (hdr[4] != c->nl_active ||
-        (c->nl_active && (hdr[6] != l.n || hdr[7] != l.kmax || hdr[9] != l.naux ||
-                          hdr[10] != l.ngroups || hdr[11] != l.hcap))) {
+    auto fits = [&] {
+        return hdr[4] == c->nl_active &&
+               (!c->nl_active || (hdr[6] == l.n && hdr[7] == l.kmax && hdr[9] == l.naux && hdr[10] == l.ngroups &&
+                                  hdr[11] == l.hcap));
+    };
+    if (!fits() && c->nl_group_opt < 0) {
+        // lists in the other of the two default shapes there have been
+        c->nl_two_per_cu = !c->nl_two_per_cu;
+        rc = nl_setup(c);
+        if (!rc && !fits()) {
+            c->nl_two_per_cu = !c->nl_two_per_cu;
+            rc = nl_setup(c);
+        }
+        if (rc) {
+            fclose(fp);
+            return rc;
+        }
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+    }
+    if (!fits()) {
         fclose(fp);
         return set_err(c, COMD_ERR_STATE, "the snapshot's neighbour lists do not fit this context");
     }
@@ -2633,13 +2669,15 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
     }
     // the pair passes over the neighbour lists when the context has them
     // (every group an EAM one, the staged halo in LDS) and, by default, there
-    // is a group per CU at least (a block per group: fewer groups leave CUs
-    // idle, where the link-cell passes, a wave per cell, measured faster);
-    // else over the link cells.  Whether the forward pass left the lists
-    // valid comes back with the results (waiting for it here left the GPU
-    // idle for some 40 us): if not, the link cells run after all
+    // are groups for five CUs in eight at least (a block per group: fewer
+    // leave CUs idle, where the link-cell passes, a wave per cell, are faster:
+    // a gradient of 32 000 atoms, 216 groups, 299 us against 391; of 4000, 54
+    // groups, 297 against 275); else over the link cells.  Whether the
+    // forward pass left the lists valid comes back with the results (waiting
+    // for it here left the GPU idle for some 40 us): if not, the link cells
+    // run after all
     bool nl = c->adj_lists && c->nl_active && !c->nl_invalid_seen && c->nl_lj_groups == 0 &&
-              (c->adj_lists == 2 || c->nl.pass_blocks >= c->ncu) &&
+              (c->adj_lists == 2 || 8L * c->nl.pass_blocks >= 5L * c->ncu) &&
               cm_adj_nl_lds(c->nl) + (12 << 10) <= (size_t)c->lds_block;
     std::vector<double> out((size_t)CM_ADJ_STAGES * NM), E3((size_t)3 * nrep);
     for (;;) {

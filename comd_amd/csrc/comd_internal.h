@@ -264,6 +264,7 @@ struct CmList {
     int rows_lds;            // table rows in LDS: 0 never, else whenever they fit
     int pass_blocks, pass_threads;  // one block per group (passes and build)
     int build_threads;       // of a build block
+    int adj_threads;         // of an adjoint pass' block (one lane per atom)
     int tailq;               // build: list entries per thread held back for the list's end (k_nl_build)
     int lanes;               // force passes: lanes per home atom (1, 2, 4, 8 or 16), each taking every
                              // lanes-th chunk of 8 entries of the atom's list

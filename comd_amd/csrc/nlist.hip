@@ -271,6 +271,14 @@ __device__ __forceinline__ unsigned group_slots(const CmList &l, int g, int w)
     return ((const CM_GLOBAL unsigned *)l.gslot)[((size_t)g * l.gwords + min(w, l.gwords - 1)) * blockDim.x + threadIdx.x];
 }
 
+// The slot of halo entry h, by any thread (the words are those of a force pass'
+// threads).
+__device__ __forceinline__ int group_slot(const CmList &l, int g, int h)
+{
+    const int k = h / l.pass_threads, t = h - k * l.pass_threads;
+    return ((const uint8_t *)l.gslot)[4 * (((size_t)g * l.gwords + (k >> 2)) * l.pass_threads + t) + (k & 3)];
+}
+
 // bytes (a multiple of 16) of global memory straight into LDS, 16 bytes a
 // lane, in flight until the caller's wait (vmcnt) and barrier: table rows need
 // no registers on the way and their wait is shared with the halo's.
@@ -727,10 +735,10 @@ __global__ __launch_bounds__(1024) void k_nl_tables(CmList l)
 // together (values in the convention of src-flat/cheby.c:290-310: c_0 / 2 +
 // sum of c_k T_k).  The basis is run forward, T_{k+1} = 2y T_k - T_{k-1}, and
 // shared by the series: S + 1 operations a term in place of the 2 S of a
-// Clenshaw sum for each.  Coefficients by scalar loads common to the N pairs, a block ahead of their
-// use; at[s]: the series' first coefficient from cg.  x[u] is clamped below at
-// a as in cheb64; the argument is formed with 1 / (b - a) computed once rather
-// than a division per pair.  The passes are bound by these operations (43 % of
+// Clenshaw sum for each.  Coefficients by scalar loads common to the N pairs,
+// a block ahead of their use; at[s]: the series' first coefficient from cg.
+// x[u] is clamped below at a as in cheb64; the argument is formed with
+// 1 / (b - a) computed once rather than a division per pair.  The passes are bound by these operations (43 % of
 // the issue slots of 256 000 atoms' FP64 density pass) and by the few waves
 // beside them: 248 -> 162 us, embedding force 118 -> 102; of the mixed passes
 // phi' and rho' alone take this sum: a step 351 -> 326 us, of 48 484 atoms
@@ -1394,14 +1402,12 @@ __global__ __launch_bounds__(768) void k_adj_nl(DevState d, PotDev P, CmList l, 
     const NlRep R = nl_rep(l, l.group_rep[g]);
     const GroupGeo G = group_geo(R, g - R.group_base);
     const int H = group_load(l, G, g, S);
-    unsigned word = group_slots(l, g, 0);
     const int t0 = l.gstart[g], t1 = l.gstart[g + 1];
     const double ox = (G.x0 + 0.5 * G.lx) * R.ab0, oy = (G.y0 + 0.5 * G.ly) * R.ab1,
                  oz = (G.z0 + 0.5 * G.lz) * R.ab2;
     __syncthreads();
-    for (int h = threadIdx.x, n = 0; h < H; h += blockDim.x, n++) {
-        if (n > 0 && (n & 3) == 0) word = group_slots(l, g, n >> 2);
-        const int sl = (int)((word >> (8 * (n & 3))) & 0xffu);
+    for (int h = threadIdx.x; h < H; h += blockDim.x) {
+        const int sl = group_slot(l, g, h);
         slot_of[h] = (uint8_t)sl;
         const CmPos p = load_pos(l.pos, S.base[sl] + h);
         frame_pos(R, G, S.uxyz[sl], p, ox, oy, oz, hx[h], hy[h], hz[h]);
@@ -1624,7 +1630,7 @@ template <int MIXED, int NC>
 static void adj_nl_launch(const DevState &d, const PotDev &P, const CmList &l, const CmAdjNl &A, int pass,
                           hipStream_t st)
 {
-    const dim3 grid(l.pass_blocks), block(l.pass_threads);
+    const dim3 grid(l.pass_blocks), block(l.adj_threads);
     const size_t lds = cm_adj_nl_lds(l);
     switch (pass) {
     case 1: hipLaunchKernelGGL((k_adj_nl<1, MIXED, NC>), grid, block, lds, st, d, P, l, A); break;

@@ -178,15 +178,16 @@ enum comd_tune_key {
     COMD_TUNE_LIST_GROUPS = 9,     /* -1 (default), 0..4: auxiliary cells per group of the
                                       neighbour-list passes, 4x4x3, 4x4x2, 4x2x2, 2x2x2, 2x2x1 (from the
                                       option given, the first whose staged halo fits the LDS of a
-                                      block; by default the largest fitting shape that still gives two
-                                      groups per compute unit, else the one with the most groups) */
+                                      block; by default the fitting shape with the least work on the
+                                      busiest compute unit: rounds of one group per unit times a
+                                      group's own atoms and a tenth of its staged ones) */
     COMD_TUNE_LIST_ROWS_LDS = 10,  /* -1 (default, = 1), 0, 1: table rows of the list passes staged in
                                       LDS when they fit beside the halo */
     COMD_TUNE_LIST_THREADS_DIV = 11, /* 1 (default) or 2..4: home atoms per thread of the list passes
                                       (threads per block = a group's atoms / this, in waves) */
     COMD_TUNE_ADJOINT_LISTS = 12,  /* the adjoint's pair passes over the neighbour lists when the
-                                      context uses them: 1 (default) if it has a list group per CU at
-                                      least, 2 always, 0 never (link cells) */
+                                      context uses them: 1 (default) if it has list groups for five CUs
+                                      in eight at least, 2 always, 0 never (link cells) */
     COMD_TUNE_LIST_LANES = 13,     /* 0 (default): by the system's size; 1, 2, 4, 8 or 16: adjacent lanes per
                                       home atom in the list force passes, each taking every lanes-th
                                       chunk of the atom's list (more waves for small systems) */

@@ -379,7 +379,7 @@ def test_eight_and_sixteen_lanes_equal_one(gpu, cu500, lanes, evaluation, precis
                 tol=1e-6 if (evaluation, precision) == ("table", "mixed") else 1e-12)
 
 
-@pytest.mark.parametrize("evaluation,lanes", [("table", 4), ("cheby", 8)])
+@pytest.mark.parametrize("evaluation,lanes", [("table", 4), ("cheby", 4)])
 def test_default_lanes_of_small_systems(gpu, cu500, evaluation, lanes):
     a, _ = pair_of_sims(cu500, 6, 3.615, 600.0, 0.1, 5, evaluation, "fp64")
     a.force()

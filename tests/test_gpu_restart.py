@@ -52,3 +52,30 @@ def test_restart_continues_bit_for_bit(gpu, cu500, tmp_path, precision, lanes):
 def test_restart_with_more_lanes(gpu, cu500, tmp_path, lanes):
     """The lanes per atom come from the file for any number there is."""
     test_restart_continues_bit_for_bit(gpu, cu500, tmp_path, "fp64", lanes)
+
+
+def test_restart_from_lists_of_the_earlier_default_shape(gpu, cu500, tmp_path):
+    """Snapshots of 32 000 atoms were written with 2 x 2 x 1 cells to a group
+    by default, now 2 x 2 x 2: a context with the default takes the file's
+    shape and continues bit for bit; one whose shape was tuned refuses it."""
+    n = 20
+    xyz, p, bounds = seeded_atoms(n, 3.615, cu500.mass, temp=600.0, disp=0.1, seed=5)
+    path = str(tmp_path / "s.bin")
+    a = CA.Simulation(cu500, bounds, defgrad=0.0)
+    a.tune(list_groups=4)
+    a.bin_atoms(xyz, p)
+    a.force()
+    a.nsteps(5)
+    a.snapshot_save(path)
+    b = CA.Simulation(cu500, bounds, defgrad=0.0)
+    b.snapshot_load(path)
+    c = CA.Simulation(cu500, bounds, defgrad=0.0)
+    c.tune(list_groups=2)
+    with pytest.raises(CA.ComdError):
+        c.snapshot_load(path)
+    for s in (a, b):
+        s.nsteps(30)
+    assert b.list_info()["valid"] == 1
+    ga, gb = a.download(), b.download()
+    for k in ("natoms", "id", "itype", "r", "p", "f", "rho", "fi"):
+        assert np.array_equal(ga[k], gb[k]), k
