@@ -227,168 +227,201 @@ __global__ __launch_bounds__(64) void k_move4(DevState d, double dtk, double dtd
         move_atom<TWO>(d, g, c, ix, iy, iz, c * CM_SLOTS + t, dtk, dtd, kick, drift, rebin);
 }
 
+// The two kernels below are chains of cache misses (the lists were written by
+// other XCDs), so what a cell needs is read in as few turns as its addresses
+// allow, wanted or not: the cell beside the number of touched cells, then its
+// words, arrivals and movers, then the movers' records.  With the scan in
+// registers (it ran in LDS, one lane over every slot), the four launches of a
+// step: 864 atoms 50.5 -> 48.5 us a step, 32 000 70 -> 66, 48 484 131.7 -> 128,
+// 256 000 FP64 152 -> 148.7, 2 048 000 632 -> 629.
+
+// Touched cell i of pass P, read beside their number; -1 past the end.
+__device__ __forceinline__ int first_touched(const RebinSet &P, int i)
+{
+    int c = P.tc[i], n = *P.ntc;
+    asm volatile("" : "+v"(c), "+v"(n));  // both loads before the branch
+    return __builtin_amdgcn_readfirstlane(i < n ? c : -1);
+}
+
 // Per touched cell (one wave each): count arrivals from lower/higher cells,
-// then run the cell's own swap-with-last scan with n_low never-departing
+// then the cell's own swap-with-last scan with n_low never-departing
 // placeholders appended, recording each departure's rank and the resulting
-// arrangement.  The lanes load the arrivals and the departing atoms' mover
-// records together; lane 0 runs the scan in LDS.
+// arrangement.  Only departures are walked: the atoms and placeholders beyond
+// the shrinking end are where they began, so the element that fills a hole, or
+// leaves in its turn, is known from its place (lane L keeps slot L's rank and
+// what ends in it).
 // second: pass B of a fused pair (P: its lists).  A replica with a flag of the
 // pass or an earlier one is left out.
 __global__ __launch_bounds__(64) void k_rebox_scan(DevState d, RebinSet P, int second)
 {
-    __shared__ uint8_t perm[128];
-    __shared__ int rank_of[CM_SLOTS];
     const int L = threadIdx.x;
-    const int ntc = *P.ntc, replay = second ? 3 : 1;
-    for (int i = blockIdx.x; i < ntc; i += gridDim.x) {
-        const int c = P.tc[i];
-        if (d.mh[rep_of(d, c)] & replay) continue;  // the same in every lane: replayed serially
-        const int n0 = d.natoms[c];
-        int na = P.arr_cnt[c];
-        // which of the cell's own atoms leave (set by k_move per departure)
-        const unsigned long long leaves = P.leave[c];
-        unsigned fl = 0;
-        if (na > CM_ACAP) {
-            fl |= CM_FLAG_OVERFLOW;
-            na = CM_ACAP;
-        }
-        bool low = false;
-        if (L < na) low = (d.mv_slot[P.arr[c * CM_ACAP + L]] / CM_SLOTS) < c;
-        const bool leaving = L < n0 && ((leaves >> L) & 1ull);
-        const int mv = leaving ? d.mvidx[c * CM_SLOTS + L] : -1;
-        const int nlow = __popcll(__ballot(low));
-        const int nhigh = na - nlow;
-        if (nlow > 0 && n0 + nlow >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
-        int len = n0 + nlow;
-        if (len > 127) len = 127;
-        for (int k = L; k < len; k += 64) perm[k] = (uint8_t)(k < n0 ? k : CM_SLOTS + (k - n0));
-        __syncthreads();
-        if (L == 0) {
-            int p = 0, rk = 0;
-            while (p < len) {
-                const int e = perm[p];
-                if (e < CM_SLOTS && ((leaves >> e) & 1ull)) {
-                    rank_of[e] = rk++;
+    const int replay = second ? 3 : 1;
+    int c = first_touched(P, blockIdx.x);
+    if (c < 0) return;
+    const int ntc = *P.ntc;
+    for (int i = blockIdx.x;;) {
+        int rep = d.mh[rep_of(d, c)], n0 = d.natoms[c], na = P.arr_cnt[c];
+        unsigned long long leaves = P.leave[c];  // set by k_move per departure
+        int m = P.arr[c * CM_ACAP + L], mv = d.mvidx[c * CM_SLOTS + L];
+        asm volatile("" : "+v"(rep), "+v"(n0), "+v"(na), "+v"(leaves), "+v"(m), "+v"(mv));
+        n0 = __builtin_amdgcn_readfirstlane(n0);
+        na = __builtin_amdgcn_readfirstlane(na);
+        if (!(__builtin_amdgcn_readfirstlane(rep) & replay)) {  // else replayed serially
+            unsigned fl = 0;
+            if (na > CM_ACAP) {
+                fl |= CM_FLAG_OVERFLOW;
+                na = CM_ACAP;
+            }
+            bool low = false;
+            if (L < na) low = d.mv_slot[m] / CM_SLOTS < c;
+            unsigned long long left = (unsigned)__builtin_amdgcn_readfirstlane((int)leaves) |
+                                      (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(leaves >> 32)) << 32;
+            if (n0 < CM_SLOTS) left &= (1ull << n0) - 1;
+            const bool leaving = (left >> L) & 1ull;
+            const int nlow = __popcll(__ballot(low));
+            const int nhigh = na - nlow;
+            if (nlow > 0 && n0 + nlow >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
+            int len = n0 + nlow;
+            if (len > 127) len = 127;
+            int rank = 0, rk = 0;
+            int in = L < n0 ? L : CM_SLOTS + (L - n0);  // what slot L holds at the end
+            while (left) {
+                const int p = __ffsll((long long)left) - 1;  // the next hole
+                left &= left - 1;
+                for (int e = p;;) {
+                    if (L == e) rank = rk;
+                    rk++;
                     len--;
-                    perm[p] = perm[len];
-                } else {
-                    p++;
+                    if (len == p) break;  // the last one itself
+                    if (len < CM_SLOTS && ((left >> len) & 1ull)) {
+                        e = len;  // the last one fills the hole and leaves too
+                        left &= ~(1ull << e);
+                        continue;
+                    }
+                    if (L == p) in = len < n0 ? len : CM_SLOTS + (len - n0);
+                    break;
                 }
             }
+            if (leaving) d.mv_rank[mv] = rank;
+            if (nhigh > 0 && len + nhigh >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
+            const int keep = len < CM_SLOTS ? len : CM_SLOTS;
+            if (L < keep) d.perm[c * CM_SLOTS + L] = (uint8_t)in;
+            if (L == 0) {
+                d.meta[4 * c + 0] = len;
+                d.meta[4 * c + 1] = nlow;
+                d.meta[4 * c + 2] = nhigh;
+                d.meta[4 * c + 3] = n0;
+                if (fl) atomicOr(d.flags, fl);
+            }
         }
-        len = __shfl(len, 0, 64);
-        __syncthreads();
-        if (leaving) d.mv_rank[mv] = rank_of[L];
-        if (nhigh > 0 && len + nhigh >= CM_SLOTS) fl |= CM_FLAG_OVERFLOW;
-        const int keep = len < CM_SLOTS ? len : CM_SLOTS;
-        if (L < keep) d.perm[c * CM_SLOTS + L] = perm[L];
-        if (L == 0) {
-            d.meta[4 * c + 0] = len;
-            d.meta[4 * c + 1] = nlow;
-            d.meta[4 * c + 2] = nhigh;
-            d.meta[4 * c + 3] = n0;
-            if (fl) atomicOr(d.flags, fl);
-        }
-        __syncthreads();
+        i += gridDim.x;
+        if (i >= ntc) return;
+        c = P.tc[i];
     }
 }
 
 // Per touched cell (one wave each, lane = output slot): order the arrivals by
 // (source cell, rank), then write survivors and low arrivals in the scanned
-// arrangement followed by the high arrivals.  All lanes read before any lane
+// arrangement followed by the high arrivals.  Lane L reads arrival L's record,
+// the output lanes take it from there.  All lanes read before any lane
 // writes, so the cell is updated in place.  Clears the cell's pass state.
 // FIRST: pass A of a fused pair; the moves of pass B by the cell's atoms are
 // put under their new slots, and those of its arrivals recorded.
 template <int FIRST>
 __global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int second)
 {
-    __shared__ int sm[2][CM_SLOTS];  // movers by low / high arrival order
+    __shared__ int sm[2][CM_SLOTS];  // arrivals by low / high order
     const int L = threadIdx.x;
-    const int ntc = *P.ntc, replay = second ? 3 : 1;
-    for (int i = blockIdx.x; i < ntc; i += gridDim.x) {
-        const int c = P.tc[i];
+    const int replay = second ? 3 : 1;
+    int c = first_touched(P, blockIdx.x);
+    if (c < 0) return;
+    const int ntc = *P.ntc;
+    for (int i = blockIdx.x;;) {
+        int rep = d.mh[rep_of(d, c)], len = d.meta[4 * c + 0], nhigh = d.meta[4 * c + 2], na = P.arr_cnt[c];
+        int m = P.arr[c * CM_ACAP + L], e = d.perm[c * CM_SLOTS + L];
+        unsigned long long leave_b = FIRST ? d.rb.leave[c] : 0ull;
+        asm volatile("" : "+v"(rep), "+v"(len), "+v"(nhigh), "+v"(na), "+v"(m), "+v"(e), "+v"(leave_b));
+        len = __builtin_amdgcn_readfirstlane(len);
+        nhigh = __builtin_amdgcn_readfirstlane(nhigh);
+        na = __builtin_amdgcn_readfirstlane(na);
         // cells of a replica whose pass is replayed serially are left as the
         // move kernel left them (the same in every lane)
-        const bool serial = (d.mh[rep_of(d, c)] & replay) != 0;
+        const bool serial = (__builtin_amdgcn_readfirstlane(rep) & replay) != 0;
         if (!serial) {
-            const int len = d.meta[4 * c + 0];
-            const int nhigh = d.meta[4 * c + 2];
-            int na = P.arr_cnt[c];
             na = na < CM_ACAP ? na : CM_ACAP;
-            int m = -1, src = 0, rk = 0;
-            if (L < na) {
-                m = P.arr[c * CM_ACAP + L];
-                src = d.mv_slot[m] / CM_SLOTS;
-                rk = d.mv_rank[m];
-            }
-            // rank among arrivals of the same class, by (source cell, rank)
-            const bool low = src < c;
-            int pos = 0;
-            for (int u = 0; u < na; u++) {
-                const int su = __shfl(src, u, 64);
-                const int ru = __shfl(rk, u, 64);
-                const bool lu = su < c;
-                pos += (lu == low) && (su < src || (su == src && ru < rk));
-            }
-            if (L < na && pos < CM_SLOTS) sm[low ? 0 : 1][pos] = m;
-            __syncthreads();
-            // gather this lane's output atom
             const int tot = len + nhigh;
             const int nout = tot < CM_SLOTS ? tot : CM_SLOTS;
             const int keep = len < CM_SLOTS ? len : CM_SLOTS;
-            int gid = 0, git = 0;
-            float4 gq = {0.0f, 0.0f, 0.0f, 0.0f};
-            double gx = 0, gy = 0, gz = 0, gpx = 0, gpy = 0, gpz = 0;
-            int mv = -1, own = -1, mb = -1;
-            if (L < nout) {
-                if (L < keep) {
-                    const int e = d.perm[c * CM_SLOTS + L];
-                    if (e < CM_SLOTS) own = c * CM_SLOTS + e;
-                    else mv = sm[0][(e - CM_SLOTS) & (CM_SLOTS - 1)];
-                } else {
-                    mv = sm[1][(L - len) & (CM_SLOTS - 1)];
+            int src = 0, rk = 0;
+            Mover in = {};  // arrival L
+            if (L < na) {
+                src = d.mv_slot[m] / CM_SLOTS;
+                rk = d.mv_rank[m];
+                in = Mover{d.mv_rx[m], d.mv_ry[m], d.mv_rz[m], d.mv_px[m], d.mv_py[m], d.mv_pz[m],
+                           d.mv_nlr[m], d.mv_id[m], d.mv_itype[m]};
+            }
+            Mover out = {};
+            const int own = L < keep && e < CM_SLOTS ? c * CM_SLOTS + e : -1;
+            int mb = -1;
+            if (own >= 0) {
+                if (FIRST && ((leave_b >> e) & 1ull)) mb = d.mvidx[own];
+                out = Mover{d.rx[own], d.ry[own], d.rz[own], d.px[own], d.py[own], d.pz[own],
+                            d.nlr[own], d.id[own], d.itype[own]};
+            }
+            bool arrived = false;
+            if (na > 0) {
+                // rank among arrivals of the same class, by (source cell, rank)
+                const bool low = src < c;
+                int pos = 0;
+                for (int u = 0; u < na; u++) {
+                    const int su = __shfl(src, u, 64);
+                    const int ru = __shfl(rk, u, 64);
+                    const bool lu = su < c;
+                    pos += (lu == low) && (su < src || (su == src && ru < rk));
                 }
-                if (own >= 0) {
-                    if (FIRST && ((d.rb.leave[c] >> (own - c * CM_SLOTS)) & 1ull)) mb = d.mvidx[own];
-                    gid = d.id[own];
-                    gq = d.nlr[own];
-                    git = d.itype[own];
-                    gx = d.rx[own];
-                    gy = d.ry[own];
-                    gz = d.rz[own];
-                    gpx = d.px[own];
-                    gpy = d.py[own];
-                    gpz = d.pz[own];
-                } else if (mv >= 0) {
-                    gid = d.mv_id[mv];
-                    gq = d.mv_nlr[mv];
-                    git = d.mv_itype[mv];
-                    gx = d.mv_rx[mv];
-                    gy = d.mv_ry[mv];
-                    gz = d.mv_rz[mv];
-                    gpx = d.mv_px[mv];
-                    gpy = d.mv_py[mv];
-                    gpz = d.mv_pz[mv];
+                if (L < na && pos < CM_SLOTS) sm[low ? 0 : 1][pos] = L;
+                __syncthreads();
+                int from = L;
+                if (L < nout && own < 0) {
+                    arrived = true;
+                    from = L < keep ? sm[0][(e - CM_SLOTS) & (CM_SLOTS - 1)] : sm[1][(L - len) & (CM_SLOTS - 1)];
+                }
+                auto take = [&](double &o, double v) {
+                    v = __shfl(v, from, 64);
+                    if (arrived) o = v;
+                };
+                take(out.x, in.x);
+                take(out.y, in.y);
+                take(out.z, in.z);
+                take(out.px, in.px);
+                take(out.py, in.py);
+                take(out.pz, in.pz);
+                const float qx = __shfl(in.nlr.x, from, 64), qy = __shfl(in.nlr.y, from, 64),
+                            qz = __shfl(in.nlr.z, from, 64), qw = __shfl(in.nlr.w, from, 64);
+                const int id = __shfl(in.id, from, 64), itype = __shfl(in.itype, from, 64);
+                if (arrived) {
+                    out.nlr = make_float4(qx, qy, qz, qw);
+                    out.id = id;
+                    out.itype = itype;
                 }
             }
             __syncthreads();  // every lane has read its source before any slot is overwritten
+            const int o = c * CM_SLOTS + L;
             if (L < nout) {
-                const int o = c * CM_SLOTS + L;
-                if (d.nl_slot) d.nl_slot[grid_of(d, c).nl_id_base + gid] = o;
-                d.id[o] = gid;
-                d.nlr[o] = gq;
-                d.itype[o] = git;
-                d.rx[o] = gx;
-                d.ry[o] = gy;
-                d.rz[o] = gz;
-                d.px[o] = gpx;
-                d.py[o] = gpy;
-                d.pz[o] = gpz;
+                if (d.nl_slot) d.nl_slot[grid_of(d, c).nl_id_base + out.id] = o;
+                d.id[o] = out.id;
+                d.nlr[o] = out.nlr;
+                d.itype[o] = out.itype;
+                d.rx[o] = out.x;
+                d.ry[o] = out.y;
+                d.rz[o] = out.z;
+                d.px[o] = out.px;
+                d.py[o] = out.py;
+                d.pz[o] = out.pz;
             }
             if (L == 0) d.natoms[c] = nout;
             if (FIRST) {
                 // pass B: the cell's own movers renamed, its arrivals' found
-                const int o = c * CM_SLOTS + L;
                 if (mb >= 0) {
                     d.mvidx[o] = mb;
                     d.mv_slot[mb] = o;
@@ -396,16 +429,16 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int
                 const Grid g = grid_of(d, c);
                 double bx = 0, by = 0, bz = 0;
                 int dstb = -1;
-                if (mv >= 0) {
+                if (arrived) {
                     int ix, iy, iz;
                     cell_xyz(g, c, ix, iy, iz);
-                    dstb = hop(g, c, ix, iy, iz, gx, gy, gz, bx, by, bz);
+                    dstb = hop(g, c, ix, iy, iz, out.x, out.y, out.z, bx, by, bz);
                 }
                 const unsigned long long leave = __ballot(mb >= 0 || dstb >= 0);
                 if (L == 0) d.rb.leave[c] = leave;
                 if (dstb >= 0) {
                     if (hops_again(g, c, dstb, bx, by, bz)) request_replay(d, g, 2);
-                    put_mover(d, d.rb, c, o, dstb, Mover{bx, by, bz, gpx, gpy, gpz, gq, gid, git});
+                    put_mover(d, d.rb, c, o, dstb, Mover{bx, by, bz, out.px, out.py, out.pz, out.nlr, out.id, out.itype});
                 }
             }
         }
@@ -416,6 +449,9 @@ __global__ __launch_bounds__(64) void k_rebox_gather(DevState d, RebinSet P, int
             if (!(FIRST && serial)) P.leave[c] = 0;
         }
         __syncthreads();
+        i += gridDim.x;
+        if (i >= ntc) return;
+        c = P.tc[i];
     }
 }
 

@@ -211,3 +211,48 @@ def test_replay_of_the_second_pass_alone():
     m = (np.arange(M)[None, :] < natoms[:, None]).reshape(-1)
     assert np.array_equal(st["natoms"], natoms) and np.array_equal(st["id"][m], ids[m])
     assert np.array_equal(st["r"][m], r[m])
+
+
+def scan_by_slots(n0, nlow, leaves):
+    """The reference's scan of one cell: rank of each departure, and what is
+    in each slot at the end (64 and up: the low arrivals)."""
+    perm = list(range(n0)) + [M + k for k in range(nlow)]
+    rank, p, n = {}, 0, n0 + nlow
+    while p < n:
+        e = perm[p]
+        if e < M and e in leaves:
+            rank[e] = len(rank)
+            n -= 1
+            perm[p] = perm[n]
+        else:
+            p += 1
+    return rank, perm[:n]
+
+
+def scan_by_departures(n0, nlow, leaves):
+    """The same, walking the departures alone (k_rebox_scan)."""
+    left, rank, n = sorted(leaves), {}, n0 + nlow
+    perm = [k if k < n0 else M + k - n0 for k in range(n)]
+    while left:
+        p = e = left.pop(0)
+        while True:
+            rank[e] = len(rank)
+            n -= 1
+            if n == p:
+                break
+            if n in left:
+                e = n
+                left.remove(n)
+                continue
+            perm[p] = n if n < n0 else M + n - n0
+            break
+    return rank, perm[:n]
+
+
+def test_scan_by_departures_equals_scan_by_slots():
+    rng = np.random.default_rng(3)
+    for _ in range(4000):
+        n0, nlow = int(rng.integers(0, M + 1)), int(rng.choice([0, 0, 1, 2, 5, 20, 64]))
+        k = int(rng.integers(0, n0 + 1)) if rng.uniform() < 0.5 else min(n0, int(rng.integers(0, 4)))
+        leaves = set(rng.permutation(n0)[:k].tolist())
+        assert scan_by_slots(n0, nlow, leaves) == scan_by_departures(n0, nlow, leaves)
