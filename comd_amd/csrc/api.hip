@@ -127,7 +127,7 @@ struct comd_ctx {
     int adj_nblocks;
     double *adj_gb, *adj_part_nl;  // list passes: dL/df in build order, partial moments
     long adj_gb_cap, adj_part_nl_cap;
-    int adj_lists;        // COMD_TUNE_ADJOINT_LISTS: 0 link cells, 1 lists with a group per CU, 2 lists
+    int adj_lists;        // COMD_TUNE_ADJOINT_LISTS: 0 link cells, 1 lists from a size on, 2 lists
     int adj_have_target;  // adj_ft holds a target (comd_eam_cheb_grad with f_target NULL reuses it)
     double *adj_E;        // per replica: the energy reduction's output (3 doubles each)
     double *adj_epart;    // per replica: its energy reduction's partials (nparts x 3 doubles)
@@ -2668,16 +2668,16 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
         cm_launch_adj_resid(d, J, c->adj_ft, c->stream);
     }
     // the pair passes over the neighbour lists when the context has them
-    // (every group an EAM one, the staged halo in LDS) and, by default, there
-    // are groups for five CUs in eight at least (a block per group: fewer
-    // leave CUs idle, where the link-cell passes, a wave per cell, are faster:
-    // a gradient of 32 000 atoms, 216 groups, 299 us against 391; of 4000, 54
-    // groups, 297 against 275); else over the link cells.  Whether the
-    // forward pass left the lists valid comes back with the results (waiting
-    // for it here left the GPU idle for some 40 us): if not, the link cells
-    // run after all
+    // (every group an EAM one, the staged halo in LDS) and, by default, they
+    // fill the chip: 72 atoms per CU, in a batch a group per CU (a block per
+    // group; with fewer the link-cell passes, a wave per cell, are as fast or
+    // faster: a gradient of 32 000 atoms 299 us against 391, of 16 384 300
+    // against 299, of 4000 297 against 275); else over the link cells.  Whether
+    // the forward pass left the lists valid comes back with the results
+    // (waiting for it here left the GPU idle for some 40 us): if not, the link
+    // cells run after all
     bool nl = c->adj_lists && c->nl_active && !c->nl_invalid_seen && c->nl_lj_groups == 0 &&
-              (c->adj_lists == 2 || 8L * c->nl.pass_blocks >= 5L * c->ncu) &&
+              (c->adj_lists == 2 || (nrep > 1 ? c->nl.pass_blocks >= c->ncu : c->ntot >= 72L * c->ncu)) &&
               cm_adj_nl_lds(c->nl) + (12 << 10) <= (size_t)c->lds_block;
     std::vector<double> out((size_t)CM_ADJ_STAGES * NM), E3((size_t)3 * nrep);
     for (;;) {

@@ -186,8 +186,8 @@ enum comd_tune_key {
     COMD_TUNE_LIST_THREADS_DIV = 11, /* 1 (default) or 2..4: home atoms per thread of the list passes
                                       (threads per block = a group's atoms / this, in waves) */
     COMD_TUNE_ADJOINT_LISTS = 12,  /* the adjoint's pair passes over the neighbour lists when the
-                                      context uses them: 1 (default) if it has list groups for five CUs
-                                      in eight at least, 2 always, 0 never (link cells) */
+                                      context uses them: 1 (default) from 72 atoms per CU on, in a batch
+                                      from a list group per CU on, 2 always, 0 never (link cells) */
     COMD_TUNE_LIST_LANES = 13,     /* 0 (default): by the system's size; 1, 2, 4, 8 or 16: adjacent lanes per
                                       home atom in the list force passes, each taking every lanes-th
                                       chunk of the atom's list (more waves for small systems) */
