@@ -325,6 +325,7 @@ __global__ __launch_bounds__(1024) void k_adj_final(CmAdjParts J)
     const double *part = J.part[blockIdx.x];
     const int nblocks = J.nblocks[blockIdx.x];
     const int k = threadIdx.x & 63, j = threadIdx.x >> 6;
+    if (blockIdx.x == 0 && threadIdx.x == 0) J.out[CM_ADJ_STAGES * ANMOM] = J.nl_flags ? (double)*J.nl_flags : 0.0;
     double s = 0.0;
     for (int b0 = j * 8; b0 < nblocks; b0 += 16 * 8) {
         double v[8];

@@ -457,6 +457,16 @@ static int run_steps(comd_ctx *c, int n, double dt)
     return COMD_OK;
 }
 
+// The host has seen the lists' flags.  Lists found invalid: the link-cell
+// passes beside the list passes get their full grid until the lists are valid
+// again.
+static void lists_seen(comd_ctx *c, unsigned flags)
+{
+    const int inv = (flags & CM_NL_INVALID) != 0;
+    if (inv != c->nl_invalid_seen) invalidate_graph(c);
+    c->nl_invalid_seen = inv;
+}
+
 static int check_flags(comd_ctx *c)
 {
     HIPCHK(c, hipMemcpyAsync(c->host_flags, c->flags, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
@@ -464,13 +474,7 @@ static int check_flags(comd_ctx *c)
         HIPCHK(c, hipMemcpyAsync(c->host_flags + 1, c->nl.flags, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const unsigned f = *c->host_flags;
-    // lists found invalid: the link-cell passes beside the list passes get
-    // their full grid until the lists are valid again
-    if (c->nl_active) {
-        const int inv = (c->host_flags[1] & CM_NL_INVALID) != 0;
-        if (inv != c->nl_invalid_seen) invalidate_graph(c);
-        c->nl_invalid_seen = inv;
-    }
+    if (c->nl_active) lists_seen(c, c->host_flags[1]);
     if (f & CM_FLAG_OVERFLOW) return set_err(c, COMD_ERR_OVERFLOW, "a link cell reached %d atoms", CM_SLOTS);
     if (f & CM_FLAG_OUTSIDE) return set_err(c, COMD_ERR_OUTSIDE, "an atom fell outside the cell grid");
     return COMD_OK;
@@ -2594,7 +2598,7 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
         alloc((void **)&c->adj_ft, S * 3 * 8);
         alloc((void **)&c->adj_f2, 64 * 8);
         alloc((void **)&c->adj_part, (size_t)CM_ADJ_STAGES * c->adj_nblocks * NM * 8);
-        alloc((void **)&c->adj_out, (size_t)CM_ADJ_STAGES * NM * 8);
+        alloc((void **)&c->adj_out, ((size_t)CM_ADJ_STAGES * NM + 1) * 8);
         alloc((void **)&c->adj_rep, (size_t)2 * c->nrep * 8);
         alloc((void **)&c->adj_E, (size_t)3 * c->nrep * 8);
         alloc((void **)&c->adj_epart, (size_t)3 * c->nrep * c->nparts * 8);
@@ -2668,6 +2672,7 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
         J.parts.nblocks[k] = c->adj_nblocks;
     }
     J.parts.out = c->adj_out;
+    J.parts.nl_flags = c->nl_active ? c->nl.flags : nullptr;
     PotDev P = R0.pot;  // series, domains and cutoff common to the replicas
     P.eval = COMD_EVAL_CHEB;
     DevState d = dev_state(c);
@@ -2684,11 +2689,11 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
     // against 299, of 4000 297 against 275); else over the link cells.  Whether
     // the forward pass left the lists valid comes back with the results
     // (waiting for it here left the GPU idle for some 40 us): if not, the link
-    // cells run after all
+    // cells run after all, and at once in the calls that follow
     bool nl = c->adj_lists && c->nl_active && !c->nl_invalid_seen && c->nl_lj_groups == 0 &&
               (c->adj_lists == 2 || (nrep > 1 ? c->nl.pass_blocks >= c->ncu : c->ntot >= 72L * c->ncu)) &&
               cm_adj_nl_lds(c->nl) + (12 << 10) <= (size_t)c->lds_block;
-    std::vector<double> out((size_t)CM_ADJ_STAGES * NM), E3((size_t)3 * nrep);
+    std::vector<double> out((size_t)CM_ADJ_STAGES * NM + 1), E3((size_t)3 * nrep);
     for (;;) {
         CmAdjoint K = J;
         if (nl) {
@@ -2734,10 +2739,9 @@ static int cheb_grad(comd_ctx *c, const double *coef, int n, const double *f_tar
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipMemcpyAsync(out.data(), c->adj_out, out.size() * 8, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipMemcpyAsync(E3.data(), c->adj_E, E3.size() * 8, hipMemcpyDeviceToHost, c->stream));
-        if (nl)
-            HIPCHK(c, hipMemcpyAsync(c->host_flags + 1, c->nl.flags, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        if (!nl || !(c->host_flags[1] & CM_NL_INVALID)) break;
+        if (c->nl_active) lists_seen(c, (unsigned)out.back());
+        if (!nl || !c->nl_invalid_seen) break;
         nl = false;
     }
     double lossE = 0.0;

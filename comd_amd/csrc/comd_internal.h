@@ -181,11 +181,13 @@ void cm_launch_adj_rep(const double *E, const double *w, const double *rw, int n
 
 // Partial moments of the adjoint's stages 0-3 and, as stage 4, of the weighted
 // sum of squared force residuals: per stage its blocks' partials
-// (cm_adjoint_moments() doubles each) and their number; out: their sums.
+// (cm_adjoint_moments() doubles each) and their number; out: their sums, then
+// the lists' flags as the forward pass left them (0 without lists).
 #define CM_ADJ_STAGES 5
 struct CmAdjParts {
     double *part[CM_ADJ_STAGES];
     int nblocks[CM_ADJ_STAGES];
+    const unsigned *nl_flags;
     double *out;
 };
 // Device buffers and scalars of the Chebyshev-coefficient adjoint

@@ -423,3 +423,59 @@ def test_series_of_every_length_equal_their_zero_padded_32(gpu, cu500, n, precis
         err = np.abs(gn - gp[:, :n]).max(axis=1) / np.abs(gp).max(axis=1)
         print(f"[{n} terms, {precision}, lists={lists}] {err}", flush=True)
         assert (err <= tol).all()
+
+
+@pytest.mark.parametrize("kind", ["single", "batch"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("lists", [0, 2])
+def test_gradient_over_invalid_lists(gpu, cu500, kind, precision, lists):
+    """A crystal slab in a box four times as long: its atoms have more
+    neighbours than the lists' capacity, which goes by the mean density.  The
+    first gradient call finds the lists invalid with its results and evaluates
+    the link cells after all; the next ones know, and their forward pass is
+    the link-cell kernels' (two launches).  Both give the loss and gradient
+    of a context without lists, which runs those kernels from the start: the
+    same sums in the same order, 1e-12; in mixed precision the forward
+    passes of the two launches are compiled apart, 1e-6."""
+    xyz, p, (lx, ly, lz) = seeded_atoms(6, 3.615, 63.55, temp=0.0, disp=0.1, seed=21)
+    bounds = (4.0 * lx, ly, lz)
+    c0 = cu500.cheb[:3].copy()
+
+    def make(skin):
+        if kind == "single":
+            s = CA.Simulation(cu500, bounds, defgrad=0.0, precision=precision, evaluation="cheby")
+        else:
+            s = CA.Batch([dict(pot=cu500, bounds=bounds, defgrad=0.0)] * 2, precision=precision)
+        s.tune(skin=skin, adjoint_lists=lists)
+        for r in range(s.nrep) if kind == "batch" else (None,):
+            s.bin_atoms(*(() if r is None else (r,)), xyz, p)
+        return s
+
+    def grad(s):
+        n = s.nslots if kind == "single" else s.ncells * 64 // 2
+        ft = np.zeros((n, 3))
+        return s.cheb_grad(c0, ft, -10.0, 1e-4) if kind == "single" else s.cheb_grad(c0, [ft, ft], [-10.0, -11.0], 1e-4)
+
+    plain, sim = make(0.0), make(0.4)
+    want_loss, want = grad(plain)
+    sim.timing(True)
+
+    def cell_launches():
+        return sim.timing_read()[1][CA.K_CELL_FALLBACK]
+
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    for call in range(3):
+        before = cell_launches()
+        loss, g = grad(sim)
+        info = sim.list_info()
+        assert info["active"] == 1 and info["valid"] == 0
+        assert cell_launches() - before == (0 if call == 0 else 2)
+        assert abs(loss - want_loss) <= tol * abs(want_loss)
+        compare(g, want, f"invalid lists, call {call}", tol)
+    # atoms that the lists hold: back to them
+    if kind == "single":
+        sim.bin_atoms(xyz * [4.0, 1.0, 1.0], p)
+        before = cell_launches()
+        for _ in range(2):
+            grad(sim)
+        assert cell_launches() == before and sim.list_info()["valid"] == 1
