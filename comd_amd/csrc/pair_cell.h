@@ -13,7 +13,9 @@
 // ---------------------------------------------------------------------------
 // per-wave LDS: halo x,y,z (HMAX doubles each), halo F' (EAM pass 3), queue
 // (QCAP x 64 uint16), per-lane queue counts, stencil cell ids / offsets /
-// shifts.  The reduction scratch (7 x 64 values) reuses the halo area.
+// shifts.  The reduction scratch (7 x 64 values) reuses the halo area.  In
+// whole 16-byte words: a block's waves are carved one behind the other, and
+// each starts with its doubles.
 struct WaveLds {
     double *hx, *hy, *hz, *hf;
     uint16_t *q;
@@ -24,8 +26,8 @@ struct WaveLds {
 
 __host__ __device__ constexpr int wave_lds_bytes(int kind)
 {
-    return HMAX * 8 * (kind == CM_KIND_EAM3 ? 4 : 3) + 27 * 3 * 8 + QCAP * 64 * 2 +
-           (kind == CM_KIND_EAM1 ? CM_PLIST * 64 * 2 : 0) + 64 * 4 + 27 * 4 + 28 * 4;
+    return (HMAX * 8 * (kind == CM_KIND_EAM3 ? 4 : 3) + 27 * 3 * 8 + QCAP * 64 * 2 +
+            (kind == CM_KIND_EAM1 ? CM_PLIST * 64 * 2 : 0) + 64 * 4 + 27 * 4 + 28 * 4 + 15) / 16 * 16;
 }
 
 __device__ __forceinline__ WaveLds carve(char *base, int kind)
