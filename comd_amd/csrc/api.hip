@@ -319,6 +319,15 @@ static bool any_eam(const comd_ctx *c)
     return false;
 }
 
+// Whether the list passes' launches do the link cells' work themselves should
+// the lists be invalid: until the host has seen it, and not with mixed
+// Lennard-Jones passes, which do not hold that code.
+static bool cells_inside(const comd_ctx *c)
+{
+    return !c->nl_invalid_seen &&
+           (c->nl_lj_groups == 0 || cm_nl_cells_inside(CM_KIND_LJ, c->precision == COMD_PREC_MIXED));
+}
+
 // replay_dtd: after a fused pair of half drifts whose serial replay is still
 // to be checked for (op_middle), a half drift's time
 static void op_force(comd_ctx *c, double replay_dtd = 0.0)
@@ -328,12 +337,12 @@ static void op_force(comd_ctx *c, double replay_dtd = 0.0)
     hipEvent_t ev = nullptr;
     // with neighbour lists: the (usually skipped) list build, then each pass
     // over the lists.  Should they be invalid, the link cells do the pass,
-    // inside the list passes' launches (cells) until the host has seen it, by
-    // the link-cell kernels from then on.  With mixed Lennard-Jones passes,
-    // which do not hold that code, those kernels run beside the passes every
-    // time, on a small grid (idle beside valid lists) until then
+    // inside the list passes' launches (cells_inside) until the host has seen
+    // it, by the link-cell kernels from then on.  Where the passes do not hold
+    // that code those kernels run beside them every time, on a small grid
+    // (idle beside valid lists) until then
     const bool nl = c->nl_active != 0;
-    const bool cells = !c->nl_invalid_seen && (c->nl_lj_groups == 0 || cm_nl_cells_inside(CM_KIND_LJ, mixed));
+    const bool cells = cells_inside(c);
     auto cfg_of = [&](int kind) {
         ForceCfg cfg = force_cfg(c, kind, mixed);
         if (nl && !c->nl_invalid_seen && cfg.blocks > c->ncu) cfg.blocks = c->ncu;
@@ -2116,7 +2125,7 @@ int comd_list_occupancy(comd_ctx *c, int *blocks_per_cu, int *lds_bytes, int *th
     const int mixed = c->precision == COMD_PREC_MIXED;
     const int kinds[2] = {P.kind == COMD_POT_LJ ? CM_KIND_LJ : CM_KIND_EAM1, CM_KIND_EAM3};
     for (int k = 0; k < (P.kind == COMD_POT_LJ ? 1 : 2); k++)
-        blocks_per_cu[k] = cm_nl_occupancy(P, c->nl, kinds[k], mixed, &lds_bytes[k]);
+        blocks_per_cu[k] = cm_nl_occupancy(P, c->nl, kinds[k], mixed, cells_inside(c), &lds_bytes[k]);
     *threads = c->nl.pass_threads;
     return COMD_OK;
 }

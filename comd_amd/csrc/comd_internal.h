@@ -321,8 +321,8 @@ bool cm_nl_cells_inside(int kind, int mixed);
 void cm_nl_force(const DevState &d, const PotDev &P, const CmList &l, int kind, int mixed, hipStream_t st, int g0,
                  int ng, int cells);
 // Resident blocks per CU of a list pass (-1 if the runtime cannot tell) and
-// its dynamic LDS bytes.
-int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int *lds_bytes);
+// its dynamic LDS bytes, as cm_nl_force launches it.
+int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int cells, int *lds_bytes);
 
 // Adjoint pair passes over the lists (nlist.hip): pass 1 (phi moments and
 // the energy moments), 2 (rho' moments and lambda), 3 (rho moments), one

@@ -1540,60 +1540,65 @@ size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int
     return halo + (tl ? tab : 0);
 }
 
+// A list pass as it is launched: the kernel, its dynamic LDS and, of that, the
+// table rows and what the link cells' work may use (0: none in the launch).
+struct NlPass {
+    void (*kernel)(DevState, PotDev, CmList, int, int, int);
+    size_t lds;
+    int tab, cells_lds;
+};
+
+template <int KIND, int EVAL, int MIXED>
+static NlPass nl_pass(const PotDev &P, const CmList &l, int cells)
+{
+    int tl = 0;
+    NlPass p;
+    p.lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
+    p.tab = tl ? (int)nl_tab_bytes(P, KIND, MIXED) : 0;
+    if (cells) p.lds = std::max<size_t>(p.lds, wave_lds_bytes(KIND));
+    p.cells_lds = cells ? (int)p.lds : 0;
+    p.kernel = l.lanes > 1 ? k_nl_pair<KIND, EVAL, MIXED, 0, 1> : k_nl_pair<KIND, EVAL, MIXED, 0, 0>;
+    if constexpr (EVAL == COMD_EVAL_TABLE && KIND != CM_KIND_LJ)
+        if (tl) p.kernel = l.lanes > 1 ? k_nl_pair<KIND, EVAL, MIXED, 1, 1> : k_nl_pair<KIND, EVAL, MIXED, 1, 0>;
+    return p;
+}
+
 template <int KIND, int EVAL, int MIXED>
 static void nl_launch(const DevState &d, const PotDev &P, const CmList &l, hipStream_t st, int g0, int ng, int cells)
 {
-    int tl = 0;
-    size_t lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
-    const int tab = tl ? (int)nl_tab_bytes(P, KIND, MIXED) : 0;
-    if (cells) lds = std::max<size_t>(lds, wave_lds_bytes(KIND));
-    const int cl = cells ? (int)lds : 0;
-    const dim3 grid(ng), block(l.pass_threads);
-    if constexpr (EVAL == COMD_EVAL_TABLE && KIND != CM_KIND_LJ) {
-        if (tl) {
-            if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 1>), grid, block, lds, st, d, P, l, tab, g0, cl);
-            else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 1, 0>), grid, block, lds, st, d, P, l, tab, g0, cl);
-            return;
-        }
-    }
-    if (l.lanes > 1) hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 1>), grid, block, lds, st, d, P, l, 0, g0, cl);
-    else hipLaunchKernelGGL((k_nl_pair<KIND, EVAL, MIXED, 0, 0>), grid, block, lds, st, d, P, l, 0, g0, cl);
+    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, cells);
+    hipLaunchKernelGGL(p.kernel, dim3(ng), dim3(l.pass_threads), p.lds, st, d, P, l, p.tab, g0, p.cells_lds);
 }
 
 // Resident blocks per CU of the pass nl_launch would start, and its dynamic LDS.
 template <int KIND, int EVAL, int MIXED>
-static int nl_occupancy(const PotDev &P, const CmList &l, int *lds_bytes)
+static int nl_occupancy(const PotDev &P, const CmList &l, int cells, int *lds_bytes)
 {
-    int tl = 0;
-    const size_t lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
-    const bool ln = l.lanes > 1;
-    const void *fn = ln ? (const void *)k_nl_pair<KIND, EVAL, MIXED, 0, 1> : (const void *)k_nl_pair<KIND, EVAL, MIXED, 0, 0>;
-    if constexpr (EVAL == COMD_EVAL_TABLE && KIND != CM_KIND_LJ)
-        if (tl)
-            fn = ln ? (const void *)k_nl_pair<KIND, EVAL, MIXED, 1, 1> : (const void *)k_nl_pair<KIND, EVAL, MIXED, 1, 0>;
+    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, cells);
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, l.pass_threads, lds) != hipSuccess) nb = -1;
-    if (lds_bytes) *lds_bytes = (int)lds;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)p.kernel, l.pass_threads, p.lds) != hipSuccess)
+        nb = -1;
+    if (lds_bytes) *lds_bytes = (int)p.lds;
     return nb;
 }
 
-int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int *lds_bytes)
+int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int cells, int *lds_bytes)
 {
     if (kind == CM_KIND_LJ)
-        return mixed ? nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 1>(P, l, lds_bytes)
-                     : nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 0>(P, l, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
     if (P.eval == COMD_EVAL_CHEB) {
         if (kind == CM_KIND_EAM1)
-            return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 1>(P, l, lds_bytes)
-                         : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 0>(P, l, lds_bytes);
-        return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 1>(P, l, lds_bytes)
-                     : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 0>(P, l, lds_bytes);
+            return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 1>(P, l, cells, lds_bytes)
+                         : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 0>(P, l, cells, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 1>(P, l, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 0>(P, l, cells, lds_bytes);
     }
     if (kind == CM_KIND_EAM1)
-        return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 1>(P, l, lds_bytes)
-                     : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 0>(P, l, lds_bytes);
-    return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 1>(P, l, lds_bytes)
-                 : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 0>(P, l, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
+    return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
+                 : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
 }
 
 template <int KIND, int EVAL>

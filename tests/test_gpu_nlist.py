@@ -401,3 +401,18 @@ def test_series_sums_of_the_list_passes(gpu, ncheb):
             s.force()
         assert a.list_info()["valid"] == 1
         assert_same(a, b, f"{ncheb} terms, shift {shift}", tol=1e-12)
+
+
+def test_occupancy_of_small_halos(gpu, cu500):
+    """The mixed Chebyshev density pass of a small crystal stages less than
+    one wave of the link cells' work takes (the halo alone: 12 bytes a staged
+    atom), which its launch can be asked to do: the launch has that much LDS
+    at least, in whole 16-byte words, and so reports it."""
+    wave = 14192  # density pass: 3 x 288 doubles, 27 shifts, two 24 x 64 queues, counts and stencil; to 16 bytes
+    a, _ = pair_of_sims(cu500, 6, 3.615, 300.0, 0.05, 3, "cheby", "mixed")
+    a.tune(list_groups=4)  # 2 x 2 x 1 cells, 4 x 4 x 3 staged: 48 cells of some 13 atoms, 9 KB
+    a.force()
+    occ = a.list_occupancy()
+    assert a.list_info()["valid"] == 1
+    assert occ["lds_bytes"][0] >= wave and occ["lds_bytes"][0] % 16 == 0
+    assert all(b > 0 for b in occ["blocks_per_cu"])
