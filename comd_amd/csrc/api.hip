@@ -1237,6 +1237,7 @@ static int nl_setup(comd_ctx *c)
     l.ngroups = (int)ngroups;
     l.hcap = (int)hcap;
     l.lds_avail = (int)lds_avail;
+    l.ncu = c->ncu;
     l.rows_lds = c->nl_rows_lds;
     l.pass_blocks = (int)ngroups;
     // threads per pass block: a group's home atoms with 10 % to spare
@@ -2125,7 +2126,8 @@ int comd_list_occupancy(comd_ctx *c, int *blocks_per_cu, int *lds_bytes, int *th
     const int mixed = c->precision == COMD_PREC_MIXED;
     const int kinds[2] = {P.kind == COMD_POT_LJ ? CM_KIND_LJ : CM_KIND_EAM1, CM_KIND_EAM3};
     for (int k = 0; k < (P.kind == COMD_POT_LJ ? 1 : 2); k++)
-        blocks_per_cu[k] = cm_nl_occupancy(P, c->nl, kinds[k], mixed, cells_inside(c), &lds_bytes[k]);
+        blocks_per_cu[k] = cm_nl_occupancy(P, c->nl, kinds[k], mixed, kinds[k] == CM_KIND_LJ ? c->nl_lj_groups : c->nl_eam_groups,
+                                           cells_inside(c), &lds_bytes[k]);
     *threads = c->nl.pass_threads;
     return COMD_OK;
 }

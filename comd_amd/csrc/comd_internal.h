@@ -263,6 +263,7 @@ struct CmList {
     int ngroups;             // groups, all replicas; the build order is group-major
     int hcap;                // staged halo capacity per group (atoms, <= 65535)
     int lds_avail;           // dynamic LDS a list kernel's block may use
+    int ncu;                 // compute units
     int rows_lds;            // table rows in LDS: 0 never, else whenever they fit
     int pass_blocks, pass_threads;  // one block per group (passes and build)
     int build_threads;       // of a build block
@@ -322,7 +323,7 @@ void cm_nl_force(const DevState &d, const PotDev &P, const CmList &l, int kind, 
                  int ng, int cells);
 // Resident blocks per CU of a list pass (-1 if the runtime cannot tell) and
 // its dynamic LDS bytes, as cm_nl_force launches it.
-int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int cells, int *lds_bytes);
+int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int ng, int cells, int *lds_bytes);
 
 // Adjoint pair passes over the lists (nlist.hip): pass 1 (phi moments and
 // the energy moments), 2 (rho' moments and lambda), 3 (rho moments), one

@@ -1186,10 +1186,10 @@ __host__ __device__ constexpr bool nl_cells_inside(int kind, int mixed) { return
 
 // The link cells' work of a pass whose lists are invalid, dealt to the waves
 // that the block's LDS has room for.  Replicas of the launch's kind: those with
-// groups in [gbase, gbase + gridDim.x).
+// groups in [gbase, gbase + ng).
 template <int KIND, int EVAL, int MIXED>
 __device__ __forceinline__ void cells_instead(const DevState &d, const PotDev &P, const CmList &l, char *lds, int lds_bytes,
-                                              int gbase)
+                                              int gbase, int ng)
 {
     const int W = min((int)blockDim.x >> 6, lds_bytes / wave_lds_bytes(KIND)), wv = (int)threadIdx.x >> 6;
     if (wv >= W) return;
@@ -1197,7 +1197,7 @@ __device__ __forceinline__ void cells_instead(const DevState &d, const PotDev &P
     for (int c = (int)blockIdx.x * W + wv; c < d.ncells; c += (int)gridDim.x * W) {
         if (d.ngrids > 1) {
             const int b = l.rep[rep_of(d, c)].group_base;
-            if (b < gbase || b >= gbase + (int)gridDim.x) continue;
+            if (b < gbase || b >= gbase + ng) continue;
         }
         pair_cell<KIND, EVAL, MIXED>(d, grid_of(d, c), P, w, c, (int)threadIdx.x & 63);
     }
@@ -1230,13 +1230,17 @@ constexpr int nl_pass_waves(int kind, int eval, int mixed, int lanes)
 template <int KIND, int EVAL, int MIXED, int TLDS, int LANES>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, EVAL == COMD_EVAL_CHEB ? 768 : 1024)))
 __attribute__((amdgpu_waves_per_eu(nl_pass_waves(KIND, EVAL, MIXED, LANES))))
-void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase, int cells_lds)
+void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase, int ng, int cells_lds)
 {
     extern __shared__ __align__(16) char nls[];
     __shared__ PassLds S;
+    // blocks beyond the groups are here for the link cells' work alone (left
+    // before the branch: returning after it costs the mixed embedding-force
+    // pass four more spilled registers, 188 -> 194 us at 2 048 000 atoms)
+    if ((int)blockIdx.x >= ng && !(l.flags[0] & CM_NL_INVALID)) return;
     if (l.flags[0] & CM_NL_INVALID) {
         if constexpr (nl_cells_inside(KIND, MIXED)) {
-            if (cells_lds) cells_instead<KIND, EVAL, MIXED>(d, P, l, nls, cells_lds, gbase);
+            if (cells_lds) cells_instead<KIND, EVAL, MIXED>(d, P, l, nls, cells_lds, gbase, ng);
         }
         return;
     }
@@ -1258,7 +1262,7 @@ void k_nl_pair(DevState d, PotDev P, CmList l, int tab_bytes, int gbase, int cel
     // XCD takes a contiguous range of groups, so that neighbouring groups,
     // which share halo cells, stage them through the same L2
     {
-        const int nb = gridDim.x, qb = nb / 8, rem = nb % 8;
+        const int nb = ng, qb = nb / 8, rem = nb % 8;
         const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
         const int g = gbase + (nb < 8 ? (int)blockIdx.x : xcd * qb + min(xcd, rem) + idx);
         const NlRep R = nl_rep(l, l.group_rep[g]);
@@ -1540,22 +1544,45 @@ size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int
     return halo + (tl ? tab : 0);
 }
 
-// A list pass as it is launched: the kernel, its dynamic LDS and, of that, the
-// table rows and what the link cells' work may use (0: none in the launch).
+// A list pass over ng groups as it is launched: the kernel, its grid, its
+// dynamic LDS and, of that, the table rows and what the link cells' work may
+// use (0: none in the launch).
+//
+// cells: the launch can do the link cells' work, a wave with 14 KB of LDS a
+// cell, bound by the waves at work.  The shape of the lists alone gave it one
+// to three waves a block and no block on a CU without a group, where the
+// link-cell kernels, launched beside the lists before, had four waves per CU.
+// It gets what costs the lists nothing: LDS as long as as many blocks stay
+// resident as there are groups per CU (or as the halo and the threads allow),
+// and blocks for the CUs that have no group.  A force call over lists
+// that are invalid and not yet seen to be (a slab in a box four times as long,
+// FP64 tables; link-cell kernels beside, lists' shape, this): 864 atoms 52,
+// 91, 50 us; 4000 atoms 98, 134, 54; 87 808 atoms 905, 1183, 381; 256 000 atoms
+// 2941, 975, 861; Chebyshev 87 808 atoms 1533, 1908, 647.  The passes over valid
+// lists take what they took.
 struct NlPass {
-    void (*kernel)(DevState, PotDev, CmList, int, int, int);
+    void (*kernel)(DevState, PotDev, CmList, int, int, int, int);
+    int grid;
     size_t lds;
     int tab, cells_lds;
 };
 
 template <int KIND, int EVAL, int MIXED>
-static NlPass nl_pass(const PotDev &P, const CmList &l, int cells)
+static NlPass nl_pass(const PotDev &P, const CmList &l, int ncells, int ng, int cells)
 {
     int tl = 0;
     NlPass p;
+    p.grid = ng;
     p.lds = cm_nl_pass_lds(P, l, KIND, MIXED, &tl);
     p.tab = tl ? (int)nl_tab_bytes(P, KIND, MIXED) : 0;
-    if (cells) p.lds = std::max<size_t>(p.lds, wave_lds_bytes(KIND));
+    if (cells) {
+        const int wb = wave_lds_bytes(KIND), room = l.lds_avail + CM_NL_STATIC_LDS, threads = l.pass_threads;
+        const int resident = std::max(1, std::min({(ng + l.ncu - 1) / l.ncu, 2048 / threads,
+                                                   room / std::max(1, (int)p.lds)}));  // at most
+        const int waves = std::max(1, std::min(threads / 64, (room / resident - CM_NL_STATIC_LDS) / wb));
+        p.lds = std::max(p.lds, (size_t)waves * wb);
+        p.grid = std::max(ng, std::min((ncells + waves - 1) / waves, l.ncu * std::max(1, 256 / threads)));
+    }
     p.cells_lds = cells ? (int)p.lds : 0;
     p.kernel = l.lanes > 1 ? k_nl_pair<KIND, EVAL, MIXED, 0, 1> : k_nl_pair<KIND, EVAL, MIXED, 0, 0>;
     if constexpr (EVAL == COMD_EVAL_TABLE && KIND != CM_KIND_LJ)
@@ -1566,15 +1593,15 @@ static NlPass nl_pass(const PotDev &P, const CmList &l, int cells)
 template <int KIND, int EVAL, int MIXED>
 static void nl_launch(const DevState &d, const PotDev &P, const CmList &l, hipStream_t st, int g0, int ng, int cells)
 {
-    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, cells);
-    hipLaunchKernelGGL(p.kernel, dim3(ng), dim3(l.pass_threads), p.lds, st, d, P, l, p.tab, g0, p.cells_lds);
+    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, d.ncells, ng, cells);
+    hipLaunchKernelGGL(p.kernel, dim3(p.grid), dim3(l.pass_threads), p.lds, st, d, P, l, p.tab, g0, ng, p.cells_lds);
 }
 
 // Resident blocks per CU of the pass nl_launch would start, and its dynamic LDS.
 template <int KIND, int EVAL, int MIXED>
-static int nl_occupancy(const PotDev &P, const CmList &l, int cells, int *lds_bytes)
+static int nl_occupancy(const PotDev &P, const CmList &l, int ng, int cells, int *lds_bytes)
 {
-    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, cells);
+    const NlPass p = nl_pass<KIND, EVAL, MIXED>(P, l, 0, ng, cells);  // the grid plays no part
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)p.kernel, l.pass_threads, p.lds) != hipSuccess)
         nb = -1;
@@ -1582,23 +1609,23 @@ static int nl_occupancy(const PotDev &P, const CmList &l, int cells, int *lds_by
     return nb;
 }
 
-int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int cells, int *lds_bytes)
+int cm_nl_occupancy(const PotDev &P, const CmList &l, int kind, int mixed, int ng, int cells, int *lds_bytes)
 {
     if (kind == CM_KIND_LJ)
-        return mixed ? nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
-                     : nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 1>(P, l, ng, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_LJ, COMD_EVAL_TABLE, 0>(P, l, ng, cells, lds_bytes);
     if (P.eval == COMD_EVAL_CHEB) {
         if (kind == CM_KIND_EAM1)
-            return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 1>(P, l, cells, lds_bytes)
-                         : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 0>(P, l, cells, lds_bytes);
-        return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 1>(P, l, cells, lds_bytes)
-                     : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 0>(P, l, cells, lds_bytes);
+            return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 1>(P, l, ng, cells, lds_bytes)
+                         : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_CHEB, 0>(P, l, ng, cells, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 1>(P, l, ng, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_CHEB, 0>(P, l, ng, cells, lds_bytes);
     }
     if (kind == CM_KIND_EAM1)
-        return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
-                     : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
-    return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 1>(P, l, cells, lds_bytes)
-                 : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 0>(P, l, cells, lds_bytes);
+        return mixed ? nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 1>(P, l, ng, cells, lds_bytes)
+                     : nl_occupancy<CM_KIND_EAM1, COMD_EVAL_TABLE, 0>(P, l, ng, cells, lds_bytes);
+    return mixed ? nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 1>(P, l, ng, cells, lds_bytes)
+                 : nl_occupancy<CM_KIND_EAM3, COMD_EVAL_TABLE, 0>(P, l, ng, cells, lds_bytes);
 }
 
 template <int KIND, int EVAL>

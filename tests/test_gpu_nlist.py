@@ -416,3 +416,43 @@ def test_occupancy_of_small_halos(gpu, cu500):
     assert a.list_info()["valid"] == 1
     assert occ["lds_bytes"][0] >= wave and occ["lds_bytes"][0] % 16 == 0
     assert all(b > 0 for b in occ["blocks_per_cu"])
+
+
+@pytest.mark.parametrize("n,precision", [(6, "fp64"), (10, "fp64"), (10, "mixed"), (20, "fp64")])
+@pytest.mark.parametrize("evaluation", ["table", "cheby"])
+def test_link_cells_inside_the_passes_of_few_groups(gpu, cu500, n, evaluation, precision):
+    """A crystal slab in a box four times as long, whose lists overflow: few
+    groups, small blocks, cells without a group's block to each CU.  The link
+    cells' work inside the list launches covers every cell (forces of a context
+    without lists, as above) and takes no longer than half as much again as the
+    link-cell kernels that replace it once the host has seen the lists invalid
+    (with the waves of the lists' own shape alone it took two to five times as
+    long)."""
+    xyz, p, (lx, ly, lz) = seeded_atoms(n, 3.615, 63.55, temp=300.0, disp=0.1, seed=2)
+
+    def make(skin):
+        s = CA.Simulation(cu500, (4.0 * lx, ly, lz), defgrad=0.0, precision=precision, evaluation=evaluation)
+        s.tune(skin=skin)
+        s.bin_atoms(xyz, p)
+        s.force()
+        return s
+
+    a, b = make(0.4), make(0.0)
+    assert a.list_info()["active"] == 1 and a.list_info()["valid"] == 0
+    assert_same(a, b, f"slab {n} {evaluation} {precision}")
+    a.timing(True)
+
+    def best(passes):
+        times = []
+        for _ in range(10):
+            before = a.timing_read()[0]
+            a.force()
+            after = a.timing_read()[0]
+            times.append(sum(after[k] - before[k] for k in passes))
+        return min(times)
+
+    inside = best((CA.K_DENSITY, CA.K_EMBED_FORCE))
+    a.sync()  # the host looks
+    beside = best((CA.K_CELL_FALLBACK,))
+    print(f"[slab {n} {evaluation} {precision}] inside {1e3 * inside:.1f} us, beside {1e3 * beside:.1f} us", flush=True)
+    assert beside > 0.0 and inside <= 1.5 * beside
