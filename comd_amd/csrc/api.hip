@@ -150,7 +150,8 @@ struct comd_ctx {
     int nl_invalid_seen; // the lists were invalid when the host last looked
     int nl_group_opt;   // COMD_TUNE_LIST_GROUPS (-1: by size, nl_setup)
     int nl_two_per_cu;  // the default shape of earlier snapshots: the largest with two groups per CU
-                        // (set by loading one)
+                        // (set by loading one, until the atoms are replaced or the
+                        // shape is tuned)
     int nl_rows_lds;    // COMD_TUNE_LIST_ROWS_LDS (-1: whenever they fit)
     int nl_threads_div; // COMD_TUNE_LIST_THREADS_DIV: home atoms per thread of the list passes
     int nl_lanes;       // COMD_TUNE_LIST_LANES: lanes per home atom of the list passes (0: by size)
@@ -1561,6 +1562,7 @@ static int upload_rep(comd_ctx *c, int r, const int *natoms, const int *id, cons
     c->reps[r].ntot = tot;
     c->have_atoms = 1;
     c->reps[r].nl_ids = nids;
+    c->nl_two_per_cu = 0;
     return nl_setup(c);
 }
 
@@ -1586,6 +1588,7 @@ static int bin_rep_device(comd_ctx *c, int r, int n, const double *d_xyz, const 
     c->reps[r].ntot = n;
     c->have_atoms = 1;
     c->reps[r].nl_ids = n;
+    c->nl_two_per_cu = 0;
     return nl_setup(c);
 }
 
@@ -1903,6 +1906,7 @@ int comd_tune(comd_ctx *c, int key, int value)
     case COMD_TUNE_LIST_GROUPS:
         if (value < -1 || value > 4) return set_err(c, COMD_ERR_ARG, "list group option must be -1..4");
         c->nl_group_opt = value;
+        c->nl_two_per_cu = 0;
         if (c->have_atoms) return nl_setup(c);
         break;
     case COMD_TUNE_LIST_ROWS_LDS:
@@ -1973,6 +1977,7 @@ static int autotune_lists(comd_ctx *c, int *group_opt, int *rows_lds, int *threa
     double best = 1e300;
     int bg = g0, br = r0, bd = d0;
     int rc = COMD_OK;
+    c->nl_two_per_cu = 0;
     for (int g = -1; g <= 4 && !rc; g++)
         for (int r = rows_matter ? 0 : -1; r >= -1 && !rc; r--)
             for (int dv = 1; dv <= 2 && !rc; dv++) {

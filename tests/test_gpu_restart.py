@@ -79,3 +79,33 @@ def test_restart_from_lists_of_the_earlier_default_shape(gpu, cu500, tmp_path):
     ga, gb = a.download(), b.download()
     for k in ("natoms", "id", "itype", "r", "p", "f", "rho", "fi"):
         assert np.array_equal(ga[k], gb[k]), k
+
+
+@pytest.mark.parametrize("how", ["bin", "upload", "tune", "autotune"])
+def test_the_earlier_shape_ends_with_its_atoms(gpu, cu500, tmp_path, how):
+    """A context that took a file's lists in the earlier default shape has
+    today's shape again once its atoms are replaced or the shape is tuned."""
+    xyz, p, bounds = seeded_atoms(20, 3.615, cu500.mass, temp=600.0, disp=0.1, seed=5)
+    path = str(tmp_path / "s.bin")
+    a = CA.Simulation(cu500, bounds, defgrad=0.0)
+    a.bin_atoms(xyz, p)
+    today = a.list_occupancy()
+    a.tune(list_groups=4)
+    earlier = a.list_occupancy()
+    assert earlier != today
+    a.force()
+    a.snapshot_save(path)
+    b = CA.Simulation(cu500, bounds, defgrad=0.0)
+    b.snapshot_load(path)
+    assert b.list_occupancy() == earlier
+    if how == "bin":
+        b.bin_atoms(xyz, p)
+    elif how == "upload":
+        s = b.download()
+        b.upload(*[s[k] for k in ("natoms", "id", "itype", "r", "p")])
+    elif how == "tune":
+        b.tune(list_groups=-1)
+    else:
+        b.autotune_lists()
+        b.tune(list_groups=-1, list_rows_lds=-1, list_threads_div=1)
+    assert b.list_occupancy() == today
