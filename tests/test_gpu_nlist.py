@@ -456,3 +456,79 @@ def test_link_cells_inside_the_passes_of_few_groups(gpu, cu500, n, evaluation, p
     beside = best((CA.K_CELL_FALLBACK,))
     print(f"[slab {n} {evaluation} {precision}] inside {1e3 * inside:.1f} us, beside {1e3 * beside:.1f} us", flush=True)
     assert beside > 0.0 and inside <= 1.5 * beside
+
+
+@pytest.mark.parametrize("lists", [True, False])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [3, 8, 9, 17, 24, 25, 31])
+def test_short_series_equal_their_zero_padded_32(gpu, cu500, n, precision, lists):
+    """A series of n terms and the one of 32 with zeros behind are the same
+    sums: Clenshaw's recurrence starts with exact zeros at those terms, and
+    the shared basis adds exact zeros.  So the passes give the same bits, for
+    every stride of the series (8, 16, 24, 32) and in both precisions."""
+    short = np.ascontiguousarray(cu500.cheb[:3, :n])
+    padded = np.zeros((3, 32))
+    padded[:, :n] = short
+    got = []
+    for pot, coef in ((CA.EAMPotential(cu500.name, ncheb=n), short), (cu500, padded)):
+        s = pair_of_sims(pot, 6, 3.615, 600.0, 0.1, 7, "cheby", precision)[0 if lists else 1]
+        s.set_cheb(coef)
+        s.force()
+        assert s.list_info()["active"] == lists and (not lists or s.list_info()["valid"] == 1)
+        got.append(compact(s.download()))
+    for k in ("f", "rho", "fi"):
+        assert np.isfinite(got[0][k]).all() and np.array_equal(got[0][k], got[1][k]), k
+
+
+def clenshaw32_bound(c, a, b, x):
+    """What an FP32 Clenshaw sum of the series c on [a, b] at x (arrays), from
+    FP32 coefficients, may differ from the exact one: the rounding of each
+    term's recurrence (three operations, and the coefficient's own) reaches the
+    sum times |U_k(y)| <= k + 1; an argument off by the rounding of its own
+    forming (x, a, b to FP32, two additions and a product) and by the 2e-8 A of
+    the fixed-point positions, times |S'(y)| <= sum k^2 |c_k|."""
+    u = 2.0 ** -24
+    n = len(c)
+    y = (2.0 * x - a - b) / (b - a)
+    d = dd = np.zeros_like(y)
+    err = np.zeros_like(y)
+    for k in range(n - 1, -1, -1):
+        size = np.abs(2.0 * y * d) + np.abs(dd) + np.abs(c[k])
+        err = err + (k + 1) * 4.0 * u * size
+        d, dd = 2.0 * y * d - dd + c[k], d
+    arg = (6.0 * u * (2.0 * np.abs(x) + abs(a) + abs(b)) + 4e-8) / (b - a)
+    return err + arg * np.sum(np.arange(n) ** 2 * np.abs(c))
+
+
+@pytest.mark.parametrize("n", [3, 9, 24, 31])
+@pytest.mark.parametrize("shift", [0.0, 0.37])
+def test_mixed_series_sums_of_the_list_passes(gpu, n, shift):
+    """As test_series_sums_of_the_list_passes in mixed precision: the lists and
+    the link cells sum phi and rho in FP32, each within clenshaw32_bound of
+    the exact series per pair, and the list passes their eight pairs' values
+    too (7 x 2^-24 of them).  So rho differs by twice that times the
+    neighbours at most, the energy by half of phi's and F'(rho) times rho's."""
+    pot = CA.EAMPotential("cu500", ncheb=n)
+    pot.cheb_dom[1, 1] += shift
+    a, b = pair_of_sims(pot, 6, 3.615, 600.0, 0.1, 7, "cheby", "mixed")
+    for s in (a, b):
+        s.force()
+    assert a.list_info()["valid"] == 1
+    ga, gb = (compact(s.download()) for s in (a, b))
+    m = np.arange(64)[None, :] < b.download()["natoms"][:, None]
+    nnb = b.download_aux()[0].reshape(-1, 64)[m]
+    r = np.linspace(2.0, pot.cutoff, 4000)
+
+    def per_pair(k):
+        lo, hi = pot.cheb_dom[k]
+        c = pot.cheb[k, :n]
+        y = (2.0 * r - lo - hi) / (hi - lo)
+        value = np.abs(np.polynomial.chebyshev.chebval(y, c) - 0.5 * c[0]).max()
+        return (clenshaw32_bound(c, lo, hi, r) + 8.0 * 2.0 ** -24 * value).max()
+
+    drho = 2.0 * nnb * per_pair(1)
+    de = nnb * per_pair(0) + np.abs(gb["fi"]) * drho * 1.01
+    err_rho, err_e = np.abs(ga["rho"] - gb["rho"]), np.abs(ga["f"][:, 3] - gb["f"][:, 3])
+    print(f"[mixed series {n} {shift}] rho {(err_rho / drho).max():.3f}, energy {(err_e / de).max():.3f} of the bound;"
+          f" relative bound rho {(drho / np.abs(gb['rho'])).max():.1e}", flush=True)
+    assert (err_rho <= drho).all() and (err_e <= de).all()
