@@ -80,11 +80,10 @@ def log(msg):
 
 
 def run_precision(sim, precision, steps, warmup, n_atoms, timed_steps, autotune=True):
-    """steps timed as the library runs them (the step replayed as a HIP
-    graph), the energy drift over those steps, then timed_steps more with
-    HIP events around every kernel class on the simulation's stream (the
-    events break the graph into separate launches, so these steps are not
-    the throughput figure)."""
+    """steps timed as the library runs them, the energy drift over those
+    steps, then timed_steps more with HIP events around every kernel class on
+    the simulation's stream (the events add to each launch, so these steps are
+    not the throughput figure)."""
     sim.set_precision(precision)
     tuned = sim.autotune_lists() if autotune and sim.list_info()["active"] else None  # setup, not timed
     log(f"{precision}: list passes autotuned: {tuned}")
@@ -423,7 +422,7 @@ def main():
         "kernel_ms_per_step": {name: mixed["kernel_ms"][i] / mixed["timed_steps"] for i, name in enumerate(KCLASS)},
         "kernel_timing": {"steps": mixed["timed_steps"], "ms_per_step_with_events": mixed["ms_per_step_events"],
                           "note": "HIP events around each kernel class on the simulation's stream, over steps run "
-                                  "after the timed ones (the events split the step graph into separate launches)"},
+                                  "after the timed ones (the events add to each launch)"},
         "neighbour_lists": {"active": mixed["lists"], "skin_A": 0.4, "builds_in_timed_steps": mixed["builds"],
                             "list_capacity": mixed["kmax"], "lanes_per_atom": mixed["lanes"],
                             "autotuned_shape": {"mixed": mixed["autotune"], "fp64": fp64["autotune"]}},

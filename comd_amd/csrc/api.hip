@@ -1015,15 +1015,14 @@ static int nl_setup(comd_ctx *c)
         const double expect = 4.0 / 3.0 * 3.141592653589793 * rl * rl * rl * (double)R.ntot / vol;
         kmax = std::max<long>(kmax, (((long)(1.5 * expect) + 16 + 15) / 16) * 16);
     }
-    // groups of auxiliary cells: of the options whose staged halo (1.2x the
+    // groups of auxiliary cells: one of the options whose staged halo (1.2x the
     // mean occupancy, plus 64 atoms, in the densest replica) fits the LDS a
     // block may use in every pass (16 B per halo atom in mixed precision, up
-    // to 32 B in FP64, and a byte of slot map) beside the kernels' static
-    // LDS, the largest that still gives two groups (blocks) per CU, else the
-    // one with the most groups; a tuned option is taken as the largest
-    // allowed.  Each replica's auxiliary grid is rounded down to whole groups
-    // per dimension (cells a little larger than cutoff + skin): a partial
-    // group at an edge would take a whole block for a sliver of atoms.
+    // to 32 B in FP64, and a byte of the build's slot map) beside the kernels'
+    // static LDS: by the work on the busiest CU (below), a tuned option as the
+    // largest allowed.  Each replica's auxiliary grid is rounded down to whole
+    // groups per dimension (cells a little larger than cutoff + skin): a
+    // partial group at an edge would take a whole block for a sliver of atoms.
     const int gopts[5][3] = {{4, 4, 3}, {4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {2, 2, 1}};
     // the shapes of the per-replica search of batches (the halo of each,
     // (x + 2)(y + 2)(z + 2) slots, within CM_NL_SLOTS)
@@ -1043,9 +1042,12 @@ static int nl_setup(comd_ctx *c)
     // atoms 61 -> 53 us, eight lanes 60; 13 500 atoms 72 -> 65, eight 67;
     // 32 000: 93 both ways; tables, 864 atoms 53.4 -> 51.2, 4000 60.0 against
     // 61.9).  Lennard-Jones and batches, whose groups are shaped for one
-    // lane's threads: two below 128 per CU (32 000 Lennard-Jones atoms, pass 34 ->
-    // 26 us; 256 000 121 us a step against 130; 3 x 23 328 atoms' gradient 668
-    // against 682)
+    // lane's threads: two below 128 per CU (Lennard-Jones, one lane and two, us a
+    // step: 16 384 atoms 44.8, 39.3; 32 000 42.3, 41.4; from 512 per CU on one
+    // lane, 131 072 atoms 69.7, 75.3; 256 000 97.5, 107.6; between the two lines
+    // two lanes are 1 to 4 % faster, 87 808 atoms 62.6, 60.3, and would give
+    // those systems' forces in another order of their sums.  3 x 23 328 atoms'
+    // gradient 668 against 682)
     long natoms_all = 0;
     bool lj = false, cheb = true;
     for (const Replica &R : c->reps) {
@@ -1059,10 +1061,13 @@ static int nl_setup(comd_ctx *c)
                       : natoms_all < (cheb ? 64L : 8L) * c->ncu             ? 4
                                                                             : 2;
     // threads of a pass' block for its group's home atoms: 10 % more than
-    // the mean group's; 80 % where the system is small, whose groups of few
-    // cells differ most in their atoms: one atom more than threads and the
-    // block runs a second round (4000 atoms, two lanes, tables 69 -> 56 us a
-    // step, Chebyshev 136 -> 91; 32 000 atoms 69.9 -> 68.8)
+    // the mean group's, 80 % with several lanes per atom, whose groups have
+    // fewer cells or less room: one atom more than threads and the block runs a
+    // second round (10 % and 80 %, us a step: 4000 atoms tables 53, 41, Chebyshev
+    // 81, 67; 16 384 atoms 62, 50 and 102, 69; 87 808 atoms 84-89, 78 and 144, 133;
+    // from 157 216 atoms to the end of the two-lane range the block is cut to
+    // 768 threads either way and the two take the same: 256 000 atoms 137, 137
+    // and 251, 251; 500 000 214-217, 214 and 414, 414).
     // The build keeps to 10 % and two lanes' threads: its threads' queues set
     // the order of the lists (k_nl_build), which should not vary with the
     // passes' shape
@@ -1241,7 +1246,7 @@ static int nl_setup(comd_ctx *c)
     l.ncu = c->ncu;
     l.rows_lds = c->nl_rows_lds;
     l.pass_blocks = (int)ngroups;
-    // threads per pass block: a group's home atoms with 10 % to spare
+    // threads per pass block: a group's home atoms with room to spare (above)
     l.pass_threads = (int)pass_threads;
     l.build_threads = (int)std::min<long>(768, build_threads);
     l.adj_threads = (int)std::min<long>(768, adj_threads);
@@ -1352,10 +1357,14 @@ static int nl_setup(comd_ctx *c)
 
 // Chunks of a state transfer.  A chunk's packing over PCIe (57 GB/s) runs
 // while the host copies the one before it out of its buffer; one thread does
-// that at about 28 GB/s, two at 48 (r, p and ids of 12.5 M slots, 650 MB: 23
-// and 13.4 ms), more gain nothing.  A second thread costs about 0.03 ms to
-// start and pays from 64 MB on.  Below that 1 MB chunks overlap better (8 MB:
-// 25 GB/s against 22) and need less pinned memory.
+// that at 20 to 28 GB/s, two at 38 to 48 (r, p and ids of 12.5 M slots, 650 MB:
+// 23 and 13.4 ms; the whole state, one thread in 1 MB chunks and two in 4 MB
+// ones: 250 MB 12.4 and 6.2 ms, 61 MB 2.9 and 1.66), more gain nothing.  A
+// second thread costs 0.01 to 0.03 ms to start: at 1 MB 0.066 and 0.077 ms, at 8 MB
+// 0.32 and 0.31, so that it pays somewhat below the line drawn here (31 MB 1.4
+// and 1.0 ms), which keeps the pinned memory of small states to 2 MB and their
+// calls to the caller's own thread.  With one thread 1 MB chunks overlap
+// better (8 MB: 25 GB/s against 22).
 #define CM_XF_LARGE ((size_t)64 << 20)
 #define CM_XF_CHUNK_SMALL ((size_t)1 << 20)
 #define CM_XF_CHUNK_LARGE ((size_t)4 << 20)

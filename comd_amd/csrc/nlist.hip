@@ -11,7 +11,7 @@
 // up.  Nothing waits on the host, so a step stays capturable.
 //
 // Atoms are binned into auxiliary cells of edge >= cutoff + skin, and the
-// cells into groups of up to 4 x 4 x 2.  The build order (t) is group-major,
+// cells into groups of up to 4 x 4 x 3.  The build order (t) is group-major,
 // then cell, then atom id.  A force pass stages a group's halo -- the atoms
 // of its cells and of the cells around them -- in LDS once, and each home
 // atom's list holds 16-bit indices into that halo: the neighbour positions
@@ -471,7 +471,9 @@ __device__ static void group_starts(const CmList &l)
 // TLBs and caches turned over by the passes between), and apart these were
 // four.  With the link cells' code inside the passes (cells_instead) a step's
 // launches are ten in place of fifteen: 864 atoms 53 -> 46 us, 32 000
-// Lennard-Jones atoms 71 -> 64, 256 000 atoms FP64 181 -> 175.  No fence per block
+// Lennard-Jones atoms 71 -> 64, 256 000 atoms FP64 181 -> 175.  A rebuild pays for it:
+// at 2 048 000 atoms this kernel takes 301 us where two took 157 (86 of it the
+// groups by one block), one step in 27.  No fence per block
 // is needed: the last block reads only what atomics wrote, except after a
 // replay (rare: its blocks fence, and the last one does the cells' work alone,
 // once every replica is settled).

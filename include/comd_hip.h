@@ -229,8 +229,8 @@ int comd_list_info(comd_ctx *ctx, int *active, int *valid, int *builds, int *kma
  * tuning the group shape; no counterpart in the reference. */
 int comd_list_occupancy(comd_ctx *ctx, int blocks_per_cu[2], int lds_bytes[2], int *threads);
 
-/* Lanes per home atom of the neighbour-list passes (1, 2 or 4: as tuned with
- * COMD_TUNE_LIST_LANES, else the context's default for its size); 0 while
+/* Lanes per home atom of the neighbour-list passes (1, 2, 4, 8 or 16: as tuned
+ * with COMD_TUNE_LIST_LANES, else the context's default for its size); 0 while
  * the lists are off.  A diagnostic beside comd_list_occupancy; no
  * counterpart in the reference. */
 int comd_list_lanes(comd_ctx *ctx, int *lanes);
@@ -265,8 +265,11 @@ enum comd_kclass {
     COMD_K_REDUCE = 3,
     COMD_K_LIST_BUILD = 4, /* neighbour-list rebuild check (+ rebuild) */
     COMD_K_CELL_FALLBACK = 5, /* link-cell passes launched beside the list
-                                 passes; they return at once while the lists
-                                 are valid */
+                                 passes: in mixed precision with Lennard-Jones
+                                 (they return at once while the lists are
+                                 valid), and once the lists were seen to be
+                                 invalid; until then the launches of classes 1
+                                 and 2 do the link cells' work */
     COMD_K_NCLASS = 6
 };
 int comd_timing(comd_ctx *ctx, int on);
