@@ -1552,9 +1552,10 @@ size_t cm_nl_pass_lds(const PotDev &P, const CmList &l, int kind, int mixed, int
 //
 // cells: the launch can do the link cells' work, a wave with 14 KB of LDS a
 // cell, bound by the waves at work.  The shape of the lists alone gave it one
-// to three waves a block and no block on a CU without a group, where the
-// link-cell kernels, launched beside the lists before, had four waves per CU.
-// It gets what costs the lists nothing: LDS as long as as many blocks stay
+// to three waves a block and no block on a CU without a group, and its code
+// spills where the list passes' registers are held down, so that it was slower
+// than the link-cell kernels on one wave per CU, launched beside the lists
+// before.  It gets what costs the lists nothing: LDS as long as as many blocks stay
 // resident as there are groups per CU (or as the halo and the threads allow),
 // and blocks for the CUs that have no group.  A force call over lists
 // that are invalid and not yet seen to be (a slab in a box four times as long,
