@@ -1455,14 +1455,10 @@ static int transfer(comd_ctx *c, const DevState &d, const Grid &g, const CmSlots
     const int nchunk = (g.ncells + most - 1) / most;
     const int span = nchunk > 1 ? most : g.ncells;  // cells per chunk
     const size_t size = (per * span + 255) / 256 * 256;
-    int nthr = large ? 2 : 1;
+    const int nthr = large ? 2 : 1;
     // two buffers a thread
     const XferStage stage = xfer_acquire(size * (nchunk > 1 ? 2 * nthr : 1));
     if (!stage.h) return set_err(c, COMD_ERR_NOMEM, "transfer staging");
-    if (nthr == 2 && !c->xf_stream && hipStreamCreateWithFlags(&c->xf_stream, hipStreamNonBlocking) != hipSuccess) {
-        c->xf_stream = nullptr;
-        nthr = 1;
-    }
     // by the stream, not by events: an event's completion has work in the
     // runtime's own thread after the call's return, and a caller that goes on
     // with as many threads as there are CPUs waits for it (58 000 atoms
@@ -1518,17 +1514,27 @@ static int transfer(comd_ctx *c, const DevState &d, const Grid &g, const CmSlots
         if (!wait(st)) ok = false;
         return ok;
     };
-    bool ok0, ok1 = true;
+    bool ok0, ok1 = true, shared = false;
     std::thread other;
     if (nthr == 2) {
+        // its stream on the context's device, whichever the caller's current one is
+        auto half = [&] {
+            if (hipSetDevice(c->device) != hipSuccess) return;
+            if (!c->xf_stream && hipStreamCreateWithFlags(&c->xf_stream, hipStreamNonBlocking) != hipSuccess) {
+                c->xf_stream = nullptr;
+                return;
+            }
+            shared = true;
+            ok1 = copy(1, c->xf_stream);
+        };
         try {
-            other = std::thread([&] { ok1 = hipSetDevice(c->device) == hipSuccess && copy(1, c->xf_stream); });
-        } catch (...) {  // no thread to be had: this one takes both halves
+            other = std::thread(half);
+        } catch (...) {
         }
     }
     ok0 = copy(0, c->stream);
     if (other.joinable()) other.join();
-    else if (nthr == 2) ok1 = copy(1, c->stream);
+    if (nthr == 2 && !shared) ok1 = copy(1, c->stream);  // no thread or stream to be had: both halves here
     xfer_release(stage);
     if (!ok0 || !ok1) return set_err(c, COMD_ERR_HIP, "state transfer failed");
     return COMD_OK;

@@ -58,3 +58,23 @@ def test_batch_parts_and_missing_fields():
     assert hip.comd_batch_download(b.ctx, 1, None, None, None, None, None, None, None, None) == 0
     for r in (0, 2):
         assert np.array_equal(b.download(r)["r"], given[r]["r"])
+
+
+def test_large_transfer_with_another_device_current():
+    """The second copying thread's stream belongs to the context's device, not
+    to the one that is current when the first large transfer is made."""
+    torch = pytest.importorskip("torch")
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two devices")
+    pot = CA.LJPotential(sigma=1.0, epsilon=0.01, cutoff=2.0, mass=1.0)
+    torch.cuda.set_device(0)
+    try:
+        sim = CA.Simulation(pot, [2.0 * n + 0.01 for n in (27, 27, 27)])  # 71 MB up, 131 MB down
+        given = random_slots(sim.ncells, 5)
+        torch.cuda.set_device(1)
+        sim.upload(*[given[k] for k in ("natoms", "id", "itype", "r", "p")])
+        got = sim.download()
+        for k, v in given.items():
+            assert np.array_equal(got[k], v), k
+    finally:
+        torch.cuda.set_device(0)
